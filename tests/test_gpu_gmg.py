@@ -196,6 +196,42 @@ def test_patch_bicgstab_smoother(name, ns, op_kind):
     assert relerr(mesh.interior(du32.get(), dim), mesh.interior(uref, dim)) <= 1e-4
 
 
+@pytest.mark.parametrize("ns,op_kind,neumann", [
+    ((8, 8), 0, False), ((16, 16), 0, True), ((32, 32), 0, False), ((32, 32), 0, True), ((16, 16), 1, False),
+    ((32, 32), 1, False),  # column strips, one and four waves
+    ((8, 6), 0, True), ((10, 10), 1, False), ((16, 14), 0, False), ((20, 24), 1, False), ((64, 64), 0, False),
+    ((6, 4, 8), 0, True), ((8, 8, 8), 1, False), ((16, 16, 16), 0, False)])  # staged operand, one and four waves
+def test_patch_bicgstab_shapes(ns, op_kind, neumann):
+    """Every branch of the patch BiCGStab's dispatch.  Three iterations do the same arithmetic
+    as the oracle's up to the order of sums; to a tolerance t the residuals agree to t, so the
+    solutions do to t times the patch operator's condition number, about 2 (2 n / pi)^2."""
+    _print_case("patch-bicgstab-shapes", ns, op_kind, neumann)
+    name = "2d_uniform_2x2_refined_nw_mpi1.json" if len(ns) == 2 else "3d_refined_bnw_2x2x2_mpi1.json"
+    dim, levels = load(name, ns)
+    lv, kind = levels[0], R.TRILINEAR if dim == 3 else R.BILINEAR
+    od, dd = O.Domain(dim, ns, lv), R.Domain(dim, ns, lv)
+    g = R.GhostFiller(dd, kind, R.FACES)
+    f0, u0 = random_field(od.shape(1), 43), random_field(od.shape(1), 44)
+    coeffs, dc = None, {np.float64: None, np.float32: None}
+    if op_kind == 1:
+        X = mesh.cell_centers(lv, dim, ns)
+        coeffs = np.exp(np.sin(3 * X[..., 0]) * np.cos(2 * X[..., 1]))[:, None].copy()
+        O.fill_ghost(od, coeffs, kind=kind)
+        dc = {t: R.DeviceArray.from_host(coeffs.astype(t)) for t in dc}
+    cond = 2 * (2 * max(ns) / np.pi) ** 2 * (np.e**2 if op_kind else 1)
+    for dtype, max_it, tol, bound in ((np.float64, 3, 1e-12, 1e-10), (np.float64, 1000, 1e-12, cond * 1e-12),
+                                      (np.float32, 1000, 1e-5, cond * 1e-5)):
+        uref = u0.copy()
+        O.bicgstab_smooth(od, f0.copy(), uref, kind=kind, op_kind=op_kind, neumann=neumann, coeffs=coeffs,
+                          max_it=max_it, tol=min(tol, 1e-12))
+        du = R.DeviceArray.from_host(u0.astype(dtype))
+        iters = R.DeviceArray((len(lv),), np.int32)
+        g.patch_bicgstab_smooth(R.DeviceArray.from_host(f0.astype(dtype)), du, op_kind=op_kind, neumann=neumann,
+                                coeffs=dc[dtype], max_it=max_it, tol=tol, continue_on_breakdown=True, iters=iters)
+        assert relerr(mesh.interior(du.get(), dim), mesh.interior(uref, dim)) <= bound, (dtype, max_it)
+        assert iters.get().max() <= max_it and iters.get().min() > 0
+
+
 def test_varpoisson_gmg():
     _print_case("varpoisson-gmg")
     ns = (16, 16)
