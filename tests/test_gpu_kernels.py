@@ -4,6 +4,8 @@ FP64: max-norm relative difference <= 1e-12 (the hot path's FP64 parity bar).
 FP32: the oracle runs on the float-rounded inputs in FP64; max-norm relative
 difference <= 2e-6 (a few float ulps accumulated over the stencil / transforms).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -11,6 +13,7 @@ from helpers import MESH_2D, MESH_3D, face_ghost_mask, load, random_field, reler
 from oracle import oracle as O
 from thunderegg_amd import mesh
 from thunderegg_amd import runtime as R
+from thunderegg_amd import solver
 
 pytestmark = pytest.mark.gpu
 
@@ -330,6 +333,62 @@ def test_fused_vcycle_launches(name, ns, kind, op_kind):
                 assert relerr(mesh.interior(fc.get(), dim), mesh.interior(fcr, dim)) <= tol, (dt, tf, tc)
             # u and uc are inputs only
             assert np.array_equal(u.get(), u0.astype(npd))
+
+
+@pytest.mark.parametrize("ns,base", [((5, 4), 1), ((16, 16), 0), ((16, 3), 3), ((2, 2), 0), ((6, 4, 8), 1), ((7, 5, 3), 1),
+                                     ((16, 16, 16), 2)])
+@pytest.mark.parametrize("dtype", [R.F64, R.F32])
+@pytest.mark.parametrize("off", [0, 1])
+def test_vector_kernels_shapes(ns, base, dtype, off):
+    """Rows of odd and even length, one patch to several workgroups, and vectors that start one
+    value off the paired accesses' grid: every update and reduction against numpy, the ghost
+    cells untouched.  Sums of n terms agree to n ulp of the sum of magnitudes."""
+    dim, t = len(ns), R.np_dtype(dtype)
+    lv = solver.uniform_levels(dim, base, ns)[0]
+    dd, L = R.Domain(dim, ns, lv), R.lib()
+    shape = mesh.padded_shape(len(lv), dim, ns, 2)
+    n = int(np.prod(shape))
+    h = [random_field((n + off,), 61 + k, t) for k in range(3)]
+    dev = [R.DeviceArray.from_host(v) for v in h]
+    x, a, b = (d.ptr + off * t().itemsize for d in dev)
+    xv, av, bv = (v[off:].reshape(shape).copy() for v in h)
+
+    def check(op, want, *args):
+        R.check(getattr(L, op)(dd.h, dtype, x, *args, 2, None))
+        got = dev[0].get()
+        if off:
+            assert got[0] == h[0][0]
+        got = got[off:].reshape(shape)
+        if op == "te_vec_set_with_ghost":
+            xv[...] = want
+        else:
+            mesh.interior(xv, dim)[...] = mesh.interior(np.broadcast_to(want, shape), dim)
+        assert np.allclose(got, xv, rtol=4 * np.finfo(t).eps, atol=8 * np.finfo(t).eps), op
+        xv[...] = got
+
+    check("te_vec_add_scaled", xv + t(0.3) * av, 0.3, a)
+    check("te_vec_add_scaled2", xv + (t(0.3) * av + t(-1.7) * bv), 0.3, a, -1.7, b)
+    check("te_vec_scale_then_add", t(0.9) * xv + av, 0.9, a)
+    check("te_vec_scale_then_add_scaled", t(0.9) * xv + t(0.2) * av, 0.9, 0.2, a)
+    check("te_vec_scale_then_add_scaled2", t(0.9) * xv + t(0.2) * av + t(0.7) * bv, 0.9, 0.2, a, 0.7, b)
+    check("te_vec_add", xv + av, a)
+    check("te_vec_scale", xv * t(1.1), 1.1)
+    check("te_vec_shift", xv + t(0.25), 0.25)
+    X, A = mesh.interior(xv, dim).astype(np.float64), mesh.interior(av, dim).astype(np.float64)
+    out = C.c_double()
+    bound = X.size * np.finfo(np.float64).eps
+    R.check(L.te_vec_dot(dd.h, dtype, x, a, 2, C.byref(out), None))
+    assert abs(out.value - (X * A).sum()) <= bound * np.abs(X * A).sum()
+    R.check(L.te_vec_two_norm(dd.h, dtype, x, 2, C.byref(out), None))
+    assert abs(out.value - np.sqrt((X * X).sum())) <= bound * out.value
+    R.check(L.te_vec_inf_norm(dd.h, dtype, x, 2, C.byref(out), None))
+    assert out.value == max(0.0, X.max())  # Vector::infNorm takes the largest value, not magnitude
+    vol = np.prod(lv["spacings"][:, :dim], axis=1).reshape((-1,) + (1,) * (dim + 1))
+    R.check(L.te_vec_integrate(dd.h, dtype, x, 2, C.byref(out), None))
+    assert abs(out.value - (X * vol).sum()) <= bound * np.abs(X * vol).sum()
+    check("te_vec_copy", av, a)
+    check("te_vec_set", t(-2.5), -2.5)
+    check("te_vec_set_with_ghost", t(1.5), 1.5)
 
 
 @pytest.mark.parametrize("dtype", [R.F64, R.F32])

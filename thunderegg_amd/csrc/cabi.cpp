@@ -22,6 +22,54 @@ namespace te {
 static thread_local std::string g_err;
 void set_error(const std::string& msg) { g_err = msg; }
 
+namespace {
+
+// result slots, cut from page-locked slabs: allocating one per domain would cost more than the
+// domain's tables (a batch makes thousands of domains).  A slab is freed when its last slot
+// comes back.
+constexpr int kSlotBytes = 64, kSlabSlots = 256;
+struct Slab {
+  char* base;
+  std::vector<int> free;
+};
+std::mutex g_slab_mu;
+std::vector<Slab> g_slabs;
+
+}  // namespace
+
+double* take_result()
+{
+  std::lock_guard<std::mutex> lock(g_slab_mu);
+  for (Slab& sl : g_slabs)
+    if (!sl.free.empty()) {
+      const int k = sl.free.back();
+      sl.free.pop_back();
+      return (double*)(sl.base + k * kSlotBytes);
+    }
+  void* p = nullptr;
+  if (hipHostMalloc(&p, kSlotBytes * kSlabSlots, hipHostMallocPortable) != hipSuccess) return nullptr;
+  Slab sl{ (char*)p, {} };
+  for (int k = kSlabSlots - 1; k > 0; k--) sl.free.push_back(k);
+  g_slabs.push_back(std::move(sl));
+  return (double*)p;
+}
+
+void give_result(double* r)
+{
+  std::lock_guard<std::mutex> lock(g_slab_mu);
+  for (size_t i = 0; i < g_slabs.size(); i++) {
+    Slab& sl = g_slabs[i];
+    const long off = (char*)r - sl.base;
+    if (off < 0 || off >= kSlotBytes * kSlabSlots) continue;
+    sl.free.push_back((int)(off / kSlotBytes));
+    if (sl.free.size() == kSlabSlots) {
+      (void)hipHostFree(sl.base);
+      g_slabs.erase(g_slabs.begin() + (long)i);
+    }
+    return;
+  }
+}
+
 int cu_count()
 {
   static std::atomic<int> cus[64];
@@ -260,7 +308,7 @@ int te_domain_create(int dim, const int* ns, int num_ghost, int num_patches, con
     if (e == hipSuccess) e = hipMemcpy(d->d_patches, hp.data(), sizeof(DevPatch) * num_patches, hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) e = hipMalloc(&d->d_scratch, sizeof(double) * kMaxPartials);
-  if (e == hipSuccess) e = hipMalloc(&d->d_result, sizeof(double) * 16);
+  if (e == hipSuccess && !(d->result = take_result())) e = hipErrorOutOfMemory;
   if (e == hipSuccess) e = hipMalloc(&d->d_flags, sizeof(int32_t) * 4);
   if (e == hipSuccess && dim == 2) e = upload_ring(ring_table(d, nullptr, nullptr), &d->d_ring);
   if (e != hipSuccess) {
@@ -277,7 +325,7 @@ int te_domain_destroy(te_domain* d)
   if (!d) return TE_OK;
   if (d->d_patches) (void)hipFree(d->d_patches);
   if (d->d_scratch) (void)hipFree(d->d_scratch);
-  if (d->d_result) (void)hipFree(d->d_result);
+  if (d->result) give_result(d->result);
   if (d->d_flags) (void)hipFree(d->d_flags);
   if (d->d_ring) (void)hipFree(d->d_ring);
   delete d;
@@ -759,10 +807,10 @@ static int reduce_sync(const te_domain* d, int dtype, int op, const void* a, con
     *out = 0.0;
     return TE_OK;
   }
-  int rc = launch_reduce(d, dtype, op, a, b, ncomp, d->d_result, S(s));
+  int rc = launch_reduce(d, dtype, op, a, b, ncomp, d->result, S(s));
   if (rc) return rc;
-  TE_HIP(hipMemcpyAsync(out, d->d_result, sizeof(double), hipMemcpyDeviceToHost, S(s)));
   TE_HIP(hipStreamSynchronize(S(s)));
+  *out = *(const volatile double*)d->result;
   return TE_OK;
 }
 

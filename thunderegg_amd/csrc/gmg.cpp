@@ -1224,9 +1224,9 @@ int te_gmg_cg(te_gmg* g, const double* b, double* x, int use_precond, int max_it
   };
   // dot product (RED_DOT) or two-norm (RED_SUMSQ: the launch returns the square root)
   auto reduce = [&](int op, const double* a, const double* bv, double* out) -> int {
-    TE_RC(launch_reduce(d, TE_F64, op, a, bv, 1, d->d_result, s));
-    TE_HIP(hipMemcpyAsync(out, d->d_result, sizeof(double), hipMemcpyDeviceToHost, s));
+    TE_RC(launch_reduce(d, TE_F64, op, a, bv, 1, d->result, s));
     TE_HIP(hipStreamSynchronize(s));
+    *out = *(const volatile double*)d->result;
     return TE_OK;
   };
   auto apply_a = [&](double* u, double* out) -> int {  // A.apply (PatchOperator.h:126-143)

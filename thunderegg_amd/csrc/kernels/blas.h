@@ -51,7 +51,6 @@ __device__ __forceinline__ double block_reduce(double v)
   return r;
 }
 
-int reduce_grid(const Layout& L);
 int launch_vec_op(const te_domain* d, int dtype, int op, void* x, const void* a, const void* b, double alpha,
                   double beta, double gamma, int ncomp, hipStream_t s);
 int launch_reduce(const te_domain* d, int dtype, int op, const void* a, const void* b, int ncomp, double* d_out,

@@ -14,6 +14,11 @@ namespace te {
 
 void set_error(const std::string& msg);
 
+// 64 bytes of page-locked host memory that every device writes, for results that the host reads
+// after a stream synchronisation (no copy); nullptr when there is none to be had
+double* take_result();
+void give_result(double* r);
+
 #define TE_HIP(call)                                                                                 \
   do {                                                                                               \
     hipError_t e_ = (call);                                                                          \
@@ -76,6 +81,53 @@ __device__ __forceinline__ T& at(T* base, int idx)
   return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (unsigned)idx * (unsigned)sizeof(T));
 }
 
+// x / d for 0 <= x < 2^31 and a fixed d >= 1 as one high product and a shift
+struct FastDiv {
+  unsigned d = 1, mul = 1u << 31, sh = 0;
+  FastDiv() = default;
+  explicit FastDiv(unsigned dd) : d(dd)
+  {
+    while ((1ull << sh) < dd) sh++;
+    // mul = floor(2^(31 + sh) / d) + 1 exceeds 2^(31 + sh) / d by at most 1 <= 2^sh / d, so the
+    // quotient is exact below 2^31
+    mul = (unsigned)((1ull << (31 + sh)) / dd + 1);
+  }
+  __host__ __device__ __forceinline__ int operator()(int x) const
+  {
+    return (int)((((unsigned long long)((unsigned)x << 1) * mul) >> 32) >> sh);
+  }
+};
+
+// The interior cells of a padded vector as items of V consecutive padded values: row after row
+// (ghost rows left out), each row the V-wide groups that cover its cells.  V = 2 (even n[0],
+// so that every row starts a group) puts the row's first and last cell into groups with a ghost.
+struct Rows {
+  FastDiv per_row, ny, nyz;  // groups per row, rows per slice, rows per patch and component
+  int items;                 // groups in all
+  int sx, sy, cs, last;      // last: index of a row's last group
+  Rows() = default;
+  Rows(const Layout& L, int V)
+  {
+    const int nz = L.dim == 3 ? L.n[2] : 1, groups = V == 2 ? L.n[0] / 2 + 1 : L.n[0];
+    per_row = FastDiv(groups);
+    ny = FastDiv(L.n[1]);
+    nyz = FastDiv(L.n[1] * nz);
+    items = groups * L.n[1] * nz * L.np * L.ncomp;
+    sx = L.sx;
+    sy = L.dim == 3 ? L.sy : 0;
+    cs = L.cs;
+    last = groups - 1;
+  }
+  // the padded index of item i's first value; *g: its place in the row
+  template <int V>
+  __device__ __forceinline__ int at(int i, int* g) const
+  {
+    const int row = per_row(i), pc = nyz(row), rem = row - pc * (int)nyz.d, z = ny(rem), y = rem - z * (int)ny.d;
+    *g = i - row * (int)per_row.d;
+    return pc * cs + (sy ? (z + 1) * sy : 0) + (y + 1) * sx + V * *g + (V == 1 ? 1 : 0);
+  }
+};
+
 __host__ __device__ inline int lin(const Layout& L, int p, int c, int x, int y, int z)
 {
   return p * L.ps + c * L.cs + (x + 1) + (y + 1) * L.sx + (L.dim == 3 ? (z + 1) * L.sy : 0);
@@ -93,7 +145,7 @@ struct te_domain {
   int any_coarse_fine = 0;         // some face/edge/corner is a coarse/fine interface
   double* d_scratch = nullptr;     // reduction partials
   unsigned* d_counter = nullptr;   // last-block counter for reductions
-  double* d_result = nullptr;      // reduction results
+  double* result = nullptr;        // a reduction's result: host memory that the kernels write (take_result)
   int32_t* d_flags = nullptr;      // breakdown flags
   int scratch_len = 0;
   int32_t* d_ring = nullptr;       // 2D: ring table (te::ring_table), pq fields 0
