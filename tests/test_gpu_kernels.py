@@ -108,6 +108,44 @@ def test_star_apply(name, ns, neumann):
         assert relerr(dr.get(), rref) <= tol
 
 
+@pytest.mark.parametrize("ns,kind,fill_type", [
+    ((7, 5), R.BILINEAR, R.FACES), ((4, 32), R.BIQUADRATIC, R.CORNERS), ((34, 6), R.BILINEAR, R.CORNERS),
+    ((2, 2, 2), R.TRILINEAR, R.FACES), ((6, 4, 8), R.TRILINEAR, R.EDGES), ((16, 16, 16), R.TRILINEAR, R.CORNERS)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_star_with_fill_is_fill_then_star(ns, kind, fill_type, off):
+    """The operator's launch that fills u's ghosts first: the bits of the ghost fill followed by
+    the operator on the filled ghosts, in u and in the result, for two components, single
+    values instead of pairs (odd rows, vectors one value off) and both residual operands."""
+    dim = len(ns)
+    name = "2d_uniform_2x2_mpi1.json" if ns[0] % 2 else (
+        "2d_uniform_8x8_refined_cross_mpi1.json" if dim == 2 else "3d_mid_refine_4x4x4_mpi1.json")
+    lv = load(name, ns)[1][0]
+    dd, L = R.Domain(dim, ns, lv), R.lib()
+    g = R.GhostFiller(dd, kind, fill_type)
+    shape = mesh.padded_shape(len(lv), dim, ns, 2)
+    n = int(np.prod(shape))
+    for dtype in (R.F64, R.F32):
+        t = R.np_dtype(dtype)
+        u0, f0 = random_field((n + off,), 81, t), random_field((n + off,), 82, t)
+        for neumann in (0, 1):
+            u1, u2, f = (R.DeviceArray.from_host(v) for v in (u0, u0, f0))
+            a1, a2, r1 = (R.DeviceArray.from_host(np.full(n + off, 7, t)) for _ in range(3))
+            p = [d.ptr + off * t().itemsize for d in (u1, u2, f, a1, a2, r1)]
+            R.check(L.te_ghost_fill(g.h, dtype, p[0], 2, None))
+            R.check(L.te_star_apply_patches(g.h, dtype, neumann, p[0], p[3], 2, None))
+            R.check(L.te_star_apply(g.h, dtype, neumann, p[1], p[4], 2, None))
+            assert np.array_equal(u1.get(), u2.get()) and np.array_equal(a1.get(), a2.get())
+            u2.upload(u0)
+            R.check(L.te_residual(g.h, dtype, 0, neumann, None, p[2], p[1], p[5], 2, None))
+            assert np.array_equal(u1.get(), u2.get())
+            want = f0.astype(np.float64)[off:].reshape(shape) - a1.get().astype(np.float64)[off:].reshape(shape)
+            got = r1.get()[off:].reshape(shape)
+            eps = np.finfo(t).eps * (np.abs(a1.get()).max() + np.abs(f0).max())
+            assert np.abs(mesh.interior(got, dim) - mesh.interior(want, dim)).max() <= 2 * eps
+            mesh.interior(got, dim)[...] = 0
+            assert not got.any()  # ghost cells of the output are zero
+
+
 @pytest.mark.parametrize("name,ns", [("2d_uniform_2x2_refined_nw_mpi1.json", (8, 8)),
                                      ("2d_uniform_8x8_refined_cross_mpi1.json", (16, 16)),
                                      ("3d_refined_bnw_2x2x2_mpi1.json", (4, 4, 4))])

@@ -534,8 +534,7 @@ int te_batch_bicgstab(te_batch* B, const double* const* b, double* const* x, int
     const bool m32 = use_precond && G.m32;
     TE_RC(launch_batch_copy(true, G.b, G.d_bptr, G.d_off, G.d_len, ng, G.maxlen, G.s));
     TE_RC(launch_batch_copy(true, G.x, G.d_xptr, G.d_off, G.d_len, ng, G.maxlen, G.s));
-    TE_RC(launch_ghost_fill(G.Fgf, TE_F64, G.x, 1, G.s));
-    TE_RC(launch_star(G.Fgf, TE_F64, TE_F64, TE_F64, B->o.op_kind, B->o.neumann, nullptr, G.b, G.x, G.resid, 1,
+    TE_RC(launch_star(G.Fgf, TE_F64, TE_F64, TE_F64, B->o.op_kind, B->o.neumann, nullptr, G.b, G.x, G.resid, 1, true,
                       G.s));
     TE_RC(launch_bicg(BICG_INIT, G.F, G.scal, G.rhat, G.p, G.resid, G.b, nullptr, nullptr, nullptr, G.pa, G.pb, G.s,
                       TE_F64, m32 ? G.p32 : nullptr, nullptr, 0, nullptr, 0, &G.bmap));

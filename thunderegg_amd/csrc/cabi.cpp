@@ -453,9 +453,7 @@ int te_star_apply(const te_ghost_filler* g, int dtype, int neumann, void* u, voi
 {
   TE_ARG(g && u && f && ncomp >= 1 && ncomp <= 8, "bad argument");
   TE_ARG(u != f, "u and f must be distinct vectors");
-  int rc = launch_ghost_fill(g, dtype, u, ncomp, S(s));
-  if (rc) return rc;
-  return launch_star(g, dtype, dtype, dtype, 0, neumann, nullptr, nullptr, u, f, ncomp, S(s));
+  return launch_star(g, dtype, dtype, dtype, 0, neumann, nullptr, nullptr, u, f, ncomp, true, S(s));
 }
 
 int te_star_apply_patches(const te_ghost_filler* g, int dtype, int neumann, const void* u, void* f, int ncomp,
@@ -463,7 +461,7 @@ int te_star_apply_patches(const te_ghost_filler* g, int dtype, int neumann, cons
 {
   TE_ARG(g && u && f && ncomp >= 1 && ncomp <= 8, "bad argument");
   TE_ARG(u != f, "u and f must be distinct vectors");
-  return launch_star(g, dtype, dtype, dtype, 0, neumann, nullptr, nullptr, u, f, ncomp, S(s));
+  return launch_star(g, dtype, dtype, dtype, 0, neumann, nullptr, nullptr, (void*)u, f, ncomp, false, S(s));
 }
 
 int te_varstar_apply(const te_ghost_filler* g, int dtype, const void* coeffs, void* u, void* f, int ncomp,
@@ -471,9 +469,7 @@ int te_varstar_apply(const te_ghost_filler* g, int dtype, const void* coeffs, vo
 {
   TE_ARG(g && coeffs && u && f && ncomp >= 1 && ncomp <= 8, "bad argument");
   TE_ARG(u != f, "u and f must be distinct vectors");
-  int rc = launch_ghost_fill(g, dtype, u, ncomp, S(s));
-  if (rc) return rc;
-  return launch_star(g, dtype, dtype, dtype, 1, 0, coeffs, nullptr, u, f, ncomp, S(s));
+  return launch_star(g, dtype, dtype, dtype, 1, 0, coeffs, nullptr, u, f, ncomp, true, S(s));
 }
 
 int64_t te_domain_boundary_length(const te_domain* d) { return d ? (int64_t)d->np * boundary_stride(d) : -1; }
@@ -498,9 +494,7 @@ int te_residual(const te_ghost_filler* g, int dtype, int op_kind, int neumann, c
   TE_ARG(g && f && u && r && ncomp >= 1 && ncomp <= 8, "bad argument");
   TE_ARG(op_kind == 0 || coeffs, "VarPoisson needs coefficients");
   TE_ARG(r != u, "r and u must be distinct vectors");
-  int rc = launch_ghost_fill(g, dtype, u, ncomp, S(s));
-  if (rc) return rc;
-  return launch_star(g, dtype, dtype, dtype, op_kind, neumann, coeffs, f, u, r, ncomp, S(s));
+  return launch_star(g, dtype, dtype, dtype, op_kind, neumann, coeffs, f, u, r, ncomp, true, S(s));
 }
 
 // ------------------------------------------------------------------- DFT ----

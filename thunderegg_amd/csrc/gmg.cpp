@@ -148,8 +148,7 @@ int visit(te_gmg* g, int li, const void* f, int dtf, double* u_ext, bool u_zero 
   GLevel& Cv = g->L[li + 1];
   // Cycle::restrict: r = f - A u, then restrict into the coarser level's f
   auto restrict_to_coarse = [&]() -> int {
-    TE_RC(launch_ghost_fill(Lv.gf, Lv.dt, u, 1, g->s));
-    TE_RC(launch_star(Lv.gf, Lv.dt, dtf, Lv.dt, g->o.op_kind, g->o.neumann, Lv.coeffs, f, u, Lv.r, 1, g->s));
+    TE_RC(launch_star(Lv.gf, Lv.dt, dtf, Lv.dt, g->o.op_kind, g->o.neumann, Lv.coeffs, f, u, Lv.r, 1, true, g->s));
     return launch_restrict(Lv.link, Lv.dt, Lv.r, Cv.dt, Cv.f, 1, g->s);
   };
   TE_RC(restrict_to_coarse());
@@ -1099,8 +1098,7 @@ int te_gmg_bicgstab(te_gmg* g, const double* b, double* x, int use_precond, int 
   // path in one launch from the padded b and x, launch_c3_init)
   const bool c3_init = g->c3 && g->xrfly;
   if (!c3_init) {
-    TE_RC(launch_ghost_fill(gf, TE_F64, x, 1, s));
-    TE_RC(launch_star(gf, TE_F64, TE_F64, TE_F64, g->o.op_kind, g->o.neumann, cf, b, x, g->resid, 1, s));
+    TE_RC(launch_star(gf, TE_F64, TE_F64, TE_F64, g->o.op_kind, g->o.neumann, cf, b, x, g->resid, 1, true, s));
   }
   if (g->c3) {
     C3Bicg a{};
@@ -1230,15 +1228,13 @@ int te_gmg_cg(te_gmg* g, const double* b, double* x, int use_precond, int max_it
     return TE_OK;
   };
   auto apply_a = [&](double* u, double* out) -> int {  // A.apply (PatchOperator.h:126-143)
-    TE_RC(launch_ghost_fill(gf, TE_F64, u, 1, s));
-    return launch_star(gf, TE_F64, TE_F64, TE_F64, g->o.op_kind, g->o.neumann, cf, nullptr, u, out, 1, s);
+    return launch_star(gf, TE_F64, TE_F64, TE_F64, g->o.op_kind, g->o.neumann, cf, nullptr, u, out, 1, true, s);
   };
   const bool time_its = g->timer && g->time_its;
   auto t0 = std::chrono::steady_clock::now();
   int num_its = 0, rc = TE_OK;
   // resid = b - A x (A.apply then scaleThenAdd(-1, b), as one residual launch)
-  TE_RC(launch_ghost_fill(gf, TE_F64, x, 1, s));
-  TE_RC(launch_star(gf, TE_F64, TE_F64, TE_F64, g->o.op_kind, g->o.neumann, cf, b, x, resid, 1, s));
+  TE_RC(launch_star(gf, TE_F64, TE_F64, TE_F64, g->o.op_kind, g->o.neumann, cf, b, x, resid, 1, true, s));
   TE_RC(vop(VOP_COPY, x0, x, 0.0));    // initial_guess = x
   TE_RC(vop(VOP_SET, x, nullptr, 0.0));  // x.set(0)
   double r0 = 0.0, rho = 0.0, nr = 0.0;

@@ -5,31 +5,16 @@
 // Terms are summed in the order the reference accumulates them: self terms
 // first (fillGhostCellsForLocalPatch runs before processLocalFills), then the
 // neighbour contributions in the order their calls are enumerated.
+#include <algorithm>
+
 #include "../te_internal.h"
 #include "ghost2d.h"
+#include "ghost3d.h"
 
 namespace te {
 namespace {
 
 constexpr int NB_NORMAL = 0, NB_COARSE = 1;
-
-// cell of the slice on 2D side s at depth k (k = -1 is the ghost layer), tangential t
-__device__ __forceinline__ int side_cell2(const Layout& L, int p, int c, int s, int k, int t)
-{
-  int a = s >> 1, up = s & 1;
-  int ca = up ? L.n[a] - 1 - k : k;
-  return a == 0 ? lin(L, p, c, ca, t, 0) : lin(L, p, c, t, ca, 0);
-}
-
-// 3D side s: free axes are the two other axes in increasing order (i, j).
-__device__ __forceinline__ int side_cell3(const Layout& L, int p, int c, int s, int k, int i, int j)
-{
-  int a = s >> 1, up = s & 1;
-  int ca = up ? L.n[a] - 1 - k : k;
-  if (a == 0) return lin(L, p, c, ca, i, j);
-  if (a == 1) return lin(L, p, c, i, ca, j);
-  return lin(L, p, c, i, j, ca);
-}
 
 // 2D side ghosts: one wavefront per patch walks the patch's ring of side ghost cells
 // (ring_cell order: the two x faces, then the two y faces, so the y faces' ghost rows are
@@ -48,25 +33,7 @@ __global__ void __launch_bounds__(256) ghost_ring_2d(const int4* __restrict__ ri
       int s, t;
       const int4 r = ring[ring_index(p, g, n0, n1, &s, &t)];
       if (r.x < 0) continue;  // a physical side: the operators apply its condition themselves
-      const int a = s >> 1, up = s & 1;
-      const int na = a == 0 ? n0 : n1, nt = a == 0 ? n1 : n0;
-      int bx, by;
-      side_xy(s, 0, t, na, &bx, &by);
-      const int gx = a == 0 ? (up ? n0 : -1) : bx, gy = a == 0 ? by : (up ? n1 : -1);
-      for (int c = 0; c < L.ncomp; c++) {
-        T* uc = u + c * L.cs;
-        auto U = [&](int q, int x, int y) { return at(uc, q * L.ps + (y + 1) * L.sx + x + 1); };
-        T v[4] = { T(0), T(0), T(0), T(0) };
-        ghost2d_gather<KIND>(r.x, r.y, r.z, s, t, na, nt, [&](int k, int q, int x, int y) { v[k] = U(q, x, y); });
-        const T G = ghost2d_combine<T, KIND>(r.x, r.y, t, nt,
-                                             [&](int k, int tt) {
-                                               int x, y;
-                                               side_xy(s, k, tt, na, &x, &y);
-                                               return U(p, x, y);
-                                             },
-                                             v);
-        at(uc, p * L.ps + (gy + 1) * L.sx + gx + 1) = G;
-      }
+      fill_ring_cell<T, KIND>(r, s, t, u, L, p);
     }
   }
 }
@@ -106,60 +73,14 @@ __global__ void ghost_corners_2d(const DevPatch* __restrict__ dp, T* __restrict_
   }
 }
 
-// 3D faces, TriLinearGhostFiller.cpp:33-175.
+// 3D faces: one workgroup per patch (fill_faces3), so that the patch's neighbour records are
+// wave-uniform and a cell's place on the face takes one division.
 template <typename T>
-__global__ void __launch_bounds__(256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* __restrict__ u, Layout L,
-                                                      int tmax)
+__global__ void __launch_bounds__(256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L)
 {
-  int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  int per = 6 * tmax * tmax;
-  int p = gid / per;
+  const int p = xcd_item(blockIdx.x, gridDim.x);
   if (p >= L.np) return;
-  int r = gid - p * per;
-  int s = r / (tmax * tmax);
-  r -= s * tmax * tmax;
-  int j = r / tmax;
-  int i = r - j * tmax;
-  int a = s >> 1;
-  int f0 = a == 0 ? 1 : 0, f1 = a == 2 ? 1 : 2;
-  int ni = L.n[f0], nj = L.n[f1];
-  if (i >= ni || j >= nj) return;
-  int slot = 20 + s;
-  int type = dp[p].type[slot];
-  if (type < 0) return;
-  for (int c = 0; c < L.ncomp; c++) {
-    T G;
-    if (type == NB_NORMAL) {
-      G = u[side_cell3(L, dp[p].nbr[slot][0], c, s ^ 1, 0, i, j)];
-    } else if (type == NB_COARSE) {
-      int q = dp[p].nbr[slot][0];
-      int o = dp[p].orth[slot];
-      int oi = (o & 1) ? ni : 0, oj = (o & 2) ? nj : 0;
-      int pi = ((i + oi) % 2 == 0) ? i + 1 : i - 1;
-      int pj = ((j + oj) % 2 == 0) ? j + 1 : j - 1;
-      G = T(0);
-      G += T(5.0 / 6.0) * u[side_cell3(L, p, c, s, 0, i, j)];
-      G -= T(1.0 / 6.0) * u[side_cell3(L, p, c, s, 0, pi, j)];
-      G -= T(1.0 / 6.0) * u[side_cell3(L, p, c, s, 0, i, pj)];
-      G -= T(1.0 / 6.0) * u[side_cell3(L, p, c, s, 0, pi, pj)];
-      G += T(4.0 / 6.0) * u[side_cell3(L, q, c, s ^ 1, 0, (i + oi) / 2, (j + oj) / 2)];
-    } else {
-      G = T(0);
-      G -= T(1.0 / 3.0) * u[side_cell3(L, p, c, s, 0, i, j)];
-      for (int o = 0; o < 4; o++) {
-        int q = dp[p].nbr[slot][o];
-        int oi = (o & 1) ? ni : 0, oj = (o & 2) ? nj : 0;
-        for (int fj = 2 * j - oj; fj <= 2 * j - oj + 1; fj++) {
-          if (fj < 0 || fj >= nj) continue;
-          for (int fi = 2 * i - oi; fi <= 2 * i - oi + 1; fi++) {
-            if (fi < 0 || fi >= ni) continue;
-            G += T(1.0 / 3.0) * u[side_cell3(L, q, c, s ^ 1, 0, fi, fj)];
-          }
-        }
-      }
-    }
-    u[side_cell3(L, p, c, s, -1, i, j)] = G;
-  }
+  fill_faces3<T>(L, dp[p], u, p, threadIdx.x, blockDim.x);
 }
 
 // 3D edge e (Face<3,1>): free axis = e >> 2; fixed sides in axis order with
@@ -253,7 +174,7 @@ __global__ void ghost_lowdim_3d(const DevPatch* __restrict__ dp, T* __restrict__
 }
 
 template <typename T>
-int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, hipStream_t s)
+int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, hipStream_t s)
 {
   const te_domain* d = g->d;
   if (d->np == 0) return TE_OK;
@@ -263,7 +184,8 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, hipStream_t s)
     // a wave per patch (4 per workgroup), at most 8192 workgroups walking the rest
     const int ngroups = (d->np + 3) / 4;
     const int grid = ngroups < 8192 ? ngroups : 8192;
-    if (g->kind == TE_BILINEAR)
+    if (!faces) {
+    } else if (g->kind == TE_BILINEAR)
       hipLaunchKernelGGL((ghost_ring_2d<T, TE_BILINEAR>), dim3(grid), dim3(B), 0, s, (const int4*)d->d_ring, u, L);
     else
       hipLaunchKernelGGL((ghost_ring_2d<T, TE_BIQUADRATIC>), dim3(grid), dim3(B), 0, s, (const int4*)d->d_ring, u,
@@ -276,12 +198,14 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, hipStream_t s)
         hipLaunchKernelGGL((ghost_corners_2d<T, TE_BIQUADRATIC>), dim3(cg), dim3(B), 0, s, d->d_patches, u, L);
     }
   } else {
-    int tmax = d->ns[0];
-    for (int a = 1; a < 3; a++) tmax = d->ns[a] > tmax ? d->ns[a] : tmax;
-    long total = (long)d->np * 6 * tmax * tmax;
-    int grid = (int)((total + B - 1) / B);
-    hipLaunchKernelGGL((ghost_faces_3d<T>), dim3(grid), dim3(B), 0, s, d->d_patches, u, L, tmax);
+    int face = 0;  // cells of the largest face: a thread each, up to 256
+    for (int a = 0; a < 3; a++) face = std::max(face, d->ns[a] * d->ns[(a + 1) % 3]);
+    if (faces)
+      hipLaunchKernelGGL((ghost_faces_3d<T>), dim3(xcd_grid(d->np)), dim3(std::min(256, (face + 63) / 64 * 64)), 0, s,
+                         d->d_patches, u, L);
     if (g->fill_type != TE_FACES) {
+      int tmax = d->ns[0];
+      for (int a = 1; a < 3; a++) tmax = d->ns[a] > tmax ? d->ns[a] : tmax;
       long tl = (long)d->np * (12 * tmax + 8);
       int lg = (int)((tl + B - 1) / B);
       hipLaunchKernelGGL((ghost_lowdim_3d<T>), dim3(lg), dim3(B), 0, s, d->d_patches, u, L, tmax,
@@ -296,8 +220,16 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, hipStream_t s)
 
 int launch_ghost_fill(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s)
 {
-  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, s);
-  return ghost_fill_t<float>(g, (float*)u, ncomp, s);
+  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, true, s);
+  return ghost_fill_t<float>(g, (float*)u, ncomp, true, s);
+}
+
+// the edge and corner ghosts alone (nothing for fill type Faces)
+int launch_ghost_fill_lowdim(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s)
+{
+  if (g->fill_type == TE_FACES) return TE_OK;
+  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, false, s);
+  return ghost_fill_t<float>(g, (float*)u, ncomp, false, s);
 }
 
 }  // namespace te

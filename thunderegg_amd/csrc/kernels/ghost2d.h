@@ -336,6 +336,32 @@ __device__ __forceinline__ int ring_index(int p, int g, int n0, int n1, int* s, 
   return (p * 4 + *s) * 2 + (2 * *t >= nt ? 1 : 0);
 }
 
+// Writes the ghost value of tangential cell t on side s of patch p (record r, r.x >= 0) for every
+// component of u.
+template <typename T, int KIND>
+__device__ __forceinline__ void fill_ring_cell(const int4& r, int s, int t, T* u, const Layout& L, int p)
+{
+  const int n0 = L.n[0], n1 = L.n[1], a = s >> 1, up = s & 1;
+  const int na = a == 0 ? n0 : n1, nt = a == 0 ? n1 : n0;
+  int bx, by;
+  side_xy(s, 0, t, na, &bx, &by);
+  const int gx = a == 0 ? (up ? n0 : -1) : bx, gy = a == 0 ? by : (up ? n1 : -1);
+  for (int c = 0; c < L.ncomp; c++) {
+    T* uc = u + c * L.cs;
+    auto U = [&](int q, int x, int y) { return at(uc, q * L.ps + (y + 1) * L.sx + x + 1); };
+    T v[4] = { T(0), T(0), T(0), T(0) };
+    ghost2d_gather<KIND>(r.x, r.y, r.z, s, t, na, nt, [&](int k, int q, int x, int y) { v[k] = U(q, x, y); });
+    const T G = ghost2d_combine<T, KIND>(r.x, r.y, t, nt,
+                                         [&](int k, int tt) {
+                                           int x, y;
+                                           side_xy(s, k, tt, na, &x, &y);
+                                           return U(p, x, y);
+                                         },
+                                         v);
+    at(uc, p * L.ps + (gy + 1) * L.sx + gx + 1) = G;
+  }
+}
+
 // The neighbour values ring cell g of a patch needs (record r), read from u (widened to T).
 template <typename T, int KIND, typename TU>
 __device__ __forceinline__ void ring_gather_plain(const int4& r, int g, int n0, int n1, const TU* __restrict__ u,

@@ -1,0 +1,83 @@
+// 3D face ghosts (TriLinearGhostFiller.cpp:33-175) as a gather: the value of ghost cell (i, j) on
+// side s of a patch from its own and its neighbours' interior cells, the terms in the order the
+// reference accumulates them (self terms, then the neighbours').
+#pragma once
+
+#include "../te_internal.h"
+
+namespace te {
+
+// cell (i, j) of the slice on side s at depth k (k = -1: the ghost layer); the free axes are the
+// two other axes in increasing order
+__device__ __forceinline__ int side_cell3(const Layout& L, int p, int c, int s, int k, int i, int j)
+{
+  int a = s >> 1, up = s & 1;
+  int ca = up ? L.n[a] - 1 - k : k;
+  if (a == 0) return lin(L, p, c, ca, i, j);
+  if (a == 1) return lin(L, p, c, i, ca, j);
+  return lin(L, p, c, i, j, ca);
+}
+
+// type 0 same level (neighbour q[0]), 1 coarser (q[0], orth: where on its side), 2 finer (q[0..3])
+template <typename T>
+__device__ __forceinline__ T face_ghost3(const Layout& L, int type, int orth, const int* q, const T* u, int p, int c,
+                                         int s, int i, int j)
+{
+  const int a = s >> 1, ni = L.n[a == 0 ? 1 : 0], nj = L.n[a == 2 ? 1 : 2];
+  auto U = [&](int qq, int side, int ii, int jj) { return at(u, side_cell3(L, qq, c, side, 0, ii, jj)); };
+  if (type == 0) return U(q[0], s ^ 1, i, j);
+  T G = T(0);
+  if (type == 1) {
+    const int oi = (orth & 1) ? ni : 0, oj = (orth & 2) ? nj : 0;
+    const int pi = ((i + oi) % 2 == 0) ? i + 1 : i - 1;
+    const int pj = ((j + oj) % 2 == 0) ? j + 1 : j - 1;
+    G += T(5.0 / 6.0) * U(p, s, i, j);
+    G -= T(1.0 / 6.0) * U(p, s, pi, j);
+    G -= T(1.0 / 6.0) * U(p, s, i, pj);
+    G -= T(1.0 / 6.0) * U(p, s, pi, pj);
+    G += T(4.0 / 6.0) * U(q[0], s ^ 1, (i + oi) / 2, (j + oj) / 2);
+    return G;
+  }
+  // the 2 x 2 fine cells against it: even cells per side (TriLinearGhostFiller.cpp:576-584), so
+  // all four lie in the finer neighbour that covers this quarter of the side
+  const int hi = 2 * i >= ni, hj = 2 * j >= nj;
+  const int fq = q[hi + 2 * hj], fi = 2 * i - (hi ? ni : 0), fj = 2 * j - (hj ? nj : 0);
+  G -= T(1.0 / 3.0) * U(p, s, i, j);
+#pragma unroll
+  for (int dj = 0; dj < 2; dj++)
+#pragma unroll
+    for (int di = 0; di < 2; di++) G += T(1.0 / 3.0) * U(fq, s ^ 1, fi + di, fj + dj);
+  return G;
+}
+
+// The face ghosts of patch p, by the nt threads t = 0 .. nt - 1: each thread
+// takes the same cell of all six sides, so that their loads are in flight together.
+template <typename T>
+__device__ __forceinline__ void fill_faces3(const Layout& L, const DevPatch& P, T* u, int p, int t, int nt)
+{
+  int cells[6], most = 0;
+#pragma unroll
+  for (int s = 0; s < 6; s++) {
+    const int a = s >> 1;
+    cells[s] = P.type[20 + s] < 0 ? 0 : L.n[a == 0 ? 1 : 0] * L.n[a == 2 ? 1 : 2];
+    most = cells[s] > most ? cells[s] : most;
+  }
+  for (int c = 0; c < L.ncomp; c++)
+    for (int k = t; k < most; k += nt) {
+      T G[6];
+#pragma unroll
+      for (int s = 0; s < 6; s++) {
+        if (k >= cells[s]) continue;
+        const int ni = L.n[s < 2 ? 1 : 0], j = k / ni;
+        G[s] = face_ghost3<T>(L, P.type[20 + s], P.orth[20 + s], P.nbr[20 + s], u, p, c, s, k - j * ni, j);
+      }
+#pragma unroll
+      for (int s = 0; s < 6; s++) {
+        if (k >= cells[s]) continue;
+        const int ni = L.n[s < 2 ? 1 : 0], j = k / ni;
+        at(u, side_cell3(L, p, c, s, -1, k - j * ni, j)) = G[s];
+      }
+    }
+}
+
+}  // namespace te

@@ -1,97 +1,200 @@
 // Star stencils: Poisson (Poisson/StarPatchOperator.h:75-101) and VarPoisson
 // (VarPoisson/StarPatchOperator.h:61-109), 5-point in 2D and 7-point in 3D,
 // optionally fused with the residual r = f - A u of Cycle::restrict
-// (GMG/Cycle.h:57-65).  One thread per padded cell: ghost cells of the output
-// are written 0 (f.setWithGhost(0), PatchOperator.h:136), interior cells get
+// (GMG/Cycle.h:57-65) and with the ghost fill before it (PatchOperator.h:126-143).  Ghost cells
+// of the output are written 0 (f.setWithGhost(0), PatchOperator.h:136), interior cells get
 // the stencil.  Physical-boundary ghosts of u are applied inline
 // (enforceBoundaryConditions, :115-144): -u (Dirichlet) or +u (Neumann).
+#include <algorithm>
+
 #include "../te_internal.h"
+#include "ghost2d.h"
+#include "ghost3d.h"
 
 namespace te {
 namespace {
 
-template <typename T, typename TF, typename TO, int D, int OP, bool RESID>
-__global__ void __launch_bounds__(256) star_kernel(const DevPatch* __restrict__ dp, const T* __restrict__ u,
+constexpr int kNoFill = -1;
+
+// One patch per workgroup (3D) or per wavefront (2D), so that its neighbour records and spacings
+// are wave-uniform and a cell's place takes one or two multiply-shift divisions.  FILL (a
+// te_filler_kind): the patch's own side ghosts first, written to u for the caller; they depend
+// on interior cells only, so no patch waits for another's, and the stencil then reads them back
+// from this workgroup's cache.  The stencil runs over the padded patch in groups of V = 2
+// values (rows of even length start on them): one 16-byte (FP64) or 8-byte access per row
+// neighbour and for the output, kStarItems groups in flight a thread.  Patches go to the XCDs in
+// contiguous eighths (xcd_item), which takes 9 to 10 us off both cases below: the ghost phase
+// reads most of the neighbours' lines.
+// A u with ghosts, two launches of one thread per cell before / this one: 2,535 patches of 16^3
+// (refined octree, FP32) 117 / 45 us, of which the stencil alone 74 / 26 (a copy of the padded
+// vector takes 23); 19,543 patches of 16^2 (refined quadtree, FP64) 56 / 30 us.
+// Marching each thread along z (three rows' loads together) was 3 to 4 us slower in 3D.
+constexpr int kStarItems = 2;
+
+template <typename T, typename TF, typename TO, int D, int OP, int FILL, int V>
+__global__ void __launch_bounds__(256) star_kernel(const DevPatch* __restrict__ dp, const int4* __restrict__ ring, T* u,
                                                    const T* __restrict__ cf, const TF* __restrict__ fin,
-                                                   TO* __restrict__ out, Layout L, int neumann)
+                                                   TO* __restrict__ out, Layout L, int neumann, FastDiv per_row,
+                                                   FastDiv rows)
 {
-  long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long total = (long)L.np * L.ps;
-  if (gid >= total) return;
-  int idx = (int)gid;
-  int p = idx / L.ps;
-  int rem = idx - p * L.ps;
-  int c = rem / L.cs;
-  int q = rem - c * L.cs;
-  int x, y, z = 0;
-  if (D == 2) {
-    y = q / L.sx;
-    x = q - y * L.sx;
-  } else {
-    z = q / L.sy;
-    int r2 = q - z * L.sy;
-    y = r2 / L.sx;
-    x = r2 - y * L.sx;
-    z -= 1;
-  }
-  x -= 1;
-  y -= 1;
-  bool inter = x >= 0 && x < L.n[0] && y >= 0 && y < L.n[1] && (D == 2 || (z >= 0 && z < L.n[2]));
-  if (!inter) {
-    out[idx] = TO(0);
-    return;
-  }
+  constexpr bool WAVE = D == 2;
+  const int b = xcd_item(blockIdx.x, gridDim.x);
+  const int p = WAVE ? __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6)) : b;
+  if (p >= L.np) return;
+  const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
   const DevPatch& P = dp[p];
-  T mid = u[idx];
-  T bc = (OP == 0 && neumann) ? mid : -mid;
-  int coord[3] = { x, y, z };
-  int st[3] = { 1, L.sx, L.sy };
-  T acc = T(0);
-#pragma unroll
-  for (int a = 0; a < D; a++) {
-    bool lo_phys = coord[a] == 0 && P.type[(D == 2 ? 4 : 20) + 2 * a] < 0;
-    bool hi_phys = coord[a] == L.n[a] - 1 && P.type[(D == 2 ? 4 : 20) + 2 * a + 1] < 0;
-    T lower = lo_phys ? bc : u[idx - st[a]];
-    T upper = hi_phys ? bc : u[idx + st[a]];
-    T ih2 = T(P.inv_h2[a]);
-    if (OP == 0) {
-      acc += (upper - T(2) * mid + lower) * ih2;
+  if (FILL != kNoFill) {
+    if (D == 2) {
+      const int nr = 2 * (L.n[0] + L.n[1]);
+      for (int g = t; g < nr; g += 64) {
+        int s, tt;
+        const int4 r = ring[ring_index(p, g, L.n[0], L.n[1], &s, &tt)];
+        if (r.x >= 0) fill_ring_cell<T, FILL == TE_BILINEAR ? TE_BILINEAR : TE_BIQUADRATIC>(r, s, tt, u, L, p);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // one wave wrote what it reads below
     } else {
-      T cm = cf[p * L.cs + q];
-      T cl = cf[p * L.cs + q - st[a]];
-      T cu = cf[p * L.cs + q + st[a]];
-      acc += ((cu + cm) * (upper - mid) - (cl + cm) * (mid - lower)) * (ih2 * T(0.5));
+      fill_faces3<T>(L, P, u, p, t, nt);
+      __syncthreads();
     }
   }
-  if (RESID) out[idx] = TO(T(fin[idx]) - acc);
-  else out[idx] = TO(acc);
+  constexpr int SB = D == 2 ? 4 : 20;
+  bool phys[2 * D];
+  T ih2[D];
+#pragma unroll
+  for (int a = 0; a < D; a++) {
+    ih2[a] = T(P.inv_h2[a]);
+    phys[2 * a] = P.type[SB + 2 * a] < 0;
+    phys[2 * a + 1] = P.type[SB + 2 * a + 1] < 0;
+  }
+  const T bs = (OP == 0 && neumann) ? T(1) : T(-1);
+  const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1;
+  const int per = (n0 + 2) / V, items = per * (n1 + 2) * (D == 3 ? n2 + 2 : 1);
+  for (int c = 0; c < L.ncomp; c++) {
+    const int base = p * L.ps + c * L.cs, cbase = p * L.cs;
+    for (int i0 = t; i0 < items; i0 += kStarItems * nt) {
+      // row neighbours of a group: below / above along y and z; single values left and right of it
+      T m[kStarItems][V], yl[kStarItems][V], yu[kStarItems][V], zl[kStarItems][V], zu[kStarItems][V];
+      T lf[kStarItems], rt[kStarItems];
+      TF fv[kStarItems][V];
+      int xx[kStarItems], yy[kStarItems], zz[kStarItems];
+      bool in[kStarItems];
+      auto load = [](auto& dst, const auto* src) {
+        typedef typename std::remove_const<typename std::remove_reference<decltype(*src)>::type>::type E;
+        if (V == 2) {
+          typedef E E2 __attribute__((ext_vector_type(2)));
+          const E2 v = *reinterpret_cast<const E2*>(src);
+          dst[0] = v[0];
+          dst[V - 1] = v[1];
+        } else {
+          dst[0] = *src;
+        }
+      };
+#pragma unroll
+      for (int k = 0; k < kStarItems; k++) {
+        const int i = i0 + k * nt;
+        const int row = per_row(i);
+        zz[k] = D == 3 ? rows(row) : 1;
+        yy[k] = D == 3 ? row - zz[k] * (n1 + 2) : row;
+        xx[k] = V * (i - row * per) - 1;
+        in[k] = i < items && yy[k] >= 1 && yy[k] <= n1 && zz[k] >= 1 && zz[k] <= n2;
+        if (V == 1) in[k] = in[k] && xx[k] >= 0 && xx[k] < n0;
+        if (!in[k]) continue;
+        const T* q = u + base + V * i;
+        load(m[k], q);
+        load(yl[k], q - L.sx);
+        load(yu[k], q + L.sx);
+        if (D == 3) {
+          load(zl[k], q - L.sy);
+          load(zu[k], q + L.sy);
+        }
+        lf[k] = q[-1];
+        rt[k] = q[V];
+        if (fin) load(fv[k], fin + base + V * i);
+      }
+#pragma unroll
+      for (int k = 0; k < kStarItems; k++) {
+        const int i = i0 + k * nt;
+        if (i >= items) continue;
+        TO res[V];
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+          res[j] = TO(0);
+          const int x = xx[k] + j;
+          if (!in[k] || x < 0 || x >= n0) continue;
+          const T mid = m[k][j];
+          const T bc = bs * mid;
+          T acc = T(0);
+          auto axis = [&](int a, T lower, T upper, int cells, int at0, int st) {
+            if (at0 == 0 && phys[2 * a]) lower = bc;
+            if (at0 == cells - 1 && phys[2 * a + 1]) upper = bc;
+            if (OP == 0) {
+              acc += (upper - T(2) * mid + lower) * ih2[a];
+            } else {
+              const int ci = cbase + V * i + j;
+              const T cm = at(cf, ci), cl = at(cf, ci - st), cu = at(cf, ci + st);
+              acc += ((cu + cm) * (upper - mid) - (cl + cm) * (mid - lower)) * (ih2[a] * T(0.5));
+            }
+          };
+          axis(0, j == 0 ? lf[k] : m[k][0], j == V - 1 ? rt[k] : m[k][V - 1], n0, x, 1);
+          axis(1, yl[k][j], yu[k][j], n1, yy[k] - 1, L.sx);
+          if (D == 3) axis(D - 1, zl[k][j], zu[k][j], n2, zz[k] - 1, L.sy);
+          res[j] = fin ? TO(T(fv[k][j]) - acc) : TO(acc);
+        }
+        TO* o = out + base + V * i;
+        if (V == 2) {
+          typedef TO O2 __attribute__((ext_vector_type(2)));
+          O2 w;
+          w[0] = res[0];
+          w[1] = res[V - 1];
+          *reinterpret_cast<O2*>(o) = w;
+        } else {
+          *o = res[0];
+        }
+      }
+    }
+  }
 }
 
-template <typename T, typename TF, typename TO, int D, int OP, bool RESID>
-void launch_one(const te_domain* d, const T* u, const T* cf, const TF* fin, TO* out, int ncomp, int neumann,
+template <typename T, typename TF, typename TO, int D, int OP>
+void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* out, int ncomp, int neumann, bool fill,
                 hipStream_t s)
 {
+  const te_domain* d = g->d;
   Layout L = make_layout(d->dim, d->ns, ncomp, d->np);
-  long total = (long)L.np * L.ps;
-  const int B = 256;
-  int grid = (int)((total + B - 1) / B);
-  hipLaunchKernelGGL((star_kernel<T, TF, TO, D, OP, RESID>), dim3(grid), dim3(B), 0, s, d->d_patches, u, cf, fin,
-                     out, L, neumann);
+  const bool pairs = L.n[0] % 2 == 0 && (uintptr_t)u % (2 * sizeof(T)) == 0 && (uintptr_t)fin % (2 * sizeof(TF)) == 0 &&
+                     (uintptr_t)out % (2 * sizeof(TO)) == 0;
+  const int V = pairs ? 2 : 1, per = (L.n[0] + 2) / V;
+  const int items = per * (L.n[1] + 2) * (D == 3 ? L.n[2] + 2 : 1);
+  // 3D: kStarItems groups or more a thread, up to 256 threads
+  const int block = D == 2 ? 256 : std::min(256, (items / kStarItems + 63) / 64 * 64);
+  const int grid = xcd_grid(D == 2 ? (d->np + 3) / 4 : d->np);
+#define TE_ST(F_, V_)                                                                                               \
+  hipLaunchKernelGGL((star_kernel<T, TF, TO, D, OP, F_, V_>), dim3(grid), dim3(block), 0, s, d->d_patches,          \
+                     (const int4*)d->d_ring, u, cf, fin, out, L, neumann, FastDiv(per), FastDiv(L.n[1] + 2))
+#define TE_SF(F_)          \
+  do {                     \
+    if (V == 2) TE_ST(F_, 2); \
+    else TE_ST(F_, 1);     \
+  } while (0)
+  if (!fill) TE_SF(kNoFill);
+  else if (D == 3) TE_SF((D == 3 ? TE_TRILINEAR : kNoFill));
+  else if (g->kind == TE_BILINEAR) TE_SF((D == 2 ? TE_BILINEAR : kNoFill));
+  else TE_SF((D == 2 ? TE_BIQUADRATIC : kNoFill));
+#undef TE_SF
+#undef TE_ST
 }
 
 template <typename T, typename TF, typename TO>
-void launch_dim(const te_domain* d, int op_kind, bool resid, const T* u, const T* cf, const TF* fin, TO* out,
-                int ncomp, int neumann, hipStream_t s)
+void launch_dim(const te_ghost_filler* g, int op_kind, T* u, const T* cf, const TF* fin, TO* out, int ncomp,
+                int neumann, bool fill, hipStream_t s)
 {
-#define TE_L(D_, OP_, R_) launch_one<T, TF, TO, D_, OP_, R_>(d, u, cf, fin, out, ncomp, neumann, s)
-  if (d->dim == 2) {
-    if (op_kind == 0) { if (resid) TE_L(2, 0, true); else TE_L(2, 0, false); }
-    else { if (resid) TE_L(2, 1, true); else TE_L(2, 1, false); }
+  if (g->d->dim == 2) {
+    if (op_kind == 0) launch_one<T, TF, TO, 2, 0>(g, u, cf, fin, out, ncomp, neumann, fill, s);
+    else launch_one<T, TF, TO, 2, 1>(g, u, cf, fin, out, ncomp, neumann, fill, s);
   } else {
-    if (op_kind == 0) { if (resid) TE_L(3, 0, true); else TE_L(3, 0, false); }
-    else { if (resid) TE_L(3, 1, true); else TE_L(3, 1, false); }
+    if (op_kind == 0) launch_one<T, TF, TO, 3, 0>(g, u, cf, fin, out, ncomp, neumann, fill, s);
+    else launch_one<T, TF, TO, 3, 1>(g, u, cf, fin, out, ncomp, neumann, fill, s);
   }
-#undef TE_L
 }
 
 }  // namespace
@@ -99,20 +202,22 @@ void launch_dim(const te_domain* d, int op_kind, bool resid, const T* u, const T
 // fin != nullptr: out = fin - A u (residual); else out = A u.  dt: type of u and coeffs,
 // dtf: type of fin, dto: type of out.  Supported: (f64,f64,f64), (f32,f32,f32), (f32,f64,f32).
 int launch_star(const te_ghost_filler* g, int dt, int dtf, int dto, int op_kind, int neumann, const void* coeffs,
-                const void* fin, const void* u, void* out, int ncomp, hipStream_t s)
+                const void* fin, void* u, void* out, int ncomp, bool fill, hipStream_t s)
 {
-  const te_domain* d = g->d;
-  if (d->np == 0) return TE_OK;
-  bool resid = fin != nullptr;
+  if (g->d->np == 0) return TE_OK;
+  if (fill) {
+    int rc = launch_ghost_fill_lowdim(g, dt, u, ncomp, s);
+    if (rc) return rc;
+  }
   if (dt == TE_F64 && dtf == TE_F64 && dto == TE_F64)
-    launch_dim<double, double, double>(d, op_kind, resid, (const double*)u, (const double*)coeffs,
-                                       (const double*)fin, (double*)out, ncomp, neumann, s);
+    launch_dim<double, double, double>(g, op_kind, (double*)u, (const double*)coeffs, (const double*)fin, (double*)out,
+                                       ncomp, neumann, fill, s);
   else if (dt == TE_F32 && dtf == TE_F32 && dto == TE_F32)
-    launch_dim<float, float, float>(d, op_kind, resid, (const float*)u, (const float*)coeffs, (const float*)fin,
-                                    (float*)out, ncomp, neumann, s);
+    launch_dim<float, float, float>(g, op_kind, (float*)u, (const float*)coeffs, (const float*)fin, (float*)out, ncomp,
+                                    neumann, fill, s);
   else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F32)
-    launch_dim<float, double, float>(d, op_kind, resid, (const float*)u, (const float*)coeffs,
-                                     (const double*)fin, (float*)out, ncomp, neumann, s);
+    launch_dim<float, double, float>(g, op_kind, (float*)u, (const float*)coeffs, (const double*)fin, (float*)out,
+                                     ncomp, neumann, fill, s);
   else {
     set_error("unsupported dtype combination for the star stencil");
     return TE_ERR_UNSUPPORTED;

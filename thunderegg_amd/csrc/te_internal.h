@@ -98,6 +98,12 @@ struct FastDiv {
   }
 };
 
+// The item of workgroup b when the grid is 8 * ceil(n / 8) workgroups and XCD x (workgroups are
+// dealt round-robin over the 8) takes the x-th contiguous eighth of n items: patches are in
+// Morton order, so most neighbours are then read through the same L2.  n or more: no item.
+__host__ __device__ inline int xcd_grid(int n) { return (n + 7) / 8 * 8; }
+__device__ __forceinline__ int xcd_item(int b, int grid) { return (b & 7) * (grid >> 3) + (b >> 3); }
+
 // The interior cells of a padded vector as items of V consecutive padded values: row after row
 // (ghost rows left out), each row the V-wide groups that cover its cells.  V = 2 (even n[0],
 // so that every row starts a group) puts the row's first and last cell into groups with a ghost.
@@ -194,8 +200,11 @@ bool timer_has_domain(const te_timer* t, int domain_id);
 
 // ---- launchers (defined in kernels/*.hip) ----
 int launch_ghost_fill(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s);
+int launch_ghost_fill_lowdim(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s);
+// out = A u, or fin - A u where fin is given.  fill: u's ghosts are filled first (as
+// launch_ghost_fill) in the same launch; otherwise they are read as they are.
 int launch_star(const te_ghost_filler* g, int dt, int dtf, int dto, int op_kind, int neumann, const void* coeffs,
-                const void* fin, const void* u, void* out, int ncomp, hipStream_t s);
+                const void* fin, void* u, void* out, int ncomp, bool fill, hipStream_t s);
 // extrapolate: LinearRestrictor's extrapolate_boundary_ghosts
 int launch_restrict(const te_level_link* l, int dtype_in, const void* fine, int dtype_out, void* coarse, int ncomp,
                     hipStream_t s, bool extrapolate = false);
