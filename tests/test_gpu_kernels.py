@@ -200,6 +200,34 @@ def test_restrict_interpolate(name, ns):
             assert relerr(dfv.get(), fref) <= tol
 
 
+@pytest.mark.parametrize("ns", [(2, 2), (4, 10), (16, 16), (5, 7), (2, 4, 6), (16, 16, 16), (6, 3, 5)])
+@pytest.mark.parametrize("ncomp", [1, 3])
+def test_transfer_shapes(ns, ncomp):
+    """Restriction and interpolation between the two finest levels of a mesh with copied and
+    with refined children: FP64 has the oracle's bits (dividing by 2^D is exact and the sums run in
+    its order), FP32 stays within the roundings of its at most 8 additions.  Odd sizes
+    interpolate value by value (their restriction adds two children into a cell, in the oracle
+    in no fixed order)."""
+    dim = len(ns)
+    name = "2d_uniform_8x8_refined_cross_mpi1.json" if dim == 2 else "3d_mid_refine_4x4x4_mpi1.json"
+    lv = load(name, ns)[1][:2]
+    of, oc = (O.Domain(dim, ns, v) for v in lv)
+    of.link_parents(oc)
+    link = R.LevelLink(*(R.Domain(dim, ns, v) for v in lv))
+    f0, c0 = random_field(of.shape(ncomp), 91), random_field(oc.shape(ncomp), 92)
+    for t in (np.float64, np.float32):
+        f, c = f0.astype(t).astype(np.float64), c0.astype(t).astype(np.float64)
+        cref, fref = O.restrict(of, oc, f), f.copy()
+        O.interpolate(oc, of, c, fref)
+        df, dc, dr = (R.DeviceArray.from_host(v.astype(t)) for v in (f, c, c))
+        link.restrict(df, dr)
+        link.interpolate(dc, df)
+        even = all(v % 2 == 0 for v in ns)
+        if t == np.float64:
+            assert np.array_equal(df.get(), fref) and (not even or np.array_equal(dr.get(), cref))
+        assert relerr(df.get(), fref) <= 2.0**-24 and (not even or relerr(dr.get(), cref) <= 8 * 2.0**-24)
+
+
 @pytest.mark.parametrize("name,ns", [("2d_uniform_2x2_mpi1.json", (8, 8)),
                                      ("2d_uniform_2x2_refined_nw_mpi1.json", (16, 16)),
                                      ("2d_uniform_8x8_refined_cross_mpi1.json", (32, 32)),

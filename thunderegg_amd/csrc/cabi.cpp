@@ -359,6 +359,7 @@ int te_level_link_create(const te_domain* fine, const te_domain* coarse, te_leve
   l->fine = fine;
   l->coarse = coarse;
   l->parent.resize(fine->np);
+  for (int a = 0; a < fine->dim; a++) l->regular = l->regular && fine->ns[a] % 2 == 0;
   std::vector<int32_t> orth(fine->np), child((size_t)coarse->np * 8, -1), nchild(coarse->np, 0);
   for (int i = 0; i < fine->np; i++) {
     auto it = cid.find(fine->patches[i].parent_id);
@@ -374,6 +375,12 @@ int te_level_link_create(const te_domain* fine, const te_domain* coarse, te_leve
       delete l;
       set_error("too many children for coarse patch " + std::to_string(coarse->patches[cp].id));
       return TE_ERR_ARG;
+    }
+    const int o = orth[i];
+    if (o >= (1 << fine->dim)) l->regular = false;
+    for (int k = 0; k < nchild[cp]; k++) {
+      const int q = orth[child[(size_t)cp * 8 + k]];
+      if (o < 0 || q < 0 || q == o) l->regular = false;
     }
     child[(size_t)cp * 8 + nchild[cp]++] = i;  // fine local order = increasing
   }

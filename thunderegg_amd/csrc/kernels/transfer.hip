@@ -11,6 +11,8 @@
 //  - DirectInterpolator (GMG/DirectInterpolator.h:60-91): fine[i] += coarse[(i+s)/2].
 // Children of a coarse patch are visited in increasing fine local index and fine
 // cells in x-fastest order, the order in which the reference accumulates them.
+#include <algorithm>
+
 #include "../te_internal.h"
 
 namespace te {
@@ -149,44 +151,163 @@ __global__ void __launch_bounds__(256) restrict_kernel(const int32_t* __restrict
   coarse[idx] = TO(acc);
 }
 
-template <typename TC, typename TF, int D>
+// V values of type T from addresses that are multiples of T only: one access
+template <typename T, int V, class Out>
+__device__ __forceinline__ void load_at(const T* q, Out put)
+{
+  if (V == 2) {
+    typedef T T2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    const T2 v = *reinterpret_cast<const T2*>(q);
+    put(0, v[0]);
+    put(1, v[1]);
+  } else {
+    put(0, *q);
+  }
+}
+template <typename T, int V, class Get>
+__device__ __forceinline__ void store_at(T* q, Get get)
+{
+  if (V == 2) {
+    typedef T T2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    T2 v;
+    v[0] = get(0);
+    v[1] = get(1);
+    *reinterpret_cast<T2*>(q) = v;
+  } else {
+    *q = get(0);
+  }
+}
+
+// One patch per workgroup (3D) or wavefront (2D) in both kernels below, so that the link's
+// records are wave-uniform, and pairs of values along rows (even cells per side).
+
+// Restriction where every coarse cell has one child over it (te_level_link::regular): a thread
+// forms the two coarse cells of an aligned pair, each from 2^(D - 1) accesses of two fine cells,
+// in the order of the general kernel above.
+template <typename TI, typename TO, int D>
+__global__ void __launch_bounds__(256) restrict_regular_kernel(const int32_t* __restrict__ child,
+                                                               const int32_t* __restrict__ nchild,
+                                                               const int32_t* __restrict__ orth,
+                                                               const TI* __restrict__ fine, TO* __restrict__ coarse,
+                                                               Layout L, int np_coarse, FastDiv per_row, FastDiv rows)
+{
+  constexpr bool WAVE = D == 2;
+  __shared__ int tabs[4][8];  // child of each octant of the patch(es), -1: none
+  const int b = xcd_item(blockIdx.x, gridDim.x);
+  const int w = WAVE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int p = WAVE ? b * 4 + w : b;
+  const bool live = p < np_coarse;
+  const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
+  const int nc = live ? nchild[p] : 0;
+  const bool copy = nc == 1 && orth[child[p * 8]] < 0;
+  if (t < 8) {
+    int f = -1;
+    for (int k = 0; k < nc; k++) {
+      const int q = child[p * 8 + k];
+      if (copy || orth[q] == t) f = q;
+    }
+    tabs[w][t] = f;
+  }
+  __syncthreads();
+  if (!live) return;
+  const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1, h0 = n0 / 2, h1 = n1 / 2, h2 = n2 / 2;
+  const int per = (n0 + 2) / 2, items = per * (n1 + 2) * (D == 3 ? n2 + 2 : 1);
+  const TI wt = TI(1.0 / (1 << D));
+  for (int c = 0; c < L.ncomp; c++) {
+    for (int i = t; i < items; i += nt) {
+      const int row = per_row(i);
+      const int Z = D == 3 ? rows(row) - 1 : 0, Y = D == 3 ? row - (Z + 1) * (n1 + 2) - 1 : row - 1;
+      const int X0 = 2 * (i - row * per) - 1;
+      const bool in = Y >= 0 && Y < n1 && (D == 2 || (Z >= 0 && Z < n2));
+      TI v[2][D == 3 ? 8 : 4];
+      bool has[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int X = X0 + j;
+        const int o = (X >= h0 ? 1 : 0) | (Y >= h1 ? 2 : 0) | (D == 3 && Z >= h2 ? 4 : 0);
+        const int f = tabs[w][o];
+        has[j] = in && X >= 0 && X < n0 && f >= 0;
+        if (!has[j]) continue;
+        if (copy) {
+          v[j][0] = fine[lin(L, f, c, X, Y, Z)];
+          continue;
+        }
+        const TI* q = fine + lin(L, f, c, 2 * X - (X >= h0 ? n0 : 0), 2 * Y - (Y >= h1 ? n1 : 0),
+                                 D == 3 ? 2 * Z - (Z >= h2 ? n2 : 0) : 0);
+#pragma unroll
+        for (int r = 0; r < (D == 3 ? 4 : 2); r++)
+          load_at<TI, 2>(q + (r & 1) * L.sx + (r >> 1) * L.sy, [&](int e, TI x) { v[j][2 * r + e] = x; });
+      }
+      TO res[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        TI acc = TI(0);
+        if (has[j]) {
+          if (copy) {
+            acc += v[j][0];
+          } else {
+#pragma unroll
+            for (int r = 0; r < (D == 3 ? 8 : 4); r++) acc += v[j][r] * wt;
+          }
+        }
+        res[j] = TO(acc);
+      }
+      store_at<TO, 2>(coarse + p * L.ps + c * L.cs + 2 * i, [&](int j) { return res[j]; });
+    }
+  }
+}
+
+// DirectInterpolator: fine += the coarse cell over it, over the interior rows of each fine patch
+template <typename TC, typename TF, int D, int V>
 __global__ void __launch_bounds__(256) interp_kernel(const int32_t* __restrict__ parent,
                                                      const int32_t* __restrict__ orth, const TC* __restrict__ coarse,
-                                                     TF* __restrict__ fine, Layout L)
+                                                     TF* __restrict__ fine, Layout L, FastDiv per_row, FastDiv rows)
 {
-  long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long total = (long)L.np * L.ps;
-  if (gid >= total) return;
-  int idx = (int)gid;
-  int p = idx / L.ps;
-  int rem = idx - p * L.ps;
-  int c = rem / L.cs;
-  int q = rem - c * L.cs;
-  int x, y, z = 0;
-  if (D == 2) {
-    y = q / L.sx;
-    x = q - y * L.sx;
-  } else {
-    z = q / L.sy;
-    int r2 = q - z * L.sy;
-    y = r2 / L.sx;
-    x = r2 - y * L.sx;
-    z -= 1;
+  constexpr bool WAVE = D == 2;
+  constexpr int U = 2;  // pairs in flight a thread
+  const int b = xcd_item(blockIdx.x, gridDim.x);
+  const int p = WAVE ? __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6)) : b;
+  if (p >= L.np) return;
+  const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
+  const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1;
+  const int per = V == 2 ? n0 / 2 + 1 : n0, items = per * n1 * n2;
+  const int cp = parent[p], o = orth[p], sh = o < 0 ? 0 : 1;
+  const int s0 = sh && (o & 1) ? n0 : 0, s1 = sh && (o & 2) ? n1 : 0, s2 = sh && (o & 4) ? n2 : 0;
+  for (int c = 0; c < L.ncomp; c++) {
+    const TC* cb = coarse + cp * L.ps + c * L.cs;
+    TF* fb = fine + p * L.ps + c * L.cs;
+    for (int i0 = t; i0 < items; i0 += U * nt) {
+      TF fv[U][V];
+      TC cv[U][V];
+      int off[U], x0[U];
+#pragma unroll
+      for (int k = 0; k < U; k++) {
+        const int i = i0 + k * nt;
+        if (i >= items) continue;
+        const int row = per_row(i), z = D == 3 ? rows(row) : 0, y = row - z * n1;
+        x0[k] = V == 2 ? 2 * (i - row * per) - 1 : i - row * per;
+        const int up = D == 3 ? L.sy : 0;
+        off[k] = (z + 1) * up + (y + 1) * L.sx + x0[k] + 1;
+        load_at<TF, V>(fb + off[k], [&](int j, TF v) { fv[k][j] = v; });
+        const int crow = (((z + s2) >> sh) + 1) * up + (((y + s1) >> sh) + 1) * L.sx + 1;
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+          const int x = min(max(x0[k] + j, 0), n0 - 1);  // an end pair's ghost value is not written
+          cv[k][j] = cb[crow + ((x + s0) >> sh)];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < U; k++) {
+        const int i = i0 + k * nt;
+        if (i >= items) continue;
+#pragma unroll
+        for (int j = 0; j < V; j++) fv[k][j] = TF(fv[k][j] + TF(cv[k][j]));
+        if (V == 1 || (x0[k] >= 0 && x0[k] + 1 < n0)) store_at<TF, V>(fb + off[k], [&](int j) { return fv[k][j]; });
+        else if (x0[k] < 0) fb[off[k] + 1] = fv[k][V - 1];
+        else fb[off[k]] = fv[k][0];
+      }
+    }
   }
-  x -= 1;
-  y -= 1;
-  bool inter = x >= 0 && x < L.n[0] && y >= 0 && y < L.n[1] && (D == 2 || (z >= 0 && z < L.n[2]));
-  if (!inter) return;
-  int cp = parent[p];
-  int o = orth[p];
-  int ci;
-  if (o < 0) {
-    ci = lin(L, cp, c, x, y, z);
-  } else {
-    int sx0 = (o & 1) ? L.n[0] : 0, sy0 = (o & 2) ? L.n[1] : 0, sz0 = (o & 4) ? L.n[2] : 0;
-    ci = lin(L, cp, c, (x + sx0) / 2, (y + sy0) / 2, D == 3 ? (z + sz0) / 2 : 0);
-  }
-  fine[idx] = TF(fine[idx] + TF(coarse[ci]));
 }
 
 template <typename TI, typename TO>
@@ -196,6 +317,18 @@ void restrict_t(const te_level_link* l, const TI* fine, TO* coarse, int ncomp, b
   Layout L = make_layout(c->dim, c->ns, ncomp, l->fine->np);
   long total = (long)c->np * L.ps;
   if (total == 0) return;
+  if (!ex && l->regular) {
+    const int per = (L.n[0] + 2) / 2, rows = L.n[1] + 2;
+    const int items = per * rows * (c->dim == 3 ? L.n[2] + 2 : 1);
+    if (c->dim == 2)
+      hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 2>), dim3(xcd_grid((c->np + 3) / 4)), dim3(256), 0, s,
+                         l->d_child, l->d_nchild, l->d_orth, fine, coarse, L, c->np, FastDiv(per), FastDiv(rows));
+    else
+      hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 3>), dim3(xcd_grid(c->np)),
+                         dim3(std::min(256, (items + 63) / 64 * 64)), 0, s, l->d_child, l->d_nchild, l->d_orth, fine,
+                         coarse, L, c->np, FastDiv(per), FastDiv(rows));
+    return;
+  }
   const int B = 256;
   int grid = (int)((total + B - 1) / B);
 #define TE_RK(D_, EX_)                                                                                             \
@@ -215,17 +348,23 @@ template <typename TC, typename TF>
 void interp_t(const te_level_link* l, const TC* coarse, TF* fine, int ncomp, hipStream_t s)
 {
   const te_domain* f = l->fine;
+  if (f->np == 0) return;
   Layout L = make_layout(f->dim, f->ns, ncomp, f->np);
-  long total = (long)f->np * L.ps;
-  if (total == 0) return;
-  const int B = 256;
-  int grid = (int)((total + B - 1) / B);
-  if (f->dim == 2)
-    hipLaunchKernelGGL((interp_kernel<TC, TF, 2>), dim3(grid), dim3(B), 0, s, l->d_parent, l->d_orth, coarse, fine,
-                       L);
-  else
-    hipLaunchKernelGGL((interp_kernel<TC, TF, 3>), dim3(grid), dim3(B), 0, s, l->d_parent, l->d_orth, coarse, fine,
-                       L);
+  const int V = L.n[0] % 2 == 0 ? 2 : 1, per = V == 2 ? L.n[0] / 2 + 1 : L.n[0];
+  const int items = per * L.n[1] * (f->dim == 3 ? L.n[2] : 1);
+  const int grid = xcd_grid(f->dim == 2 ? (f->np + 3) / 4 : f->np);
+  const int block = f->dim == 2 ? 256 : std::min(256, (items + 63) / 64 * 64);
+#define TE_IP(D_, V_)                                                                                              \
+  hipLaunchKernelGGL((interp_kernel<TC, TF, D_, V_>), dim3(grid), dim3(block), 0, s, l->d_parent, l->d_orth, coarse, \
+                     fine, L, FastDiv(per), FastDiv(L.n[1]))
+  if (f->dim == 2) {
+    if (V == 2) TE_IP(2, 2);
+    else TE_IP(2, 1);
+  } else {
+    if (V == 2) TE_IP(3, 2);
+    else TE_IP(3, 1);
+  }
+#undef TE_IP
 }
 
 }  // namespace

@@ -173,6 +173,9 @@ struct te_level_link {
   int32_t* d_child = nullptr;       // [np_coarse][8]
   int32_t* d_nchild = nullptr;      // [np_coarse]
   int32_t* d_ring = nullptr;        // 2D: ring table of the fine level with the pq fields set
+  // even cells per side, and every coarse patch has either one copied child or children of
+  // distinct orthants: each coarse cell then lies under one child
+  bool regular = true;
 };
 
 namespace te {
