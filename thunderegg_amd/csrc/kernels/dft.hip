@@ -157,131 +157,179 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
   }
 }
 
-// The same solve for 3D patches of 16^3 cells on the matrix cores: every axis transform is
-// 16 products of 16 x 16 matrices (the lines of one slice, or of one row of slices, against
-// the axis matrix), 4 per wave, each a chain of 16x16x4 MFMAs with operands read from LDS.
-// The patch lives in LDS with padded pitches (rows of 17, slices of 16 * 17 + 1) so that a
-// lane group's operand reads spread over the banks, in one buffer: a wave's products read
-// and write only its own slices (x and y transforms) or rows (z), and each product reads
-// all its operands before it writes, so the transforms run in place.  Interface terms,
-// eigenvalues, the per-patch transform types and the all-Neumann zero mode are the generic
-// kernel's.
-constexpr int k3N = 16, k3Row = 17, k3Slice = 16 * 17 + 1, k3Cells = 16 * k3Slice, k3Mat = 16 * 17;
+// The same solve for 3D patches of 16^3 cells on the matrix cores.  Every axis transform is a
+// chain of 16x16x4 MFMAs with the transform matrices in registers: per z-slice the x product's
+// accumulator is the y product's operand (with a matching K order), the patch crosses LDS once
+// to the z products (per y-row: forward, eigenvalues, inverse, chained through registers) and
+// once back to the inverse y-x chain.  Wave w owns the slices (then rows) w, w + 4, w + 8,
+// w + 12; in a slice lane l = c + 16 g holds the cells x = 4g .. 4g + 3 of row y = c.  The loads
+// of a batch of slices (f, and at the faces the ghost and boundary values of u) are issued
+// before its first product: 2 slices in FP32, 1 in FP64 (registers).
+// Latency-bound on small levels (one patch a CU): 8 patches in FP32 take 6.4 us where one LDS
+// round trip per axis (six, with barriers between) took 20.6; on large ones bound by memory:
+// 2,535 patches 43 us (the vectors' padded lines in 36 at a copy's rate) against 95.
+constexpr int k3N = 16, k3Row = 20, k3Slice = 16 * k3Row + 4, k3Slab = 16 * k3Slice;
 
-__device__ __forceinline__ int c3(int x, int y, int z) { return x + k3Row * y + k3Slice * z; }
-
-// one 16 x 16 x 16 product, D[i][j] = sum_k A(i, k) B(k, j), written by put(i, j, value)
-template <typename T, class GA, class GB, class Put>
-__device__ __forceinline__ void mm16(GA A, GB B, Put put, int lane)
+// four consecutive values at an address that is a multiple of TS only (rows of 18 values)
+template <typename T, typename TS>
+__device__ __forceinline__ void load_row4(const TS* base, int idx, T (&r)[4])
 {
-  typedef typename Mf<T>::V V;
-  const int c = lane & 15, g = lane >> 4;
-  V acc = { 0, 0, 0, 0 };
+  constexpr int W = 16 / sizeof(TS);
+  typedef TS Vec __attribute__((ext_vector_type(W), aligned(sizeof(TS))));
 #pragma unroll
-  for (int s = 0; s < 4; s++) {
-    const int k = 4 * s + g;
-    acc = Mf<T>::mma(A(c, k), B(k, c), acc);
-  }
+  for (int k = 0; k < 4; k += W) {
+    const Vec v = *reinterpret_cast<const Vec*>(&at(base, idx + k));
 #pragma unroll
-  for (int r = 0; r < 4; r++) put(Mf<T>::row(r, g), c, acc[r]);
-}
-
-// dst = the transform of src along axis a with matrix M (16 x 16, rows of k3Row); dst may be src
-template <typename T>
-__device__ __forceinline__ void axis16(int a, const T* M, const T* src, T* dst, int wave, int lane)
-{
-  for (int q = wave; q < k3N; q += 4) {
-    if (a == 0) {  // slice z = q: D[y][k] = sum_x X[y][x] M[k][x]
-      mm16<T>([&](int y, int x) { return src[c3(x, y, q)]; }, [&](int x, int k) { return M[k * k3Row + x]; },
-              [&](int y, int k, T v) { dst[c3(k, y, q)] = v; }, lane);
-    } else if (a == 1) {  // slice z = q: D[k][x] = sum_y M[k][y] X[y][x]
-      mm16<T>([&](int k, int y) { return M[k * k3Row + y]; }, [&](int y, int x) { return src[c3(x, y, q)]; },
-              [&](int k, int x, T v) { dst[c3(x, k, q)] = v; }, lane);
-    } else {  // row y = q: D[k][x] = sum_z M[k][z] X[z][x]
-      mm16<T>([&](int k, int z) { return M[k * k3Row + z]; }, [&](int z, int x) { return src[c3(x, q, z)]; },
-              [&](int k, int x, T v) { dst[c3(x, q, k)] = v; }, lane);
-    }
+    for (int j = 0; j < W; j++) r[k + j] = T(v[j]);
   }
 }
 
 template <typename T, typename TF, typename TO, int OP, bool UZERO>
 __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
                                                         const T* __restrict__ mats, const T* __restrict__ s2tab,
-                                                        const TF* __restrict__ f, const T* __restrict__ u,
-                                                        const T* __restrict__ coeffs, TO* __restrict__ out, Layout L)
+                                                        const TF* __restrict__ f, const T* u,
+                                                        const T* __restrict__ coeffs, TO* out, Layout L)
 {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* A = reinterpret_cast<T*>(smem_raw);
-  T* MF = A + k3Cells;       // forward matrices of the three axes, rows of k3Row
-  T* MI = MF + 3 * k3Mat;    // inverse matrices
+  __shared__ __align__(16) T slab[k3Slab];
+  typedef typename Mf<T>::V V;
+  constexpr int SB = sizeof(T) == 4 ? 2 : 1;
   const int p = blockIdx.x;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int* pt = ptype + p * 8;  // fwd type per axis [0..2], eig type per axis [3..5], zero mode [6]
   const DevPatch& P = dp[p];
+  const int row0 = p * L.ps + (c + 1) * L.sx + 4 * g + 1;  // the lane's cells in slice z: row0 + (z + 1) * sy
+  T F[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) load_row4(f, row0 + (w + 4 * i + 1) * L.sy, F[i]);
+  // the transform matrices M[i][j] (y_i = sum_j M[i][j] x_j) as MFMA operands: lane (c, g), step
+  // s holds M[c][K], K the product's K order (4g + s from memory, Mf<T>::row from an accumulator)
+  auto mat = [&](int t, int a, int i, int j) { return mats[(t * 3 + a) * kDftMatStride + i * k3N + j]; };
+  T SxB[4], SyA[4], SzA[4], SziA[4], SxiB[4], SyiA[4];
+  int tf[3], ti[3];
+#pragma unroll
   for (int a = 0; a < 3; a++) {
-    const int tf = pt[a];
-    const int ti = tf == 0 ? 1 : (tf == 3 ? 4 : tf);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
-    for (int k = threadIdx.x; k < k3N * k3N; k += blockDim.x) {
-      const int row = k >> 4, col = k & 15;
-      MF[a * k3Mat + row * k3Row + col] = mats[(tf * 3 + a) * kDftMatStride + k];
-      MI[a * k3Mat + row * k3Row + col] = mats[(ti * 3 + a) * kDftMatStride + k];
-    }
+    tf[a] = pt[a];
+    ti[a] = tf[a] == 0 ? 1 : (tf[a] == 3 ? 4 : tf[a]);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
   }
-  // f_copy = f, then modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson :168-186)
-  for (int o = threadIdx.x; o < k3N * k3N * k3N; o += blockDim.x) {
-    const int x = o & 15, y = (o >> 4) & 15, z = o >> 8;
-    const int gi = lin(L, p, 0, x, y, z);
-    T v = T(f[gi]);
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const int k1 = 4 * g + s, k2 = Mf<T>::row(s, g);
+    SxB[s] = mat(tf[0], 0, c, k1);
+    SyA[s] = mat(tf[1], 1, c, k2);
+    SzA[s] = mat(tf[2], 2, c, k1);
+    SziA[s] = mat(ti[2], 2, c, k2);
+    SxiB[s] = mat(ti[0], 0, c, k1);
+    SyiA[s] = mat(ti[1], 1, c, k2);
+  }
+  // f_copy = f, then modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson
+  // :168-186), sides in the reference's order
+  bool has[6];
+#pragma unroll
+  for (int s = 0; s < 6; s++) has[s] = P.type[20 + s] >= 0;
+  const bool onx = (g == 0 && has[0]) || (g == 3 && has[1]);
+  const bool ony = (c == 0 && has[2]) || (c == k3N - 1 && has[3]);
+  const T ih[3] = { T(P.inv_h2[0]), T(P.inv_h2[1]), T(P.inv_h2[2]) };
+  // the values of v on a face of the lane's cells: x its one boundary cell and the ghost, y and z
+  // the row of four and the ghosts over it
+  struct Face {
+    T xb, xg, b[4], y[4], z[4];
+  };
+  auto faces = [&](const T* v, int base, int z, Face& q) {
+    const int r = base + (z + 1) * L.sy;
+    const bool onz = (z == 0 && has[4]) || (z == k3N - 1 && has[5]);
+    if (onx) {
+      q.xb = at(v, g == 0 ? r : r + 3);
+      q.xg = at(v, g == 0 ? r - 1 : r + 4);
+    }
+    if (ony || onz) load_row4(v, r, q.b);
+    if (ony) load_row4(v, c == 0 ? r - L.sx : r + L.sx, q.y);
+    if (onz) load_row4(v, z == 0 ? r - L.sy : r + L.sy, q.z);
+  };
+#pragma unroll
+  for (int i0 = 0; i0 < 4; i0 += SB) {
+    Face q[SB], cq[OP == 1 ? SB : 1];
     if (!UZERO) {
-      const int cc[3] = { x, y, z };
-      const int st[3] = { 1, L.sx, L.sy };
 #pragma unroll
-      for (int a = 0; a < 3; a++) {
-#pragma unroll
-        for (int up = 0; up < 2; up++) {
-          const bool edge = up ? (cc[a] == k3N - 1) : (cc[a] == 0);
-          if (!edge || P.type[20 + 2 * a + up] < 0) continue;
-          const int gidx = up ? gi + st[a] : gi - st[a];
-          const T ih2 = T(P.inv_h2[a]);
-          if (OP == 0) {
-            v -= (u[gidx] + u[gi]) * ih2;
-          } else {
-            const int cq = gi - p * L.ps;
-            const int cg = up ? cq + st[a] : cq - st[a];
-            const T cb = coeffs[p * L.cs + cq], cgv = coeffs[p * L.cs + cg];
-            v -= (u[gidx] + u[gi]) * (cb + cgv) * (ih2 * T(0.5));
-          }
-        }
+      for (int j = 0; j < SB; j++) {
+        faces(u, row0, w + 4 * (i0 + j), q[j]);
+        if (OP == 1) faces(coeffs, row0, w + 4 * (i0 + j), cq[OP == 1 ? j : 0]);
       }
     }
-    A[c3(x, y, z)] = v;
-  }
-  __syncthreads();
-  for (int a = 0; a < 3; a++) {  // forward transform along each axis, in place
-    axis16<T>(a, MF + a * k3Mat, A, A, wave, lane);
-    __syncthreads();
-  }
-  T* src = A;
-  for (int o = threadIdx.x; o < k3N * k3N * k3N; o += blockDim.x) {  // divide by the eigenvalues
-    const int k3[3] = { o & 15, (o >> 4) & 15, o >> 8 };
-    T eig = T(0);
-    for (int a = 0; a < 3; a++) {
-      const double h = P.h[a];
-      eig -= T(4.0 / (h * h)) * s2tab[(pt[3 + a] * 3 + a) * kDftMatDim + k3[a]];
+#pragma unroll
+    for (int j = 0; j < SB; j++) {
+      const int z = w + 4 * (i0 + j);
+      T(&Fz)[4] = F[i0 + j];
+      if (!UZERO) {
+        const Face& Q = q[j];
+        const Face& C = cq[OP == 1 ? j : 0];
+        auto sub = [&](T& v, T ug, T ub, T cg, T cb, T h) {
+          if (OP == 0) v -= (ug + ub) * h;
+          else v -= (ug + ub) * (cb + cg) * (h * T(0.5));
+        };
+        if (g == 0 && has[0]) sub(Fz[0], Q.xg, Q.xb, C.xg, C.xb, ih[0]);
+        if (g == 3 && has[1]) sub(Fz[3], Q.xg, Q.xb, C.xg, C.xb, ih[0]);
+        if (ony) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) sub(Fz[k], Q.y[k], Q.b[k], C.y[k], C.b[k], ih[1]);
+        }
+        if ((z == 0 && has[4]) || (z == k3N - 1 && has[5])) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) sub(Fz[k], Q.z[k], Q.b[k], C.z[k], C.b[k], ih[2]);
+        }
+      }
+      V d1 = { 0, 0, 0, 0 };  // D1[y][kx] = sum_x F[y][x] Sx[kx][x]
+#pragma unroll
+      for (int s = 0; s < 4; s++) d1 = Mf<T>::mma(Fz[s], SxB[s], d1);
+      V d2 = { 0, 0, 0, 0 };  // D2[ky][kx] = sum_y Sy[ky][y] D1[y][kx]
+#pragma unroll
+      for (int s = 0; s < 4; s++) d2 = Mf<T>::mma(SyA[s], d1[s], d2);
+#pragma unroll
+      for (int r = 0; r < 4; r++) slab[z * k3Slice + Mf<T>::row(r, g) * k3Row + c] = d2[r];
     }
-    src[c3(k3[0], k3[1], k3[2])] /= eig;
   }
   __syncthreads();
-  if (pt[6] && threadIdx.x == 0) src[0] = T(0);  // all-Neumann patch without neighbours (:438-440)
-  __syncthreads();
-  for (int a = 0; a < 3; a++) {
-    axis16<T>(a, MI + a * k3Mat, A, A, wave, lane);
-    __syncthreads();
+  const T lx = T(4.0 / (P.h[0] * P.h[0])), ly = T(4.0 / (P.h[1] * P.h[1])), lz = T(4.0 / (P.h[2] * P.h[2]));
+  const T s2x = s2tab[(pt[3] * 3 + 0) * kDftMatDim + c];
+  T s2z[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) s2z[r] = s2tab[(pt[5] * 3 + 2) * kDftMatDim + Mf<T>::row(r, g)];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int ky = w + 4 * i;
+    V b = { 0, 0, 0, 0 };  // W[kz][kx] = sum_z Sz[kz][z] D2[z][ky][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) b = Mf<T>::mma(SzA[s], slab[(4 * g + s) * k3Slice + ky * k3Row + c], b);
+    const T s2y = s2tab[(pt[4] * 3 + 1) * kDftMatDim + ky];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {  // divide by the eigenvalues (:320-361)
+      T eig = T(0);
+      eig -= lx * s2x;
+      eig -= ly * s2y;
+      eig -= lz * s2z[r];
+      b[r] = b[r] / eig;
+      // all-Neumann patch without neighbours (:438-440)
+      if (pt[6] && ky == 0 && c == 0 && Mf<T>::row(r, g) == 0) b[r] = T(0);
+    }
+    V b2 = { 0, 0, 0, 0 };  // W'[z][kx] = sum_kz Szi[z][kz] W[kz][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) b2 = Mf<T>::mma(SziA[s], b[s], b2);
+#pragma unroll
+    for (int r = 0; r < 4; r++) slab[Mf<T>::row(r, g) * k3Slice + ky * k3Row + c] = b2[r];
   }
+  __syncthreads();
   const T scale = T(2.0) / T(16) * (T(2.0) / T(16)) * (T(2.0) / T(16));
-  for (int o = threadIdx.x; o < k3N * k3N * k3N; o += blockDim.x) {
-    const int x = o & 15, y = (o >> 4) & 15, z = o >> 8;
-    out[lin(L, p, 0, x, y, z)] = TO(src[c3(x, y, z)] * scale);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int z = w + 4 * i;
+    V r1 = { 0, 0, 0, 0 };  // R[ky][x] = sum_kx Q[ky][kx] Sxi[x][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) r1 = Mf<T>::mma(slab[z * k3Slice + c * k3Row + 4 * g + s], SxiB[s], r1);
+    V u2 = { 0, 0, 0, 0 };  // U[y][x] = sum_ky Syi[y][ky] R[ky][x]
+#pragma unroll
+    for (int s = 0; s < 4; s++) u2 = Mf<T>::mma(SyiA[s], r1[s], u2);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      at(out, p * L.ps + (z + 1) * L.sy + (Mf<T>::row(r, g) + 1) * L.sx + c + 1) = TO(u2[r] * scale);
   }
 }
 
@@ -301,9 +349,8 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
   const T* s2 = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_s2_64 : (const void*)pl->d_s2_32);
   const T* cf = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_coeffs64 : (const void*)pl->d_coeffs32);
   if (D == 3 && pl->use_mfma && d->ns[0] == 16 && d->ns[1] == 16 && d->ns[2] == 16) {
-    const size_t sh3 = sizeof(T) * ((size_t)k3Cells + 6 * (size_t)k3Mat);
 #define TE_D3(OP_, UZ_)                                                                                         \
-  hipLaunchKernelGGL((dft3_mfma_kernel<T, TF, TO, OP_, UZ_>), dim3(d->np), dim3(256), sh3, s, d->d_patches,     \
+  hipLaunchKernelGGL((dft3_mfma_kernel<T, TF, TO, OP_, UZ_>), dim3(d->np), dim3(256), 0, s, d->d_patches,     \
                      pl->d_ptype, mats, s2, f, u, cf, out, L)
     if (pl->op_kind == 0) {
       if (uzero) TE_D3(0, true); else TE_D3(0, false);
