@@ -315,8 +315,8 @@ int te_gmg_create(const te_domain* const* levels, int num_levels, const te_gmg_o
 int te_gmg_destroy(te_gmg* g);
 /* Cycle::apply(f, u) (GMG/Cycle.h:94-98): u := V-cycle(f); float64 vectors of level 0.
  * Stream-ordered and asynchronous: the cycle starts after the work enqueued on `stream` and
- * `stream`'s later work waits for it (events; the launches run on the solver's own stream
- * as one cached graph).  When `stream` is being captured into a graph, the launches are
+ * `stream`'s later work waits for it (the launches run on `stream`, a long cycle's as one cached
+ * graph; events order it after the object's earlier cycles and solves on other streams).  When `stream` is being captured into a graph, the launches are
  * enqueued on it directly, so the cycle becomes part of the caller's graph.  Exception: a
  * level with the BiCGStab patch smoother and continue_on_breakdown == 0 makes the call
  * synchronous (it reads the breakdown flag back) and not capturable. */

@@ -491,3 +491,39 @@ def test_cg_matches_oracle(cycle_type):
     xr, itr, _ = ol.cg(b.copy(), precond=True, cycle_type=cycle_type, tol=1e-10)
     assert itm <= itr + 2
     assert relerr(mesh.interior(xm, dim), mesh.interior(xr, dim)) <= 2e-5
+
+
+@pytest.mark.parametrize("ns,level,pre", [((16, 16), 2, 1), ((16, 16, 16), 1, 2), ((6, 6, 6), 2, 2), ((10, 10), 4, 3)])
+def test_cycles_and_solves_on_several_streams(ns, level, pre):
+    """One hierarchy used from two streams, the null stream and by solves in turn, without host
+    waits between: a cycle runs on its caller's stream and each use waits for the one before, so
+    every result has the bits of the same call alone (few launches, enqueued one by one, and
+    cycles long enough to be a graph)."""
+    dim = len(ns)
+    levels = solver.uniform_levels(dim, level, ns)
+    kind = R.TRILINEAR if dim == 3 else R.BILINEAR
+    g = solver.GMG(dim, ns, levels, filler_kind=kind, precision=R.F32, pre_sweeps=pre, post_sweeps=pre)
+    fs = [R.DeviceArray.from_host(random_field(g.shape, 71 + k)) for k in range(3)]
+    us = [R.DeviceArray.from_host(np.zeros(g.shape)) for _ in range(3)]
+    alone = []
+    for f, u in zip(fs, us):
+        g.vcycle_device(f, u)
+        R.sync()
+        alone.append(u.get())
+    x = R.DeviceArray.from_host(np.zeros(g.shape))
+    its, _ = g.solve_device(fs[0], x, tol=1e-8, max_it=40, precond=2)
+    solved = x.get()
+    a, b = R.Stream(), R.Stream()
+    for rep in range(3):
+        for u in us + [x]:
+            u.zero()
+        R.sync()
+        for stream, f, u in ((a.h, fs[0], us[0]), (b.h, fs[1], us[1]), (None, fs[2], us[2]), (a.h, fs[1], us[1]),
+                             (b.h, fs[0], us[0])):
+            R.check(R.lib().te_gmg_vcycle(g.h, f.ptr, u.ptr, stream))
+        assert g.solve_device(fs[0], x, tol=1e-8, max_it=40, precond=2)[0] == its
+        R.check(R.lib().te_gmg_vcycle(g.h, fs[2].ptr, us[2].ptr, b.h))
+        a.sync(), b.sync(), R.sync()
+        assert np.array_equal(mesh.interior(x.get(), dim), mesh.interior(solved, dim))
+        for u, want in zip(us, alone):
+            assert np.array_equal(mesh.interior(u.get(), dim), mesh.interior(want, dim))

@@ -408,9 +408,35 @@ int vcycle_enqueue_one(te_gmg* g, const void* f, void* u, int udt, int dtf, bool
   return visit(g, 0, f, TE_F64, ud);
 }
 
-int vcycle_launch(te_gmg* g, const double* f, double* u)
+// one cycle enqueued on s (vcycle_enqueue's launches go to g->s)
+int vcycle_enqueue_on(te_gmg* g, const double* f, double* u, hipStream_t s)
 {
-  if (!g->o.use_graph || g->timer) return vcycle_enqueue(g, f, u);
+  const hipStream_t own = g->s;
+  g->s = s;
+  const int rc = vcycle_enqueue(g, f, u);
+  g->s = own;
+  return rc;
+}
+
+// Launches of one V-cycle (about: sweeps that also fill ghosts count twice).  Up to
+// kDirectLaunches of them are enqueued one by one: the host enqueues a launch in about 3 us,
+// less than one runs, while a graph takes 20 us to start and, for every new pair of vectors,
+// some 100 us to record.  16 patches of 16^2 (4 launches): 24 us a cycle against 30 as a graph.
+// Longer cycles stay graphs, which leave the host free (59 launches: 71 against 591 us of
+// host time, 840 us on the device either way).
+constexpr int kDirectLaunches = 24;
+
+int vcycle_launches(const te_gmg* g)
+{
+  if (g->o.cycle_type != TE_CYCLE_V) return kDirectLaunches + 1;
+  const int sweeps = g->o.pre_sweeps + g->o.post_sweeps;
+  const int levels = g->fused && g->tail_from >= 0 ? g->tail_from : (int)g->L.size() - 1;
+  return levels * (g->fused || g->c3 ? sweeps + 1 : 2 * sweeps + 3) + 1 + (g->c3 ? 2 : 0);
+}
+
+int vcycle_launch(te_gmg* g, const double* f, double* u, hipStream_t s)
+{
+  if (!g->o.use_graph || g->timer || vcycle_launches(g) <= kDirectLaunches) return vcycle_enqueue_on(g, f, u, s);
   const GraphCache::Key key{ (uintptr_t)f, (uintptr_t)u, 0 };
   hipGraphExec_t it = g->vgraphs.find(key);
   if (!it) {
@@ -433,7 +459,36 @@ int vcycle_launch(te_gmg* g, const double* f, double* u)
     g->vgraphs.put(key, exec);
     it = exec;
   }
-  TE_HIP(hipGraphLaunch(it, g->s));
+  TE_HIP(hipGraphLaunch(it, s));
+  return TE_OK;
+}
+
+// A cycle runs on its caller's stream, a solve on the object's own; both use the object's
+// vectors, so each is ordered after the other's last work (events, no host blocking).
+// Before work on the own stream: it waits for the last cycle.
+int enter_own(te_gmg* g)
+{
+  if (g->cycle_pending) TE_HIP(hipStreamWaitEvent(g->s, g->ev_out, 0));
+  g->cycle_pending = false;
+  g->own_pending = true;
+  return TE_OK;
+}
+// Before a cycle on the caller's stream: it waits for the last cycle (which may have run on
+// another stream) and for the own stream's work since then.
+int enter_cycle(te_gmg* g, hipStream_t caller)
+{
+  if (g->cycle_pending) TE_HIP(hipStreamWaitEvent(caller, g->ev_out, 0));
+  if (g->own_pending) {
+    TE_HIP(hipEventRecord(g->ev_in, g->s));
+    TE_HIP(hipStreamWaitEvent(caller, g->ev_in, 0));
+    g->own_pending = false;
+  }
+  return TE_OK;
+}
+int leave_cycle(te_gmg* g, hipStream_t caller)
+{
+  TE_HIP(hipEventRecord(g->ev_out, caller));
+  g->cycle_pending = true;
   return TE_OK;
 }
 
@@ -441,18 +496,10 @@ int vcycle_launch(te_gmg* g, const double* f, double* u)
 // there), without blocking the host.
 int join_from(te_gmg* g, hipStream_t caller)
 {
+  TE_RC(enter_own(g));
   if (caller == g->s) return TE_OK;
   TE_HIP(hipEventRecord(g->ev_in, caller));
   TE_HIP(hipStreamWaitEvent(g->s, g->ev_in, 0));
-  return TE_OK;
-}
-
-// `caller` waits for the work enqueued so far on the solver's stream.
-int join_to(te_gmg* g, hipStream_t caller)
-{
-  if (caller == g->s) return TE_OK;
-  TE_HIP(hipEventRecord(g->ev_out, g->s));
-  TE_HIP(hipStreamWaitEvent(caller, g->ev_out, 0));
   return TE_OK;
 }
 
@@ -466,13 +513,13 @@ bool needs_breakdown_check(const te_gmg* g)
   return false;
 }
 
-int check_flags(te_gmg* g)
+int check_flags(te_gmg* g, hipStream_t s)
 {
   int32_t flag = 0;
-  TE_HIP(hipMemcpyAsync(&flag, g->d_flags, sizeof(int32_t), hipMemcpyDeviceToHost, g->s));
-  TE_HIP(hipStreamSynchronize(g->s));
+  TE_HIP(hipMemcpyAsync(&flag, g->d_flags, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  TE_HIP(hipStreamSynchronize(s));
   if (flag && !g->o.continue_on_breakdown) {
-    TE_HIP(hipMemsetAsync(g->d_flags, 0, sizeof(int32_t), g->s));
+    TE_HIP(hipMemsetAsync(g->d_flags, 0, sizeof(int32_t), s));
     set_error("BiCGStab broke down in a patch smoother (rho was 0)");
     return TE_ERR_BREAKDOWN;
   }
@@ -871,18 +918,15 @@ int te_gmg_vcycle(te_gmg* g, const double* f, double* u, te_stream stream)
                 "flag back and cannot be captured (use continue_on_breakdown)");
       return TE_ERR_UNSUPPORTED;
     }
-    hipStream_t own = g->s;
-    g->s = cs;
-    int rc = vcycle_enqueue(g, f, u);
-    g->s = own;
-    return rc;
+    return vcycle_enqueue_on(g, f, u, cs);
   }
-  TE_RC(join_from(g, cs));
-  TE_RC(vcycle_launch(g, f, u));
-  TE_RC(join_to(g, cs));
-  if (!needs_breakdown_check(g)) return TE_OK;
-  TE_HIP(hipStreamSynchronize(g->s));
-  return check_flags(g);
+  // on the caller's stream itself: a stream of its own would cost two waits between hardware
+  // queues per cycle
+  TE_RC(enter_cycle(g, cs));
+  int rc = vcycle_launch(g, f, u, cs);
+  TE_RC(leave_cycle(g, cs));
+  if (rc || !needs_breakdown_check(g)) return rc;
+  return check_flags(g, cs);
 }
 
 // Iterative::BiCGStab::solve (Iterative/BiCGStab.h:111-203)
@@ -1192,7 +1236,7 @@ int te_gmg_bicgstab(te_gmg* g, const double* b, double* x, int use_precond, int 
   g->last_seconds = std::chrono::duration<double>(t1 - t0).count();
   if (iterations) *iterations = num_its;
   if (rc) return rc;
-  return check_flags(g);
+  return check_flags(g, g->s);
 }
 
 // Iterative::CG::solve (Iterative/CG.h:126-194): right-preconditioned CG, ap = A (M p)
@@ -1284,7 +1328,7 @@ int te_gmg_cg(te_gmg* g, const double* b, double* x, int use_precond, int max_it
   g->last_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   if (iterations) *iterations = num_its;
   if (rc) return rc;
-  return check_flags(g);
+  return check_flags(g, g->s);
 }
 
 double te_gmg_last_solve_seconds(const te_gmg* g) { return g ? g->last_seconds : -1.0; }
@@ -1304,6 +1348,7 @@ int te_gmg_time_kernel(te_gmg* g, int which, int reps, double* ms)
     set_error("te_gmg_time_kernel: the transfer kernels need a coarser level");
     return TE_ERR_UNSUPPORTED;
   }
+  TE_RC(enter_own(g));
   GLevel& L0 = g->L[0];
   te_gmg::C3Level& C0 = g->C3[0];
   hipStream_t s = g->s;

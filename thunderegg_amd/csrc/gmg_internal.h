@@ -112,6 +112,9 @@ struct te_gmg {
   bool bsweep = false;
   // stream ordering with the caller's stream (no host blocking)
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
+  // a cycle enqueued on a caller's stream (ev_out recorded after it) that the own stream has not
+  // been ordered after, and work on the own stream that no cycle has been ordered after
+  bool cycle_pending = false, own_pending = false;
   // 3D hierarchies of 16^3 patches whose face neighbours are all on the same level: the
   // cycle and the BiCGStab work on compact vectors (interior cells only, cycle3d.h)
   bool c3 = false;
