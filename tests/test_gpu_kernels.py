@@ -299,6 +299,45 @@ def test_dft3_mfma_matches_generic(name, op_kind, neumann_mask, monkeypatch):
         assert relerr(mesh.interior(du.get(), dim), mesh.interior(uz, dim)) <= tol, dtype
 
 
+@pytest.mark.parametrize("name", ["3d_uniform_2x2x2_mpi1.json", "3d_refined_bnw_2x2x2_mpi1.json"])
+@pytest.mark.parametrize("n", [8, 16])
+@pytest.mark.parametrize("op_kind", [0, 1])
+@pytest.mark.parametrize("neumann_mask", [0, 0b100101, 0b111111])
+def test_dft3_tiles(name, n, op_kind, neumann_mask):
+    """The 3D matrix-core patch solves (8^3: a patch per wave, 8 and 15 patches on workgroups of
+    four; 16^3) against the oracle: transform types per patch, interface terms, and apply's
+    zeroed ghosts, also on vectors off the wide stores' grid."""
+    ns = (n,) * 3
+    dim, levels = load(name, ns)
+    lv = levels[0]
+    od, dd = O.Domain(dim, ns, lv), _dev(dim, ns, lv)
+    g = R.GhostFiller(dd, R.TRILINEAR, R.FACES)
+    coeffs = None
+    if op_kind == 1:
+        X = mesh.cell_centers(lv, dim, ns)
+        coeffs = np.exp(np.sin(3 * X[..., 0]) * np.cos(2 * X[..., 1]) + 0.5 * X[..., 2])[:, None].copy()
+        O.fill_ghost(od, coeffs, kind=R.TRILINEAR)
+    dc = R.DeviceArray.from_host(coeffs) if coeffs is not None else None
+    plan = R.DftPlan(g, neumann_mask=neumann_mask, op_kind=op_kind, coeffs=dc)
+    args = dict(kind=R.TRILINEAR, neumann_mask=neumann_mask, op_kind=op_kind, coeffs=coeffs)
+    for dtype, tol in [(R.F64, 1e-12), (R.F32, 2e-5)]:
+        t = R.np_dtype(dtype)
+        f0, u0 = random_field(od.shape(1), 73, t), random_field(od.shape(1), 74, t)
+        uref, uz = u0.astype(np.float64), np.zeros(od.shape(1))
+        O.dft_smooth(od, f0.astype(np.float64), uref, **args)
+        O.dft_smooth(od, f0.astype(np.float64), uz, **args)
+        df, du = R.DeviceArray.from_host(f0), R.DeviceArray.from_host(u0)
+        plan.smooth(df, du)
+        assert relerr(mesh.interior(du.get(), dim), mesh.interior(uref, dim)) <= tol, dtype
+        for off in (0, 1):
+            big = R.DeviceArray.from_host(np.full(u0.size + off, 7, t))
+            R.check(R.lib().te_dft_apply(plan.h, dtype, df.ptr, big.ptr + off * t().itemsize, None))
+            got = big.get()[off:].reshape(u0.shape)
+            assert relerr(mesh.interior(got, dim), mesh.interior(uz, dim)) <= tol, dtype
+            mesh.interior(got, dim)[...] = 0
+            assert not got.any()
+
+
 @pytest.mark.parametrize("ns", [(16, 16), (32, 32)])
 @pytest.mark.parametrize("op_kind", [0, 1])
 def test_dft_mfma_matches_generic(ns, op_kind, monkeypatch):

@@ -651,9 +651,7 @@ int te_dft_patch_solve(const te_dft_plan* p, int dtype, const void* f, void* u, 
 int te_dft_apply(const te_dft_plan* p, int dtype, const void* f, void* u, te_stream s)
 {
   TE_ARG(p && f && u, "null argument");
-  int rc = launch_vec_op(p->g->d, dtype, VOP_SET_WITH_GHOST, u, nullptr, nullptr, 0.0, 0, 0, 1, S(s));
-  if (rc) return rc;
-  return launch_dft(p, dtype, dtype, dtype, f, u, u, true, S(s));
+  return launch_dft(p, dtype, dtype, dtype, f, u, u, true, S(s), true);
 }
 
 static bool dtype_ok(int t) { return t == TE_F64 || t == TE_F32; }

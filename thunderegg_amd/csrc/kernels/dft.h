@@ -23,8 +23,9 @@ struct te_dft_plan {
 };
 
 namespace te {
+// zero_ghosts: out's ghost cells are set to 0 as well (out may not be f then)
 int launch_dft(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, const void* u, void* out, bool uzero,
-               hipStream_t s);
+               hipStream_t s, bool zero_ghosts = false);
 bool dft_mfma_supported(const te_dft_plan* pl);
 int launch_dft_mfma(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, const void* u, void* out,
                     bool uzero, hipStream_t s);

@@ -11,6 +11,7 @@
 // modifyRHSForInternalBoundaryConditions vanish and u is not read.
 #include "../te_internal.h"
 #include "dft.h"
+#include "blas.h"
 #include "dft_wave.h"
 #include "ghost2d.h"
 #include "../tune.h"
@@ -188,7 +189,8 @@ template <typename T, typename TF, typename TO, int OP, bool UZERO>
 __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
                                                         const T* __restrict__ mats, const T* __restrict__ s2tab,
                                                         const TF* __restrict__ f, const T* u,
-                                                        const T* __restrict__ coeffs, TO* out, Layout L)
+                                                        const T* __restrict__ coeffs, TO* out, Layout L,
+                                                        bool zero_ghosts)
 {
   __shared__ __align__(16) T slab[k3Slab];
   typedef typename Mf<T>::V V;
@@ -221,6 +223,9 @@ __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restri
     SxiB[s] = mat(ti[0], 0, c, k1);
     SyiA[s] = mat(ti[1], 1, c, k2);
   }
+  if (UZERO && zero_ghosts)  // 16-byte stores; the patch's results follow after the barriers
+    for (int k = threadIdx.x; k < 18 * 18 * 18 * (int)sizeof(TO) / 16; k += 256)
+      reinterpret_cast<float4*>(out + p * L.ps)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   // f_copy = f, then modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson
   // :168-186), sides in the reference's order
   bool has[6];
@@ -333,8 +338,182 @@ __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restri
   }
 }
 
+// The same solve for 3D patches of 8^3 cells, one wavefront per patch (four to a workgroup) and
+// no workgroup barrier.  A 16 x 16 product takes four 8 x 8 planes at once, arranged 2 x 2, with
+// the axis matrix twice on the diagonal (half the matrix work is on zeros; it stays far below the
+// loads): the x and y products on four z-slices, the z products on the (z, x) planes of four
+// y-rows.  Chained through registers like dft3_mfma_kernel, with one crossing of the wave's own
+// LDS to the z products and one back, on pitches that spread each access over all banks.
+// Plane q = (column half) + 2 (row half) of tile t is slice (or row) 4t + q.
+// Latency of loads and LDS; 4,096 patches in FP32: 11.1 us from zero and 12.6 with interface
+// terms, where one 128-thread group per patch with dense products in VALU took 40 and 47.
+constexpr int k3Pitch8 = 72, k3Slab8 = 8 * k3Pitch8;  // words of a slice, of the patch
+
+template <typename T, typename TF, typename TO, int OP, bool UZERO>
+__global__ void __launch_bounds__(256) dft3_tile8_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
+                                                         const T* __restrict__ mats, const T* __restrict__ s2tab,
+                                                         const TF* __restrict__ f, const T* u,
+                                                         const T* __restrict__ coeffs, TO* out, int np, bool zero_ghosts)
+{
+  constexpr int SX = 10, SY = 100, PS = 1000;
+  __shared__ T slabs[4 * k3Slab8];
+  typedef typename Mf<T>::V V;
+  const int p = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (p >= np) return;
+  T* slab = slabs + (threadIdx.x >> 6) * k3Slab8;
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int* pt = ptype + p * 8;  // fwd type per axis [0..2], eig type per axis [3..5], zero mode [6]
+  const DevPatch& P = dp[p];
+  // as an operand lane (c, g) holds four cells x = 4 (g & 1) ... of row y = c & 7 in plane qa; in an
+  // accumulator register r is row Mf::row(r, g) and column c of the tile
+  const int y = c & 7, xlow = 4 * (g & 1), qa = (g >> 1) + 2 * (c >> 3);
+  const int row0 = p * PS + (y + 1) * SX + xlow + 1;
+  T F[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; t++) load_row4(f, row0 + (4 * t + qa + 1) * SY, F[t]);
+  int tf[3], ti[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    tf[a] = pt[a];
+    ti[a] = tf[a] == 0 ? 1 : (tf[a] == 3 ? 4 : tf[a]);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
+  }
+  // element (i, j) of the doubled matrix of axis a
+  auto mat = [&](int t, int a, int i, int j) {
+    const T m = mats[(t * 3 + a) * kDftMatStride + (i & 7) * 8 + (j & 7)];
+    return (i ^ j) & 8 ? T(0) : m;
+  };
+  T SxB[4], SyA[4], SzA[4], SziA[4], SxiB[4], SyiA[4];
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const int k1 = 4 * g + s, k2 = Mf<T>::row(s, g);
+    SxB[s] = mat(tf[0], 0, c, k1);
+    SyA[s] = mat(tf[1], 1, c, k2);
+    SzA[s] = mat(tf[2], 2, c, k1);
+    SziA[s] = mat(ti[2], 2, c, k2);
+    SxiB[s] = mat(ti[0], 0, c, k1);
+    SyiA[s] = mat(ti[1], 1, c, k2);
+  }
+  if (UZERO && zero_ghosts)  // 16-byte stores; the patch's results follow below
+    for (int k = lane; k < PS * (int)sizeof(TO) / 16; k += 64)
+      reinterpret_cast<float4*>(out + p * PS)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (!UZERO) {
+    // modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson :168-186), sides in the
+    // reference's order; every lane has one cell on an x face
+    bool has[6];
+    T ih[3];
+#pragma unroll
+    for (int s = 0; s < 6; s++) has[s] = P.type[20 + s] >= 0;
+#pragma unroll
+    for (int a = 0; a < 3; a++) ih[a] = T(P.inv_h2[a]);
+    const int xc = xlow ? 3 : 0;  // the lane's cell on its x face
+    const bool onx = xlow ? has[1] : has[0], ony = (y == 0 && has[2]) || (y == 7 && has[3]);
+    struct Face {
+      T xb, xg, b[4], y[4], z[4];
+    };
+    auto faces = [&](const T* v, int z, Face& q) {
+      const int r = row0 + (z + 1) * SY;
+      const bool onz = (z == 0 && has[4]) || (z == 7 && has[5]);
+      if (onx) {
+        q.xb = at(v, r + xc);
+        q.xg = at(v, xlow ? r + 4 : r - 1);
+      }
+      if (ony || onz) load_row4(v, r, q.b);
+      if (ony) load_row4(v, y == 0 ? r - SX : r + SX, q.y);
+      if (onz) load_row4(v, z == 0 ? r - SY : r + SY, q.z);
+    };
+    Face q[2], cq[OP == 1 ? 2 : 1];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      faces(u, 4 * t + qa, q[t]);
+      if (OP == 1) faces(coeffs, 4 * t + qa, cq[OP == 1 ? t : 0]);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int z = 4 * t + qa;
+      const Face& Q = q[t];
+      const Face& C = cq[OP == 1 ? t : 0];
+      auto sub = [&](T& v, T ug, T ub, T cg, T cb, T h) {
+        if (OP == 0) v -= (ug + ub) * h;
+        else v -= (ug + ub) * (cb + cg) * (h * T(0.5));
+      };
+      if (onx && !xlow) sub(F[t][0], Q.xg, Q.xb, C.xg, C.xb, ih[0]);
+      if (onx && xlow) sub(F[t][3], Q.xg, Q.xb, C.xg, C.xb, ih[0]);
+      if (ony) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) sub(F[t][k], Q.y[k], Q.b[k], C.y[k], C.b[k], ih[1]);
+      }
+      if ((z == 0 && has[4]) || (z == 7 && has[5])) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) sub(F[t][k], Q.z[k], Q.b[k], C.z[k], C.b[k], ih[2]);
+      }
+    }
+  }
+  // the place of accumulator register r of tile t: its plane's row and column, and the plane
+  auto arow = [&](int r) { return Mf<T>::row(r, g) & 7; };
+  auto aplane = [&](int t, int r) { return 4 * t + (c >> 3) + 2 * (Mf<T>::row(r, g) >> 3); };
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    V d1 = { 0, 0, 0, 0 };  // D1[y][kx] = sum_x F[y][x] Sx[kx][x]
+#pragma unroll
+    for (int s = 0; s < 4; s++) d1 = Mf<T>::mma(F[t][s], SxB[s], d1);
+    V d2 = { 0, 0, 0, 0 };  // D2[ky][kx] = sum_y Sy[ky][y] D1[y][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) d2 = Mf<T>::mma(SyA[s], d1[s], d2);
+#pragma unroll
+    for (int r = 0; r < 4; r++) slab[aplane(t, r) * k3Pitch8 + arow(r) * 8 + (c & 7)] = d2[r];
+  }
+  wave_sync();
+  const T lx = T(4.0 / (P.h[0] * P.h[0])), ly = T(4.0 / (P.h[1] * P.h[1])), lz = T(4.0 / (P.h[2] * P.h[2]));
+  const T s2x = s2tab[(pt[3] * 3 + 0) * kDftMatDim + (c & 7)];
+  V wz[2];
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    V b = { 0, 0, 0, 0 };  // W[kz][kx] = sum_z Sz[kz][z] D2[z][ky][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int z = (4 * g + s) & 7, ky = 4 * t + (c >> 3) + 2 * (g >> 1);
+      b = Mf<T>::mma(SzA[s], slab[z * k3Pitch8 + ky * 8 + (c & 7)], b);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {  // divide by the eigenvalues (:320-361)
+      const int kz = arow(r), ky = aplane(t, r);
+      T eig = T(0);
+      eig -= lx * s2x;
+      eig -= ly * s2tab[(pt[4] * 3 + 1) * kDftMatDim + ky];
+      eig -= lz * s2tab[(pt[5] * 3 + 2) * kDftMatDim + kz];
+      b[r] = b[r] / eig;
+      // all-Neumann patch without neighbours (:438-440)
+      if (pt[6] && ky == 0 && kz == 0 && (c & 7) == 0) b[r] = T(0);
+    }
+    V b2 = { 0, 0, 0, 0 };  // W'[z][kx] = sum_kz Szi[z][kz] W[kz][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) b2 = Mf<T>::mma(SziA[s], b[s], b2);
+    wz[t] = b2;
+  }
+  wave_sync();
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) slab[arow(r) * k3Pitch8 + aplane(t, r) * 8 + (c & 7)] = wz[t][r];
+  wave_sync();
+  if (UZERO && zero_ghosts) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  const T scale = T(2.0) / T(8) * (T(2.0) / T(8)) * (T(2.0) / T(8));
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    V r1 = { 0, 0, 0, 0 };  // R[ky][x] = sum_kx Q[ky][kx] Sxi[x][kx]
+#pragma unroll
+    for (int s = 0; s < 4; s++) r1 = Mf<T>::mma(slab[(4 * t + qa) * k3Pitch8 + y * 8 + xlow + s], SxiB[s], r1);
+    V u2 = { 0, 0, 0, 0 };  // U[y][x] = sum_ky Syi[y][ky] R[ky][x]
+#pragma unroll
+    for (int s = 0; s < 4; s++) u2 = Mf<T>::mma(SyiA[s], r1[s], u2);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      at(out, p * PS + (aplane(t, r) + 1) * SY + (arow(r) + 1) * SX + (c & 7) + 1) = TO(u2[r] * scale);
+  }
+}
+
 template <typename T, typename TF, typename TO, int D>
-void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, hipStream_t s)
+void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, bool zg, hipStream_t s)
 {
   const te_domain* d = pl->g->d;
   Layout L = make_layout(d->dim, d->ns, 1, d->np);
@@ -351,13 +530,25 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
   if (D == 3 && pl->use_mfma && d->ns[0] == 16 && d->ns[1] == 16 && d->ns[2] == 16) {
 #define TE_D3(OP_, UZ_)                                                                                         \
   hipLaunchKernelGGL((dft3_mfma_kernel<T, TF, TO, OP_, UZ_>), dim3(d->np), dim3(256), 0, s, d->d_patches,     \
-                     pl->d_ptype, mats, s2, f, u, cf, out, L)
+                     pl->d_ptype, mats, s2, f, u, cf, out, L, zg)
     if (pl->op_kind == 0) {
       if (uzero) TE_D3(0, true); else TE_D3(0, false);
     } else {
       if (uzero) TE_D3(1, true); else TE_D3(1, false);
     }
 #undef TE_D3
+    return;
+  }
+  if (D == 3 && pl->use_mfma && d->ns[0] == 8 && d->ns[1] == 8 && d->ns[2] == 8) {
+#define TE_D8(OP_, UZ_)                                                                                         \
+  hipLaunchKernelGGL((dft3_tile8_kernel<T, TF, TO, OP_, UZ_>), dim3((d->np + 3) / 4), dim3(256), 0, s,          \
+                     d->d_patches, pl->d_ptype, mats, s2, f, u, cf, out, d->np, zg)
+    if (pl->op_kind == 0) {
+      if (uzero) TE_D8(0, true); else TE_D8(0, false);
+    } else {
+      if (uzero) TE_D8(1, true); else TE_D8(1, false);
+    }
+#undef TE_D8
     return;
   }
   // patches per workgroup and threads per patch: the autotuner's choice for this shape
@@ -377,10 +568,10 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
 }
 
 template <typename T, typename TF, typename TO>
-void launch_t(const te_dft_plan* pl, const void* f, const void* u, void* out, bool uzero, hipStream_t s)
+void launch_t(const te_dft_plan* pl, const void* f, const void* u, void* out, bool uzero, bool zg, hipStream_t s)
 {
-  if (pl->g->d->dim == 2) launch_d<T, TF, TO, 2>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, s);
-  else launch_d<T, TF, TO, 3>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, s);
+  if (pl->g->d->dim == 2) launch_d<T, TF, TO, 2>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, zg, s);
+  else launch_d<T, TF, TO, 3>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, zg, s);
 }
 
 // the fused sweeps of the generic kernel, 2D: gm 0 (ghosts read from u), 1 (computed here),
@@ -481,14 +672,23 @@ int launch_dft_fused(const te_dft_plan* pl, int dt, int dtf, int dto, const void
 }
 
 int launch_dft(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, const void* u, void* out, bool uzero,
-               hipStream_t s)
+               hipStream_t s, bool zero_ghosts)
 {
-  if (pl->g->d->np == 0) return TE_OK;
+  const te_domain* d = pl->g->d;
+  if (d->np == 0) return TE_OK;
+  // the 3D matrix-core kernels zero the ghosts themselves, where the patches start on 16 bytes
+  const bool own = pl->use_mfma && d->dim == 3 && (d->ns[0] == 8 || d->ns[0] == 16) && d->ns[1] == d->ns[0] &&
+                   d->ns[2] == d->ns[0] && uzero && f != out && (uintptr_t)out % 16 == 0;
+  const bool zg = zero_ghosts && own;
+  if (zero_ghosts && !own) {
+    int rc = launch_vec_op(d, dto, VOP_SET_WITH_GHOST, out, nullptr, nullptr, 0.0, 0, 0, 1, s);
+    if (rc) return rc;
+  }
   if (pl->use_mfma && dft_mfma_supported(pl)) return launch_dft_mfma(pl, dt, dtf, dto, f, u, out, uzero, s);
-  if (dt == TE_F64 && dtf == TE_F64 && dto == TE_F64) launch_t<double, double, double>(pl, f, u, out, uzero, s);
-  else if (dt == TE_F32 && dtf == TE_F32 && dto == TE_F32) launch_t<float, float, float>(pl, f, u, out, uzero, s);
-  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F32) launch_t<float, double, float>(pl, f, u, out, uzero, s);
-  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F64) launch_t<float, double, double>(pl, f, u, out, uzero, s);
+  if (dt == TE_F64 && dtf == TE_F64 && dto == TE_F64) launch_t<double, double, double>(pl, f, u, out, uzero, zg, s);
+  else if (dt == TE_F32 && dtf == TE_F32 && dto == TE_F32) launch_t<float, float, float>(pl, f, u, out, uzero, zg, s);
+  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F32) launch_t<float, double, float>(pl, f, u, out, uzero, zg, s);
+  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F64) launch_t<float, double, double>(pl, f, u, out, uzero, zg, s);
   else {
     set_error("unsupported dtype combination for the DFT patch solver");
     return TE_ERR_UNSUPPORTED;
