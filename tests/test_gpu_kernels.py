@@ -613,3 +613,30 @@ def test_restrict_extrapolate(name, ns, ncomp):
     assert np.max(np.abs(c32.get() - ref)) <= 1e-5 * np.max(np.abs(ref))
     link.restrict(dfv, dcv)
     assert np.array_equal(dcv.get(), O.restrict(of, oc, fv))
+
+
+@pytest.mark.parametrize("level", [0, 1, 2])
+@pytest.mark.parametrize("op_kind", [0, 1])
+@pytest.mark.parametrize("kind", [R.BILINEAR, R.BIQUADRATIC])
+def test_dft32_pair(level, op_kind, kind):
+    """The 32^2 patch solve on 1, 4 and 7 patches (fewer than the launch's eight groups and one
+    more; refined at the largest): ghosts read from u in place, and the zero-u apply."""
+    ns = (32, 32)
+    lv = solver.uniform_levels(2, level, ns)[0] if level < 2 else load("2d_uniform_2x2_refined_nw_mpi1.json", ns)[1][0]
+    od, dd = O.Domain(2, ns, lv), _dev(2, ns, lv)
+    coeffs = None
+    if op_kind == 1:
+        X = mesh.cell_centers(lv, 2, ns)
+        coeffs = np.exp(np.sin(3 * X[..., 0]) * np.cos(2 * X[..., 1]))[:, None].copy()
+        O.fill_ghost(od, coeffs, kind=kind)
+    plan = R.DftPlan(R.GhostFiller(dd, kind, R.FACES), op_kind=op_kind,
+                     coeffs=R.DeviceArray.from_host(coeffs) if op_kind else None)
+    for dtype, tol in [(R.F64, 1e-12), (R.F32, 2e-5)]:
+        t = R.np_dtype(dtype)
+        f0, u0 = random_field(od.shape(1), 33, t), random_field(od.shape(1), 34, t)
+        for zero in (False, True):
+            uref = np.zeros(od.shape(1)) if zero else u0.astype(np.float64)
+            O.dft_smooth(od, f0.astype(np.float64), uref, kind=kind, op_kind=op_kind, coeffs=coeffs)
+            du = R.DeviceArray.from_host(u0)
+            (plan.apply if zero else plan.smooth)(R.DeviceArray.from_host(f0), du)
+            assert relerr(mesh.interior(du.get(), 2), mesh.interior(uref, 2)) <= tol, (dtype, zero)

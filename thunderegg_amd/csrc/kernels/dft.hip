@@ -171,20 +171,6 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
 // 2,535 patches 43 us (the vectors' padded lines in 36 at a copy's rate) against 95.
 constexpr int k3N = 16, k3Row = 20, k3Slice = 16 * k3Row + 4, k3Slab = 16 * k3Slice;
 
-// four consecutive values at an address that is a multiple of TS only (rows of 18 values)
-template <typename T, typename TS>
-__device__ __forceinline__ void load_row4(const TS* base, int idx, T (&r)[4])
-{
-  constexpr int W = 16 / sizeof(TS);
-  typedef TS Vec __attribute__((ext_vector_type(W), aligned(sizeof(TS))));
-#pragma unroll
-  for (int k = 0; k < 4; k += W) {
-    const Vec v = *reinterpret_cast<const Vec*>(&at(base, idx + k));
-#pragma unroll
-    for (int j = 0; j < W; j++) r[k + j] = T(v[j]);
-  }
-}
-
 template <typename T, typename TF, typename TO, int OP, bool UZERO>
 __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
                                                         const T* __restrict__ mats, const T* __restrict__ s2tab,

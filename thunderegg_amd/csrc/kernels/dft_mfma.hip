@@ -1,7 +1,7 @@
 // DFTPatchSolver::solveSinglePatch (Poisson/DFTPatchSolver.h:420-450) on the
-// matrix cores, 2D, all-Dirichlet patches, n = 16 or 32.
+// matrix cores, 2D, all-Dirichlet patches, n = 16 or 32 (dft32_kernel: two waves a patch).
 //
-// Each wavefront solves one patch: U = S3 . ((S . F . S^T) / lambda) . S3^T * (2/n)^2,
+// n = 16: each wavefront solves one patch: U = S3 . ((S . F . S^T) / lambda) . S3^T * (2/n)^2,
 // with S the DST-II and S3 the DST-III matrix (the reference's per-line dgemv along
 // x, then along y, :205-265).  Every product is a sequence of 16x16x4 MFMAs
 // (v_mfma_f32_16x16x4_f32 / v_mfma_f64_16x16x4_f64) over 16x16 tiles:
@@ -38,15 +38,15 @@ constexpr int kWaves = 4;
 // PF (n = 16): each wave walks several patches and loads the next one while it solves the
 // current one; without PF (levels where each wave gets about one patch) a patch's loads come
 // right before its solve, which needs fewer registers, so more waves fit a SIMD.
-template <typename T, typename TF, typename TO, typename TC, int NT, int OP, bool UZERO, int GM, int KIND, bool PF>
-__global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF ? (GM == 0 ? 5 : 4) : (GM == 0 ? 8 : (KIND == TE_BILINEAR ? 5 : 4))) : 1) dft_mfma_kernel(const DevPatch* __restrict__ dp,
+template <typename T, typename TF, typename TO, typename TC, int OP, bool UZERO, int GM, int KIND, bool PF>
+__global__ void __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? (PF ? (GM == 0 ? 5 : 4) : (GM == 0 ? 8 : (KIND == TE_BILINEAR ? 5 : 4))) : 1) dft_mfma_kernel(const DevPatch* __restrict__ dp,
                                                                const T* __restrict__ mats, const T* __restrict__ s2tab,
                                                                const TF* __restrict__ f, const T* __restrict__ u,
                                                                const T* __restrict__ coeffs, TO* __restrict__ out,
                                                                Layout L, FusedArgs<T, TC> fa,
                                                                const int4* __restrict__ ring)
 {
-  constexpr int n = 16 * NT;
+  constexpr int n = 16;
   constexpr int ld = n + 1;  // padded LDS row
   // the padded layout of a one-component vector of n x n patches (L.sx, L.ps = L.cs) as
   // compile-time constants: the address arithmetic folds into shifts and adds
@@ -66,9 +66,9 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
   const int lane = threadIdx.x & 63;
   T* X = s2 + n + wave * n * ld;  // per-wave scratch n x ld
   T* Bt = s2 + n + kWaves * n * ld + wave * 4 * n;  // per-wave interface terms of the 4 sides
-  // n = 16 with ghosts computed here: the patch's own values (u, or u + P uc) are staged
+  // with ghosts computed here: the patch's own values (u, or u + P uc) are staged
   // in a padded tile first, so the ghost formulas read their self terms from LDS
-  constexpr bool TILE = GM != 0 && NT == 1;
+  constexpr bool TILE = GM != 0;
   T* Tl = s2 + n + kWaves * n * ld + kWaves * 4 * n + wave * (n + 2) * (n + 2);
   UAcc<T, TC, GM == 2> U{ u, fa.uc, fa.parent, fa.porth, L };
 
@@ -82,25 +82,24 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
   // Each wave walks its own patches with private LDS (X, Bt, Tl): wave-level ordering
   // suffices inside the loop.  The one workgroup barrier orders the shared matrices; the
   // wave's first patch is staged before it so that its loads overlap the matrices'.
-  SideInfo si[NT];  // ring cells lane + 64 j: side j * 64 / n + lane / n
+  SideInfo si[1];  // the lane's ring cell: side lane / n
   // ---- f_copy = f (interior) into LDS; the side information of the ghost pass is
   //      loaded at the same time
-  // n = 16: the next patch's right-hand side is loaded into registers while this one is
+  // the next patch's right-hand side is loaded into registers while this one is
   // solved (FPL values per lane), so a wave's loads overlap its own arithmetic
   constexpr int FPL = n * n / 64;
-  constexpr bool PREF = NT == 1;
-  TF fn[PREF ? FPL : 1];
+  TF fn[FPL];
   auto fload = [&](int p) {
     const int base = p * PS;
 #pragma unroll
-    for (int k = 0; k < (PREF ? FPL : 1); k++) {
+    for (int k = 0; k < FPL; k++) {
       const int q = lane + 64 * k, y = q / n, x = q - y * n;
       fn[k] = at(f, base + (y + 1) * SX + x + 1);
     }
   };
   auto fput = [&]() {
 #pragma unroll
-    for (int k = 0; k < (PREF ? FPL : 1); k++) {
+    for (int k = 0; k < FPL; k++) {
       const int q = lane + 64 * k, y = q / n, x = q - y * n;
       X[y * ld + x] = T(fn[k]);
     }
@@ -109,18 +108,17 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
   // (ring table: lane = ring cell, side lane / n, cell lane % n), then, once those have
   // arrived (mid-iteration), its coarse-level values and the neighbour values of every
   // lane's ghost cell (ghost2d_gather; with GM_INTERP each as u and coarse u separately)
-  constexpr bool PREF_T = TILE && PREF;
-  T un[PREF_T ? FPL : 1];
-  TC ucn[PREF_T ? FPL : 1];
+    T un[TILE ? FPL : 1];
+  TC ucn[TILE ? FPL : 1];
   int on = -1, parn = 0;
   int4 rn = make_int4(-1, 0, -1, 0), rc = rn;  // ring records of the next / current patch
   T gu[4];
   TC gc[4];
   T gv[4];  // the current patch's neighbour values (u, or u + P uc)
-  const int rs = lane / n, rt = lane - (lane / n) * n;  // the lane's ring cell (PREF_T: 4 n = 64)
+  const int rs = lane / n, rt = lane - (lane / n) * n;  // the lane's ring cell (TILE: 4 n = 64)
   auto tload_a = [&](int p) {
 #pragma unroll
-    for (int k = 0; k < (PREF_T ? FPL : 1); k++) {
+    for (int k = 0; k < (TILE ? FPL : 1); k++) {
       const int q = lane + 64 * k, y = q / n, x = q - y * n;
       un[k] = at(u, p * PS + (y + 1) * SX + x + 1);
     }
@@ -133,7 +131,7 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
   auto tload_b = [&]() {
     if (GM == 2) {
 #pragma unroll
-      for (int k = 0; k < (PREF_T ? FPL : 1); k++) {
+      for (int k = 0; k < (TILE ? FPL : 1); k++) {
         const int q = lane + 64 * k, y = q / n, x = q - y * n;
         int cx = x, cy = y;
         if (on >= 0) {
@@ -164,7 +162,7 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
   };
   auto tput = [&]() {  // the values UAcc would return, staged from the registers
 #pragma unroll
-    for (int k = 0; k < (PREF_T ? FPL : 1); k++) {
+    for (int k = 0; k < (TILE ? FPL : 1); k++) {
       const int q = lane + 64 * k, y = q / n, x = q - y * n;
       Tl[(y + 1) * (n + 2) + x + 1] = GM == 2 ? T(un[k] + T(ucn[k])) : un[k];
     }
@@ -173,28 +171,19 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
     for (int k = 0; k < 4; k++) gv[k] = GM == 2 ? T(gu[k] + T(gc[k])) : gu[k];
   };
   auto stage = [&](int p) {
-    if (PREF_T) {
+    if (TILE) {
       fput();
       tput();
       return;
     }
-    if (PREF) {
-      fput();
-    } else {
-      const int base = p * PS;
-      for (int q = lane; q < n * n; q += 64) {
-        int y = q / n, x = q - y * n;
-        X[y * ld + x] = T(f[base + (y + 1) * SX + x + 1]);
-      }
-    }
-    if (TILE) tile_interior_2d<T>(p, n, n, U, Tl, lane);
-    if (!UZERO) ring_prefetch<NT>(dp[p], n, n, lane, si);
+    fput();
+    if (!UZERO) ring_prefetch<1>(dp[p], n, n, lane, si);
   };
   const XcdRange xr = xcd_range(blockIdx.x, gridDim.x, L.np, kWaves);
   int p = xr.first + wave;
   if (PF && p < xr.end) {
-    if (PREF) fload(p);
-    if (PREF_T) {
+    fload(p);
+    if (TILE) {
       tload_a(p);
       tload_b();
     }
@@ -203,8 +192,8 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
   __syncthreads();
   for (bool first = true; p < xr.end; p += xr.step, first = false) {
     if (!PF) {
-      if (PREF) fload(p);
-      if (PREF_T) {
+      fload(p);
+      if (TILE) {
         tload_a(p);
         tload_b();
       }
@@ -215,8 +204,8 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
       wave_sync();
     }
     const bool has_next = PF && p + xr.step < xr.end;
-    if (PREF && has_next) fload(p + xr.step);
-    if (PREF_T && has_next) tload_a(p + xr.step);
+    if (has_next) fload(p + xr.step);
+    if (TILE && has_next) tload_a(p + xr.step);
     const int base = p * PS;
     const DevPatch& P = dp[p];
     // ---- modifyRHSForInternalBoundaryConditions: the interface term of every side cell
@@ -224,13 +213,12 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
     //      then applied west/east first, then south/north (sides in increasing order,
     //      Poisson/StarPatchOperator.h:165-180)
     if (!UZERO) {
-#pragma unroll
-      for (int j = 0; j < NT; j++) {  // 4 n = 64 NT ring cells
-        const int q = lane + 64 * j;
+      {  // 4 n = 64 ring cells
+        const int q = lane;
         const int s = q / n, t = q - s * n;
         const int ph = s >> 1, up = s & 1;
         T term = T(0);
-        if ((PREF_T ? rc.x : si[j].type) >= 0) {
+        if ((TILE ? rc.x : si[0].type) >= 0) {
           int gi, bi;  // padded index of the ghost and of the boundary cell
           int bx, by;  // boundary cell
           if (ph == 0) {
@@ -248,7 +236,7 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
           if (GM == 0) {
             ug = u[gi];
             ub = u[bi];
-          } else if (PREF_T) {
+          } else {
             // self terms from the tile, neighbour terms gathered during the previous patch
             ug = ghost2d_combine<T, KIND>(rc.x, rc.y, t, n,
                                           [&](int k, int tt) {
@@ -258,13 +246,6 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
                                           },
                                           gv);
             ub = Tl[(by + 1) * (n + 2) + bx + 1];
-          } else if (TILE) {
-            TileAcc<T, UAcc<T, TC, GM == 2>> A{ Tl, p, n + 2, U };
-            ug = ghost2d<T, KIND>(si[j], p, s, t, n, n, A);
-            ub = Tl[(by + 1) * (n + 2) + bx + 1];
-          } else {
-            ug = ghost2d<T, KIND>(si[j], p, s, t, n, n, U);
-            ub = U(p, bx, by);
           }
           const T ih2 = T(P.inv_h2[ph]);
           if (OP == 0) {
@@ -276,7 +257,7 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
         }
         Bt[q] = term;
       }
-      if (PREF_T && has_next) tload_b();
+      if (TILE && has_next) tload_b();
       wave_sync();
 #pragma unroll
       for (int ph = 0; ph < 2; ph++) {
@@ -291,19 +272,19 @@ __global__ void __launch_bounds__(64 * kWaves, (NT == 1 && sizeof(T) == 4) ? (PF
       }
     }
     const T lx = T(4.0 / (P.h[0] * P.h[0])), ly = T(4.0 / (P.h[1] * P.h[1]));
-    dft_solve_wave<T, TO, NT>(X, Sm, S3, s2, lx, ly, out, base, SX, true);
+    dft_solve_wave<T, TO, 1>(X, Sm, S3, s2, lx, ly, out, base, SX, true);
     wave_sync();  // X and the tile are rewritten by the next patch
   }
 }
 
-template <typename T, typename TF, typename TO, typename TC, int NT>
-void launch_nt(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, int gm, const TC* uc,
+template <typename T, typename TF, typename TO, typename TC>
+void launch_n16(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, int gm, const TC* uc,
                const te_level_link* link, hipStream_t s)
 {
   const te_domain* d = pl->g->d;
   Layout L = make_layout(2, d->ns, 1, d->np);
-  constexpr int n = 16 * NT;
-  const bool tile = gm != 0 && NT == 1;
+  constexpr int n = 16;
+  const bool tile = gm != 0;
   size_t shmem = sizeof(T) * (2 * n * (n + 1) + n + kWaves * n * (n + 1) + kWaves * 4 * n +
                               (tile ? kWaves * (n + 2) * (n + 2) : 0));
   const T* mats = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_mats64 : (const void*)pl->d_mats32);
@@ -316,30 +297,24 @@ void launch_nt(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uze
   const int kind = pl->g->kind;
   // the workgroup count: the autotuner's choice for this patch size and type (tune.h)
   const int var = tune_variant(TUNE_DFT_MFMA_2D, 2, n, sizeof(T) == 8 ? TE_F64 : TE_F32);
-  // n = 16: when every workgroup (one patch per wave) is resident at once, one round of
+  // when every workgroup (one patch per wave) is resident at once, one round of
   // the plain variant; else the prefetching variant (the next patch loaded during the
   // current solve) on as many workgroups as are resident at once, each wave solving
-  // several patches.  n = 32: at most 4096 workgroups.
+  // several patches.
 #define TE_MK1(OP_, UZ_, GM_, K_, PF_, G_)                                                                    \
-  hipLaunchKernelGGL((dft_mfma_kernel<T, TF, TO, TC, NT, OP_, UZ_, GM_, K_, PF_>), dim3(G_), dim3(64 * kWaves), \
+  hipLaunchKernelGGL((dft_mfma_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_, PF_>), dim3(G_), dim3(64 * kWaves), \
                      shmem, s, d->d_patches, mats, s2, f, u, cf, out, L, fa, ring)
 #define TE_MK(OP_, UZ_, GM_, K_)                                                                            \
   do {                                                                                                      \
-    if constexpr (NT == 1) {                                                                                \
-      const void* plain = (const void*)dft_mfma_kernel<T, TF, TO, TC, NT, OP_, UZ_, GM_, K_, false>;        \
-      if (var == MFMA_GRID_ALL ||                                                                           \
-          (var == MFMA_GRID_DEFAULT && ngroups <= resident_blocks(plain, 64 * kWaves, shmem))) {            \
-        TE_MK1(OP_, UZ_, GM_, K_, false, ngroups);                                                          \
-      } else {                                                                                              \
-        int r = resident_blocks((const void*)dft_mfma_kernel<T, TF, TO, TC, NT, OP_, UZ_, GM_, K_, true>,   \
-                                64 * kWaves, shmem);                                                        \
-        if (var == MFMA_GRID_HALF) r = r > 1 ? r / 2 : 1;                                                   \
-        TE_MK1(OP_, UZ_, GM_, K_, true, ngroups < r ? ngroups : r);                                         \
-      }                                                                                                     \
+    const void* plain = (const void*)dft_mfma_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_, false>;              \
+    if (var == MFMA_GRID_ALL ||                                                                             \
+        (var == MFMA_GRID_DEFAULT && ngroups <= resident_blocks(plain, 64 * kWaves, shmem))) {              \
+      TE_MK1(OP_, UZ_, GM_, K_, false, ngroups);                                                            \
     } else {                                                                                                \
-      const int cap = var == MFMA_GRID_RESIDENT ? 2048 : var == MFMA_GRID_HALF ? 8192                      \
-                      : var == MFMA_GRID_ALL    ? ngroups : 4096;                                           \
-      TE_MK1(OP_, UZ_, GM_, K_, false, ngroups < cap ? ngroups : cap);                                      \
+      int r = resident_blocks((const void*)dft_mfma_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_, true>,         \
+                              64 * kWaves, shmem);                                                          \
+      if (var == MFMA_GRID_HALF) r = r > 1 ? r / 2 : 1;                                                     \
+      TE_MK1(OP_, UZ_, GM_, K_, true, ngroups < r ? ngroups : r);                                           \
     }                                                                                                       \
   } while (0)
 #define TE_MKG(OP_)                                                         \
@@ -359,14 +334,202 @@ void launch_nt(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uze
 #undef TE_MK1
 }
 
+// n = 32: two waves per patch, wave J the 16 columns J of every product but the last's operand,
+// which is the one exchange through LDS (dft_mfma_kernel's n = 16 scheme on 2 x 2 tiles would
+// keep 64 accumulator values and read both operands of every MFMA from LDS):
+//   Y[I][J] = sum_K F[I][K] S^T[K][J]   F from memory in the operand layout (four cells a lane)
+//   Z[I][J] = sum_K S[I][K] Y[K][J]     Y, Z' and V chained through registers, as for n = 16
+//   V[I][J] = sum_K S3[I][K] Z'[K][J]
+//   U[I][J] = sum_K V[I][K] S3^T[K][J]  V through LDS
+// The matrices' operands live in registers (48 a lane).  The interface terms come first, one of
+// the 128 side cells per thread, and are subtracted in the operand layout, west / east then
+// south / north (Poisson/StarPatchOperator.h:165-180).
+// Against one wave a patch: 48 problems of up to 2,400 patches, a third of them 32^2, solved together
+// (mixed): 15.3 -> 13.1 ms.
+template <typename T, typename TF, typename TO, typename TC, int OP, bool UZERO, int GM, int KIND>
+__global__ void __launch_bounds__(128) dft32_kernel(const DevPatch* __restrict__ dp, const T* __restrict__ mats,
+                                                    const T* __restrict__ s2tab, const TF* __restrict__ f, const T* u,
+                                                    const T* __restrict__ coeffs, TO* out, int np, FusedArgs<T, TC> fa,
+                                                    const int4* __restrict__ ring)
+{
+  constexpr int n = 32, SX = n + 2, PS = SX * SX, LD = n + 4;
+  typedef typename Mf<T>::V V;
+  __shared__ __align__(16) T X[n * LD];
+  __shared__ T term[UZERO ? 1 : 4 * n];
+  const int p = xcd_item(blockIdx.x, gridDim.x);
+  if (p >= np) return;
+  const int J = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const DevPatch& P = dp[p];
+  const int base = p * PS + SX + 1;  // cell (0, 0)
+  // F[I][K][s]: row 16 I + c, column 16 K + 4 g + s
+  T F[2][2][4];
+#pragma unroll
+  for (int I = 0; I < 2; I++)
+#pragma unroll
+    for (int K = 0; K < 2; K++) load_row4(f, base + (16 * I + c) * SX + 16 * K + 4 * g, F[I][K]);
+  if (!UZERO) {
+    const int s = threadIdx.x >> 5, t = threadIdx.x & 31, ph = s >> 1, up = s & 1;
+    int bx, by;
+    side_xy(s, 0, t, n, &bx, &by);
+    const int bi = base + by * SX + bx, gi = bi + (up ? 1 : -1) * (ph == 0 ? 1 : SX);
+    T v = T(0);
+    if (GM == 0) {
+      if (P.type[4 + s] >= 0) v = u[gi] + u[bi];
+    } else {
+      const int4 r = ring[(p * 4 + s) * 2 + (2 * t >= n ? 1 : 0)];
+      // u, or u + P uc: parent and orthant of patch q
+      auto val = [&](int q, int par, int o, int x, int y) {
+        T a = at(u, q * PS + (y + 1) * SX + x + 1);
+        if (GM == 2) {
+          const int cx = o >= 0 ? (x + ((o & 1) ? n : 0)) / 2 : x, cy = o >= 0 ? (y + ((o & 2) ? n : 0)) / 2 : y;
+          a = T(a + T(at(fa.uc, par * PS + (cy + 1) * SX + cx + 1)));
+        }
+        return a;
+      };
+      if (r.x >= 0) {
+        const int par = GM == 2 ? fa.parent[p] : 0, o = GM == 2 ? fa.porth[p] : -1;
+        T gv[4] = { T(0), T(0), T(0), T(0) };
+        ghost2d_gather<KIND>(r.x, r.y, r.z, s, t, n, n,
+                             [&](int k, int q, int x, int y) { gv[k] = val(q, r.w >> 3, (r.w & 7) - 1, x, y); });
+        const T ug = ghost2d_combine<T, KIND>(r.x, r.y, t, n,
+                                              [&](int k, int tt) {
+                                                int x, y;
+                                                side_xy(s, k, tt, n, &x, &y);
+                                                return val(p, par, o, x, y);
+                                              },
+                                              gv);
+        v = ug + val(p, par, o, bx, by);
+      }
+    }
+    const T ih2 = T(P.inv_h2[ph]);
+    if (OP == 0) v = v * ih2;
+    else if (P.type[4 + s] >= 0) v = v * (coeffs[bi] + coeffs[gi]) * (ih2 * T(0.5));
+    term[s * n + t] = v;  // 0 on physical sides
+  }
+  // the matrices as operands: lane (c, g), step s holds element (16 B + c, K index)
+  auto mat = [&](int ty, int i, int k) { return mats[(ty * 3) * kDftMatStride + i * n + k]; };  // axis 0; 3: DST-II, 4: DST-III
+  T SB[2][4], S3B[2][4], SA[2][2][4], S3A[2][2][4];
+#pragma unroll
+  for (int K = 0; K < 2; K++)
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      SB[K][s] = mat(3, 16 * J + c, 16 * K + 4 * g + s);
+      S3B[K][s] = mat(4, 16 * J + c, 16 * K + 4 * g + s);
+#pragma unroll
+      for (int I = 0; I < 2; I++) {
+        SA[I][K][s] = mat(3, 16 * I + c, 16 * K + Mf<T>::row(s, g));
+        S3A[I][K][s] = mat(4, 16 * I + c, 16 * K + Mf<T>::row(s, g));
+      }
+    }
+  if (!UZERO) {
+    __syncthreads();
+#pragma unroll
+    for (int I = 0; I < 2; I++) {
+      if (g == 0) F[I][0][0] -= term[16 * I + c];
+      if (g == 3) F[I][1][3] -= term[n + 16 * I + c];
+    }
+#pragma unroll
+    for (int K = 0; K < 2; K++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        if (c == 0) F[0][K][s] -= term[2 * n + 16 * K + 4 * g + s];
+        if (c == 15) F[1][K][s] -= term[3 * n + 16 * K + 4 * g + s];
+      }
+  }
+  V Y[2], Z[2];
+#pragma unroll
+  for (int I = 0; I < 2; I++) {
+    V acc = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int K = 0; K < 2; K++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(F[I][K][s], SB[K][s], acc);
+    Y[I] = acc;
+  }
+  const T lx = T(4.0 / (P.h[0] * P.h[0])), ly = T(4.0 / (P.h[1] * P.h[1]));
+  const T* s2 = s2tab + (2 * 3 + 0) * kDftMatDim;
+  const T s2x = s2[16 * J + c];
+#pragma unroll
+  for (int I = 0; I < 2; I++) {
+    V acc = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int K = 0; K < 2; K++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(SA[I][K][s], Y[K][s], acc);
+    // divide by the eigenvalues -4/hx^2 s2[kx] - 4/hy^2 s2[ky] (getEigenValues, :320-361)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      T eig = T(0);
+      eig -= lx * s2x;
+      eig -= ly * s2[16 * I + Mf<T>::row(r, g)];
+      // FP32: the hardware reciprocal (1 ulp) instead of a correctly rounded division
+      if (sizeof(T) == 4) acc[r] = acc[r] * T(__builtin_amdgcn_rcpf(float(eig)));
+      else acc[r] = acc[r] / eig;
+    }
+    Z[I] = acc;
+  }
+#pragma unroll
+  for (int I = 0; I < 2; I++) {
+    V acc = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int K = 0; K < 2; K++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(S3A[I][K][s], Z[K][s], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) X[(16 * I + Mf<T>::row(r, g)) * LD + 16 * J + c] = acc[r];
+  }
+  __syncthreads();
+  const T scale = T(4.0 / double(n * n));  // prod over axes of 2/n (:442-449)
+#pragma unroll
+  for (int I = 0; I < 2; I++) {
+    V acc = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int K = 0; K < 2; K++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(X[(16 * I + c) * LD + 16 * K + 4 * g + s], S3B[K][s], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) at(out, base + (16 * I + Mf<T>::row(r, g)) * SX + 16 * J + c) = TO(acc[r] * scale);
+  }
+}
+
+template <typename T, typename TF, typename TO, typename TC>
+void launch_n32(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, int gm, const TC* uc,
+                const te_level_link* link, hipStream_t s)
+{
+  const te_domain* d = pl->g->d;
+  const T* mats = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_mats64 : (const void*)pl->d_mats32);
+  const T* s2 = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_s2_64 : (const void*)pl->d_s2_32);
+  const T* cf = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_coeffs64 : (const void*)pl->d_coeffs32);
+  FusedArgs<T, TC> fa{ uc, link ? link->d_parent : nullptr, link ? link->d_orth : nullptr };
+  const int4* ring = (const int4*)(gm == 2 ? link->d_ring : d->d_ring);
+  const int kind = pl->g->kind;
+#define TE_M32(OP_, UZ_, GM_, K_)                                                                                    \
+  hipLaunchKernelGGL((dft32_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_>), dim3(xcd_grid(d->np)), dim3(128), 0, s,       \
+                     d->d_patches, mats, s2, f, u, cf, out, d->np, fa, ring)
+#define TE_M32G(OP_)                                                             \
+  if (uzero) TE_M32(OP_, true, 0, 0);                                            \
+  else if (gm == 0) TE_M32(OP_, false, 0, 0);                                    \
+  else if (gm == 1 && kind == TE_BILINEAR) TE_M32(OP_, false, 1, TE_BILINEAR);   \
+  else if (gm == 1) TE_M32(OP_, false, 1, TE_BIQUADRATIC);                       \
+  else if (kind == TE_BILINEAR) TE_M32(OP_, false, 2, TE_BILINEAR);              \
+  else TE_M32(OP_, false, 2, TE_BIQUADRATIC);
+  if (pl->op_kind == 0) {
+    TE_M32G(0)
+  } else {
+    TE_M32G(1)
+  }
+#undef TE_M32G
+#undef TE_M32
+}
+
 template <typename T, typename TF, typename TO, typename TC>
 void launch_t(const te_dft_plan* pl, const void* f, const void* u, void* out, bool uzero, int gm, const void* uc,
               const te_level_link* link, hipStream_t s)
 {
   if (pl->g->d->ns[0] == 16)
-    launch_nt<T, TF, TO, TC, 1>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, gm, (const TC*)uc, link, s);
+    launch_n16<T, TF, TO, TC>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, gm, (const TC*)uc, link, s);
   else
-    launch_nt<T, TF, TO, TC, 2>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, gm, (const TC*)uc, link, s);
+    launch_n32<T, TF, TO, TC>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, gm, (const TC*)uc, link, s);
 }
 
 

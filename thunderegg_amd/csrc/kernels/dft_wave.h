@@ -28,6 +28,20 @@ struct Mf<double> {
   static __device__ __forceinline__ int row(int r, int g) { return 4 * r + g; }
 };
 
+// four consecutive values at an address that is a multiple of TS only (rows of n + 2 values)
+template <typename T, typename TS>
+__device__ __forceinline__ void load_row4(const TS* base, int idx, T (&r)[4])
+{
+  constexpr int W = 16 / sizeof(TS);
+  typedef TS Vec __attribute__((ext_vector_type(W), aligned(sizeof(TS))));
+#pragma unroll
+  for (int k = 0; k < 4; k += W) {
+    const Vec v = *reinterpret_cast<const Vec*>(&at(base, idx + k));
+#pragma unroll
+    for (int j = 0; j < W; j++) r[k + j] = T(v[j]);
+  }
+}
+
 // u (+ injection of the coarser level's uc) at interior cell (x, y) of patch q
 template <typename T, typename TC, bool INTERP>
 struct UAcc {

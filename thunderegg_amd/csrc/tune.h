@@ -10,7 +10,7 @@ namespace te {
 
 enum TuneFamily {
   TUNE_DFT_GENERIC = 0,  // DFT patch solve, VALU kernel (any n): patches per workgroup x threads per patch
-  TUNE_DFT_MFMA_2D = 1,  // DFT patch solve, 2D matrix-core kernel (n 16, 32): workgroups of the launch
+  TUNE_DFT_MFMA_2D = 1,  // DFT patch solve, 2D matrix-core kernel (n 16): workgroups of the launch (n 32: one shape)
   TUNE_C3_SWEEP = 2,     // 3D 16^3 fused sweeps (modes 1, 2): slices per load batch
   TUNE_FAMILIES
 };
@@ -31,10 +31,10 @@ DftGenericVariant dft_generic_variant(int v);
 
 // 2D matrix-core DFT launches: the workgroup count policy of variant v (dft_mfma.hip)
 enum DftMfmaGrid {
-  MFMA_GRID_DEFAULT = 0,    // n 16: one round of the plain kernel when every workgroup is resident at
-                            // once, else the prefetching kernel on the resident count; n 32: <= 4096
-  MFMA_GRID_RESIDENT = 1,   // the prefetching kernel (n 16) on the resident workgroup count / <= 2048 (n 32)
-  MFMA_GRID_HALF = 2,       // half the resident count (n 16) / <= 8192 (n 32)
+  MFMA_GRID_DEFAULT = 0,    // one round of the plain kernel when every workgroup is resident at once,
+                            // else the prefetching kernel on the resident count
+  MFMA_GRID_RESIDENT = 1,   // the prefetching kernel on the resident workgroup count
+  MFMA_GRID_HALF = 2,       // half the resident count
   MFMA_GRID_ALL = 3,        // one workgroup per 4 patches, plain kernel
   MFMA_GRID_VARIANTS
 };
