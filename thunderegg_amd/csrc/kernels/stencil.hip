@@ -5,8 +5,6 @@
 // of the output are written 0 (f.setWithGhost(0), PatchOperator.h:136), interior cells get
 // the stencil.  Physical-boundary ghosts of u are applied inline
 // (enforceBoundaryConditions, :115-144): -u (Dirichlet) or +u (Neumann).
-#include <algorithm>
-
 #include "../te_internal.h"
 #include "ghost2d.h"
 #include "ghost3d.h"
@@ -32,7 +30,7 @@ constexpr int kNoFill = -1;
 constexpr int kStarItems = 2;
 
 template <typename T, typename TF, typename TO, int D, int OP, int FILL, int V>
-__global__ void __launch_bounds__(256) star_kernel(const DevPatch* __restrict__ dp, const int4* __restrict__ ring, T* u,
+__global__ void __launch_bounds__(D == 2 ? 256 : 1024) star_kernel(const DevPatch* __restrict__ dp, const int4* __restrict__ ring, T* u,
                                                    const T* __restrict__ cf, const TF* __restrict__ fin,
                                                    TO* __restrict__ out, Layout L, int neumann, FastDiv per_row,
                                                    FastDiv rows)
@@ -165,8 +163,7 @@ void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* 
                      (uintptr_t)out % (2 * sizeof(TO)) == 0;
   const int V = pairs ? 2 : 1, per = (L.n[0] + 2) / V;
   const int items = per * (L.n[1] + 2) * (D == 3 ? L.n[2] + 2 : 1);
-  // 3D: kStarItems groups or more a thread, up to 256 threads
-  const int block = D == 2 ? 256 : std::min(256, (items / kStarItems + 63) / 64 * 64);
+  const int block = D == 2 ? 256 : patch_block(items / kStarItems, d->np);
   const int grid = xcd_grid(D == 2 ? (d->np + 3) / 4 : d->np);
 #define TE_ST(F_, V_)                                                                                               \
   hipLaunchKernelGGL((star_kernel<T, TF, TO, D, OP, F_, V_>), dim3(grid), dim3(block), 0, s, d->d_patches,          \

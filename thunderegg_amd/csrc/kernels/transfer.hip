@@ -11,9 +11,8 @@
 //  - DirectInterpolator (GMG/DirectInterpolator.h:60-91): fine[i] += coarse[(i+s)/2].
 // Children of a coarse patch are visited in increasing fine local index and fine
 // cells in x-fastest order, the order in which the reference accumulates them.
-#include <algorithm>
-
 #include "../te_internal.h"
+#include "ghost2d.h"
 
 namespace te {
 namespace {
@@ -185,30 +184,29 @@ __device__ __forceinline__ void store_at(T* q, Get get)
 // forms the two coarse cells of an aligned pair, each from 2^(D - 1) accesses of two fine cells,
 // in the order of the general kernel above.
 template <typename TI, typename TO, int D>
-__global__ void __launch_bounds__(256) restrict_regular_kernel(const int32_t* __restrict__ child,
-                                                               const int32_t* __restrict__ nchild,
+__global__ void __launch_bounds__(D == 2 ? 256 : 1024) restrict_regular_kernel(const int32_t* __restrict__ child,
                                                                const int32_t* __restrict__ orth,
                                                                const TI* __restrict__ fine, TO* __restrict__ coarse,
                                                                Layout L, int np_coarse, FastDiv per_row, FastDiv rows)
 {
   constexpr bool WAVE = D == 2;
-  __shared__ int tabs[4][8];  // child of each octant of the patch(es), -1: none
+  __shared__ int tabs[4][8], copies[4];  // the child of each octant (-1: none), or a copied child in entry 0
   const int b = xcd_item(blockIdx.x, gridDim.x);
   const int w = WAVE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int p = WAVE ? b * 4 + w : b;
   const bool live = p < np_coarse;
   const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
-  const int nc = live ? nchild[p] : 0;
-  const bool copy = nc == 1 && orth[child[p * 8]] < 0;
+  // the link's records of the patch by one lane each (entries past the last child are -1)
   if (t < 8) {
-    int f = -1;
-    for (int k = 0; k < nc; k++) {
-      const int q = child[p * 8 + k];
-      if (copy || orth[q] == t) f = q;
-    }
-    tabs[w][t] = f;
+    const int f = live ? child[p * 8 + t] : -1, o = f >= 0 ? orth[f] : -1;
+    if (f >= 0 && o < 0) copies[w] = 1;  // the only child then (t = 0)
+    else if (t == 0) copies[w] = 0;
+    tabs[w][t] = -1;
+    wave_sync();
+    if (f >= 0) tabs[w][o < 0 ? 0 : o] = f;
   }
   __syncthreads();
+  const bool copy = copies[w] != 0;
   if (!live) return;
   const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1, h0 = n0 / 2, h1 = n1 / 2, h2 = n2 / 2;
   const int per = (n0 + 2) / 2, items = per * (n1 + 2) * (D == 3 ? n2 + 2 : 1);
@@ -225,7 +223,7 @@ __global__ void __launch_bounds__(256) restrict_regular_kernel(const int32_t* __
       for (int j = 0; j < 2; j++) {
         const int X = X0 + j;
         const int o = (X >= h0 ? 1 : 0) | (Y >= h1 ? 2 : 0) | (D == 3 && Z >= h2 ? 4 : 0);
-        const int f = tabs[w][o];
+        const int f = tabs[w][copy ? 0 : o];
         has[j] = in && X >= 0 && X < n0 && f >= 0;
         if (!has[j]) continue;
         if (copy) {
@@ -259,7 +257,7 @@ __global__ void __launch_bounds__(256) restrict_regular_kernel(const int32_t* __
 
 // DirectInterpolator: fine += the coarse cell over it, over the interior rows of each fine patch
 template <typename TC, typename TF, int D, int V>
-__global__ void __launch_bounds__(256) interp_kernel(const int32_t* __restrict__ parent,
+__global__ void __launch_bounds__(D == 2 ? 256 : 1024) interp_kernel(const int32_t* __restrict__ parent,
                                                      const int32_t* __restrict__ orth, const TC* __restrict__ coarse,
                                                      TF* __restrict__ fine, Layout L, FastDiv per_row, FastDiv rows)
 {
@@ -322,11 +320,11 @@ void restrict_t(const te_level_link* l, const TI* fine, TO* coarse, int ncomp, b
     const int items = per * rows * (c->dim == 3 ? L.n[2] + 2 : 1);
     if (c->dim == 2)
       hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 2>), dim3(xcd_grid((c->np + 3) / 4)), dim3(256), 0, s,
-                         l->d_child, l->d_nchild, l->d_orth, fine, coarse, L, c->np, FastDiv(per), FastDiv(rows));
+                         l->d_child, l->d_orth, fine, coarse, L, c->np, FastDiv(per), FastDiv(rows));
     else
       hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 3>), dim3(xcd_grid(c->np)),
-                         dim3(std::min(256, (items + 63) / 64 * 64)), 0, s, l->d_child, l->d_nchild, l->d_orth, fine,
-                         coarse, L, c->np, FastDiv(per), FastDiv(rows));
+                         dim3(patch_block(items, c->np)), 0, s, l->d_child, l->d_orth, fine, coarse, L, c->np,
+                         FastDiv(per), FastDiv(rows));
     return;
   }
   const int B = 256;
@@ -353,7 +351,7 @@ void interp_t(const te_level_link* l, const TC* coarse, TF* fine, int ncomp, hip
   const int V = L.n[0] % 2 == 0 ? 2 : 1, per = V == 2 ? L.n[0] / 2 + 1 : L.n[0];
   const int items = per * L.n[1] * (f->dim == 3 ? L.n[2] : 1);
   const int grid = xcd_grid(f->dim == 2 ? (f->np + 3) / 4 : f->np);
-  const int block = f->dim == 2 ? 256 : std::min(256, (items + 63) / 64 * 64);
+  const int block = f->dim == 2 ? 256 : patch_block(items, f->np);
 #define TE_IP(D_, V_)                                                                                              \
   hipLaunchKernelGGL((interp_kernel<TC, TF, D_, V_>), dim3(grid), dim3(block), 0, s, l->d_parent, l->d_orth, coarse, \
                      fine, L, FastDiv(per), FastDiv(L.n[1]))

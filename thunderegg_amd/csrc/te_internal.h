@@ -102,6 +102,13 @@ struct FastDiv {
 // dealt round-robin over the 8) takes the x-th contiguous eighth of n items: patches are in
 // Morton order, so most neighbours are then read through the same L2.  n or more: no item.
 __host__ __device__ inline int xcd_grid(int n) { return (n + 7) / 8 * 8; }
+// Threads of a workgroup that works on one patch: up to 256, or up to 1024 on levels with no more
+// patches than CUs, whose launch lasts as long as one patch's chain of loads and stores.
+inline int patch_block(int items, int np)
+{
+  const int cap = np <= 256 ? 1024 : 256, want = (items + 63) / 64 * 64;
+  return want < cap ? want : cap;
+}
 __device__ __forceinline__ int xcd_item(int b, int grid) { return (b & 7) * (grid >> 3) + (b >> 3); }
 
 // The interior cells of a padded vector as items of V consecutive padded values: row after row
