@@ -527,3 +527,35 @@ def test_cycles_and_solves_on_several_streams(ns, level, pre):
         assert np.array_equal(mesh.interior(x.get(), dim), mesh.interior(solved, dim))
         for u, want in zip(us, alone):
             assert np.array_equal(mesh.interior(u.get(), dim), mesh.interior(want, dim))
+
+
+@pytest.mark.parametrize("name,n", [("3d_mid_refine_4x4x4_mpi1.json", 8), ("3d_refined_bnw_2x2x2_mpi1.json", 16),
+                                    ("3d_uniform_2x2x2_mpi1.json", 8)])
+@pytest.mark.parametrize("op_kind,neumann", [(0, False), (0, True), (1, False)])
+@pytest.mark.parametrize("sweeps", [(1, 1, 1), (2, 2, 1), (0, 1, 2), (2, 0, 0)])
+def test_vcycle3d_refined_fused(name, n, op_kind, neumann, sweeps, monkeypatch):
+    """The 3D cycle whose sweeps and residual-restrictions form their own ghosts (8^3 and 16^3
+    patches, copied and refined children) against the one launch per step cycle, whose
+    arithmetic it repeats: same sums in the same order, so to the last bits that a compiler's
+    contraction of a product and a sum can change; and against the oracle."""
+    ns = (n,) * 3
+    dim, levels = load(name, ns)
+    coeffs = None
+    if op_kind:
+        coeffs = [np.exp(np.sin(3 * X[..., 0]) * np.cos(2 * X[..., 1]))[:, None].copy()
+                  for X in (mesh.cell_centers(lv, dim, ns) for lv in levels)]
+    pre, post, coarse = sweeps
+    f = random_field(mesh.padded_shape(len(levels[0]), dim, ns), 17)
+    for prec, tol in ((R.F64, 1e-12), (R.F32, 2e-5)):
+        o = dict(filler_kind=R.TRILINEAR, precision=prec, op_kind=op_kind, coeffs=coeffs, neumann=neumann,
+                 neumann_mask=0b111111 if neumann else 0, pre_sweeps=pre, post_sweeps=post, coarse_sweeps=coarse)
+        fused = solver.GMG(dim, ns, levels, **o)
+        got = mesh.interior(fused.vcycle(f), dim)
+        assert np.array_equal(mesh.interior(fused.vcycle(f), dim), got)
+        monkeypatch.setenv("TE_NO_FUSE", "1")
+        steps = mesh.interior(solver.GMG(dim, ns, levels, **o).vcycle(f), dim)
+        monkeypatch.delenv("TE_NO_FUSE")
+        assert relerr(got, steps) <= tol
+        if op_kind == 0 and not neumann:
+            ol = O.Levels([O.Domain(dim, ns, lv) for lv in levels], filler_kind=R.TRILINEAR, smoother_kind=0)
+            assert relerr(got, mesh.interior(ol.vcycle(f.copy(), pre=pre, post=post, coarse=coarse), dim)) <= tol

@@ -260,6 +260,54 @@ int visit_fused(te_gmg* g, int li, const void* f, int dtf, void* u_ext, int ext_
   return TE_OK;
 }
 
+// VCycle::visit on 3D hierarchies of 8^3 or 16^3 patches with coarse / fine faces, padded
+// vectors: per level one launch per smoothing sweep (its ghosts formed in it), one for
+// Cycle::restrict and one for the interpolation.  Sweeps after the first read the solution from
+// one buffer and write the other; the finest level's last sweep writes the caller's u_ext (FP64).
+int visit_fused3(te_gmg* g, int li, const void* f, int dtf, double* u_ext)
+{
+  GLevel& Lv = g->L[li];
+  const int nl = (int)g->L.size();
+  const bool finest = li == 0;
+  void* buf[2] = { Lv.u, Lv.u2 };
+  int cur = 0;
+  auto sweep = [&](bool uzero, bool last_of_level) -> int {
+    const bool to_ext = finest && last_of_level;
+    void* out = to_ext ? (void*)u_ext : buf[cur ^ 1];
+    TE_RC(sweep_timing(g, li, false));
+    TE_RC(launch_dft(Lv.plan, Lv.dt, dtf, to_ext ? (int)TE_F64 : Lv.dt, f, buf[cur], out, uzero, g->s, false, true));
+    TE_RC(sweep_timing(g, li, true));
+    if (!to_ext) cur ^= 1;
+    Lv.cur = out;
+    return TE_OK;
+  };
+  auto no_sweep = [&]() -> int {  // the solution as it stands becomes the level's
+    Lv.cur = buf[cur];
+    if (!finest) return TE_OK;
+    Lv.cur = u_ext;
+    return launch_convert(te_domain_vector_length(Lv.d, 1), TE_F64, u_ext, Lv.dt, buf[cur], g->s);
+  };
+  if (li == nl - 1) {
+    const int n = g->o.coarse_sweeps;
+    if (n == 0) {
+      TE_RC(zero_with_ghost(g, li, buf[0], Lv.dt));
+      return no_sweep();
+    }
+    for (int k = 0; k < n; k++) TE_RC(sweep(k == 0, k == n - 1));
+    return TE_OK;
+  }
+  for (int k = 0; k < g->o.pre_sweeps; k++) TE_RC(sweep(k == 0, false));
+  if (g->o.pre_sweeps == 0) TE_RC(zero_with_ghost(g, li, buf[0], Lv.dt));
+  GLevel& Cv = g->L[li + 1];
+  TE_RC(launch_resid_restrict3(Lv.gf, Lv.link, g->o.op_kind, g->o.neumann, Lv.coeffs, Lv.dt, dtf, f, buf[cur], Cv.dt,
+                               Cv.f, g->s));
+  TE_RC(visit_fused3(g, li + 1, Cv.f, Cv.dt, u_ext));
+  TE_RC(launch_interpolate(Lv.link, Cv.dt, Cv.cur, Lv.dt, buf[cur], 1, g->s));
+  const int n = g->o.post_sweeps;
+  for (int k = 0; k < n; k++) TE_RC(sweep(false, k == n - 1));
+  return n == 0 ? no_sweep() : TE_OK;
+}
+
 // the face columns of compact buffer v (np patches, type dt), or nullptr when the solver
 // does not keep them
 static void* xcol_of(const te_gmg* g, const void* v, long np, int dt)
@@ -400,6 +448,7 @@ int vcycle_enqueue_one(te_gmg* g, const void* f, void* u, int udt, int dtf, bool
     return TE_ERR_UNSUPPORTED;
   }
   double* ud = (double*)u;
+  if (g->fused3) return visit_fused3(g, 0, f, TE_F64, ud);
   if (L0.dt != TE_F64 && L0.smoother != 0) {
     // the inner-Krylov smoother works on same-dtype f and u: convert f once
     TE_RC(launch_convert(te_domain_vector_length(L0.d, 1), L0.dt, L0.f, TE_F64, f, g->s));
@@ -431,7 +480,7 @@ int vcycle_launches(const te_gmg* g)
   if (g->o.cycle_type != TE_CYCLE_V) return kDirectLaunches + 1;
   const int sweeps = g->o.pre_sweeps + g->o.post_sweeps;
   const int levels = g->fused && g->tail_from >= 0 ? g->tail_from : (int)g->L.size() - 1;
-  return levels * (g->fused || g->c3 ? sweeps + 1 : 2 * sweeps + 3) + 1 + (g->c3 ? 2 : 0);
+  return levels * (g->fused || g->c3 ? sweeps + 1 : g->fused3 ? sweeps + 2 : 2 * sweeps + 2) + 1 + (g->c3 ? 2 : 0);
 }
 
 int vcycle_launch(te_gmg* g, const double* f, double* u, hipStream_t s)
@@ -744,6 +793,14 @@ int te::gmg_create(const te_domain* const* levels, int num_levels, const te_gmg_
               (i == num_levels - 1 || resid_restrict_fused_supported(Lv.gf));
     }
     g->fused = fused;
+    // the 3D hierarchies the compact path does not take
+    bool fused3 = allow && !batch && !g->c3 && opts->cycle_type == TE_CYCLE_V;
+    for (int i = 0; i < num_levels && fused3; i++) {
+      const GLevel& Lv = g->L[i];
+      fused3 = Lv.smoother == 0 && Lv.plan && dft3_mfma_supported(Lv.plan) &&
+               (i == num_levels - 1 || resid_restrict3_supported(Lv.gf, Lv.link));
+    }
+    g->fused3 = fused3;
     g->fly = allow && star_dot_fly_supported(g->L[0].gf);
     g->m32 = g->fused && g->fly && g->L[0].dt == TE_F32;
     const char* nr = std::getenv("TE_NO_RRPRE");

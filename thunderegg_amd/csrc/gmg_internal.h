@@ -88,6 +88,8 @@ struct te_gmg {
   te::GraphCache vgraphs, bgraphs;
   double last_seconds = 0.0;
   bool fused = false;  // 2D matrix-core path: ghost fills fused into the stencil / smoother launches
+  // 3D patches of 8^3 or 16^3 (refined meshes): sweeps and residual-restrictions form the ghosts they need
+  bool fused3 = false;
   std::vector<char> rr_pre;  // per level: restriction fused with the coarser level's first sweep
   bool fly = false;    // outer operator computes ghosts on the fly
   // mixed precision on the fused path: M p and M s are FP32 values (the finest level's last

@@ -23,9 +23,11 @@ struct te_dft_plan {
 };
 
 namespace te {
-// zero_ghosts: out's ghost cells are set to 0 as well (out may not be f then)
+// zero_ghosts: out's ghost cells are set to 0 as well (out may not be f then).  fill (3D matrix-core
+// plans): u's ghosts are formed in the launch and not read from u, which may not be out.
+bool dft3_mfma_supported(const te_dft_plan* pl);
 int launch_dft(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, const void* u, void* out, bool uzero,
-               hipStream_t s, bool zero_ghosts = false);
+               hipStream_t s, bool zero_ghosts = false, bool fill = false);
 bool dft_mfma_supported(const te_dft_plan* pl);
 int launch_dft_mfma(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, const void* u, void* out,
                     bool uzero, hipStream_t s);
@@ -43,6 +45,12 @@ bool resid_restrict_fused_supported(const te_ghost_filler* g);
 int launch_resid_restrict(const te_ghost_filler* g, const te_level_link* link, int op_kind, int neumann,
                           const void* coeffs, int dt, int dtf, const void* f, const void* u, int dtc, void* fc,
                           hipStream_t s);
+// Cycle::restrict in 3D (kernels/stencil.hip): fc = restriction of f - A u with u's ghosts formed in
+// the launch; 8^3 or 16^3 patches, a regular link.  fc's ghost cells are not written.
+bool resid_restrict3_supported(const te_ghost_filler* g, const te_level_link* link);
+int launch_resid_restrict3(const te_ghost_filler* g, const te_level_link* link, int op_kind, int neumann,
+                           const void* coeffs, int dt, int dtf, const void* f, const void* u, int dtc, void* fc,
+                           hipStream_t s);
 // Cycle::restrict of the level of g fused with the zero-guess sweep of the next coarser
 // level (plan pc): writes the coarse f (fc) and the coarse u (uc); 2D, 16x16 patches.
 bool rr_pre_supported(const te_ghost_filler* g, const te_dft_plan* pc);

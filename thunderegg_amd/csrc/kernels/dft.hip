@@ -14,6 +14,7 @@
 #include "blas.h"
 #include "dft_wave.h"
 #include "ghost2d.h"
+#include "ghost3d.h"
 #include "../tune.h"
 
 namespace te {
@@ -169,9 +170,12 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
 // Latency-bound on small levels (one patch a CU): 8 patches in FP32 take 6.4 us where one LDS
 // round trip per axis (six, with barriers between) took 20.6; on large ones bound by memory:
 // 2,535 patches 43 us (the vectors' padded lines in 36 at a copy's rate) against 95.
+// FILL: the ghosts of u's faces are formed here (face_ghost3, one of the 256 cells of each face
+// a thread, into LDS) instead of read from u; out may not be u then, since other patches' ghosts
+// are formed from it.  A cycle's sweep with its ghosts on 2,535 patches: 53 us against 28 + 43 apart.
 constexpr int k3N = 16, k3Row = 20, k3Slice = 16 * k3Row + 4, k3Slab = 16 * k3Slice;
 
-template <typename T, typename TF, typename TO, int OP, bool UZERO>
+template <typename T, typename TF, typename TO, int OP, bool UZERO, bool FILL>
 __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
                                                         const T* __restrict__ mats, const T* __restrict__ s2tab,
                                                         const TF* __restrict__ f, const T* u,
@@ -179,9 +183,11 @@ __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restri
                                                         bool zero_ghosts)
 {
   __shared__ __align__(16) T slab[k3Slab];
+  __shared__ T ghost[FILL ? 6 : 1][FILL ? k3N * k3N : 1];
   typedef typename Mf<T>::V V;
   constexpr int SB = sizeof(T) == 4 ? 2 : 1;
-  const int p = blockIdx.x;
+  const int p = FILL ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x;
+  if (p >= L.np) return;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int* pt = ptype + p * 8;  // fwd type per axis [0..2], eig type per axis [3..5], zero mode [6]
   const DevPatch& P = dp[p];
@@ -189,6 +195,15 @@ __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restri
   T F[4][4];
 #pragma unroll
   for (int i = 0; i < 4; i++) load_row4(f, row0 + (w + 4 * i + 1) * L.sy, F[i]);
+  if (FILL) {
+    const int i = threadIdx.x & 15, j = threadIdx.x >> 4;
+    T G[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+      G[s] = P.type[20 + s] < 0 ? T(0) : face_ghost3<T>(L, P.type[20 + s], P.orth[20 + s], P.nbr[20 + s], u, p, 0, s, i, j);
+#pragma unroll
+    for (int s = 0; s < 6; s++) ghost[FILL ? s : 0][FILL ? threadIdx.x : 0] = G[s];
+  }
   // the transform matrices M[i][j] (y_i = sum_j M[i][j] x_j) as MFMA operands: lane (c, g), step
   // s holds M[c][K], K the product's K order (4g + s from memory, Mf<T>::row from an accumulator)
   auto mat = [&](int t, int a, int i, int j) { return mats[(t * 3 + a) * kDftMatStride + i * k3N + j]; };
@@ -225,25 +240,35 @@ __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restri
   struct Face {
     T xb, xg, b[4], y[4], z[4];
   };
-  auto faces = [&](const T* v, int base, int z, Face& q) {
-    const int r = base + (z + 1) * L.sy;
-    const bool onz = (z == 0 && has[4]) || (z == k3N - 1 && has[5]);
+  // (own: u's, whose ghosts are in LDS with FILL)
+  auto faces = [&](const T* v, int z, bool own, Face& q) {
+    const int r = row0 + (z + 1) * L.sy;
+    const bool onz = (z == 0 && has[4]) || (z == k3N - 1 && has[5]), lds = FILL && own;
     if (onx) {
       q.xb = at(v, g == 0 ? r : r + 3);
-      q.xg = at(v, g == 0 ? r - 1 : r + 4);
+      q.xg = lds ? ghost[g == 0 ? 0 : (FILL ? 1 : 0)][FILL ? c + 16 * z : 0] : at(v, g == 0 ? r - 1 : r + 4);
     }
     if (ony || onz) load_row4(v, r, q.b);
-    if (ony) load_row4(v, c == 0 ? r - L.sx : r + L.sx, q.y);
-    if (onz) load_row4(v, z == 0 ? r - L.sy : r + L.sy, q.z);
+    if (lds) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (ony) q.y[k] = ghost[FILL ? (c == 0 ? 2 : 3) : 0][FILL ? 4 * g + k + 16 * z : 0];
+        if (onz) q.z[k] = ghost[FILL ? (z == 0 ? 4 : 5) : 0][FILL ? 4 * g + k + 16 * c : 0];
+      }
+    } else {
+      if (ony) load_row4(v, c == 0 ? r - L.sx : r + L.sx, q.y);
+      if (onz) load_row4(v, z == 0 ? r - L.sy : r + L.sy, q.z);
+    }
   };
+  if (FILL) __syncthreads();
 #pragma unroll
   for (int i0 = 0; i0 < 4; i0 += SB) {
     Face q[SB], cq[OP == 1 ? SB : 1];
     if (!UZERO) {
 #pragma unroll
       for (int j = 0; j < SB; j++) {
-        faces(u, row0, w + 4 * (i0 + j), q[j]);
-        if (OP == 1) faces(coeffs, row0, w + 4 * (i0 + j), cq[OP == 1 ? j : 0]);
+        faces(u, w + 4 * (i0 + j), true, q[j]);
+        if (OP == 1) faces(coeffs, w + 4 * (i0 + j), false, cq[OP == 1 ? j : 0]);
       }
     }
 #pragma unroll
@@ -333,19 +358,24 @@ __global__ void __launch_bounds__(256) dft3_mfma_kernel(const DevPatch* __restri
 // Plane q = (column half) + 2 (row half) of tile t is slice (or row) 4t + q.
 // Latency of loads and LDS; 4,096 patches in FP32: 11.1 us from zero and 12.6 with interface
 // terms, where one 128-thread group per patch with dense products in VALU took 40 and 47.
+// FILL: as in dft3_mfma_kernel, one of the 64 cells of each face a lane.
 constexpr int k3Pitch8 = 72, k3Slab8 = 8 * k3Pitch8;  // words of a slice, of the patch
 
-template <typename T, typename TF, typename TO, int OP, bool UZERO>
+template <typename T, typename TF, typename TO, int OP, bool UZERO, bool FILL>
 __global__ void __launch_bounds__(256) dft3_tile8_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
                                                          const T* __restrict__ mats, const T* __restrict__ s2tab,
                                                          const TF* __restrict__ f, const T* u,
-                                                         const T* __restrict__ coeffs, TO* out, int np, bool zero_ghosts)
+                                                         const T* __restrict__ coeffs, TO* out, Layout L,
+                                                         bool zero_ghosts)
 {
   constexpr int SX = 10, SY = 100, PS = 1000;
   __shared__ T slabs[4 * k3Slab8];
+  __shared__ T ghosts[FILL ? 4 * 6 * 64 : 1];
   typedef typename Mf<T>::V V;
-  const int p = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (p >= np) return;
+  const int p = __builtin_amdgcn_readfirstlane((FILL ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x) * 4 +
+                                               (threadIdx.x >> 6));
+  if (p >= L.np) return;
+  T* ghost = ghosts + (FILL ? (threadIdx.x >> 6) * 6 * 64 : 0);
   T* slab = slabs + (threadIdx.x >> 6) * k3Slab8;
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int* pt = ptype + p * 8;  // fwd type per axis [0..2], eig type per axis [3..5], zero mode [6]
@@ -362,6 +392,17 @@ __global__ void __launch_bounds__(256) dft3_tile8_kernel(const DevPatch* __restr
   for (int a = 0; a < 3; a++) {
     tf[a] = pt[a];
     ti[a] = tf[a] == 0 ? 1 : (tf[a] == 3 ? 4 : tf[a]);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
+  }
+  if (FILL) {
+    T G[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+      G[s] = P.type[20 + s] < 0
+               ? T(0)
+               : face_ghost3<T>(L, P.type[20 + s], P.orth[20 + s], P.nbr[20 + s], u, p, 0, s, lane & 7, lane >> 3);
+#pragma unroll
+    for (int s = 0; s < 6; s++) ghost[FILL ? s * 64 + lane : 0] = G[s];
+    wave_sync();
   }
   // element (i, j) of the doubled matrix of axis a
   auto mat = [&](int t, int a, int i, int j) {
@@ -396,22 +437,30 @@ __global__ void __launch_bounds__(256) dft3_tile8_kernel(const DevPatch* __restr
     struct Face {
       T xb, xg, b[4], y[4], z[4];
     };
-    auto faces = [&](const T* v, int z, Face& q) {
+    auto faces = [&](const T* v, int z, bool own, Face& q) {
       const int r = row0 + (z + 1) * SY;
-      const bool onz = (z == 0 && has[4]) || (z == 7 && has[5]);
+      const bool onz = (z == 0 && has[4]) || (z == 7 && has[5]), lds = FILL && own;
       if (onx) {
         q.xb = at(v, r + xc);
-        q.xg = at(v, xlow ? r + 4 : r - 1);
+        q.xg = lds ? ghost[FILL ? (xlow ? 64 : 0) + y + 8 * z : 0] : at(v, xlow ? r + 4 : r - 1);
       }
       if (ony || onz) load_row4(v, r, q.b);
-      if (ony) load_row4(v, y == 0 ? r - SX : r + SX, q.y);
-      if (onz) load_row4(v, z == 0 ? r - SY : r + SY, q.z);
+      if (lds) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          if (ony) q.y[k] = ghost[FILL ? (y == 0 ? 2 : 3) * 64 + xlow + k + 8 * z : 0];
+          if (onz) q.z[k] = ghost[FILL ? (z == 0 ? 4 : 5) * 64 + xlow + k + 8 * y : 0];
+        }
+      } else {
+        if (ony) load_row4(v, y == 0 ? r - SX : r + SX, q.y);
+        if (onz) load_row4(v, z == 0 ? r - SY : r + SY, q.z);
+      }
     };
     Face q[2], cq[OP == 1 ? 2 : 1];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-      faces(u, 4 * t + qa, q[t]);
-      if (OP == 1) faces(coeffs, 4 * t + qa, cq[OP == 1 ? t : 0]);
+      faces(u, 4 * t + qa, true, q[t]);
+      if (OP == 1) faces(coeffs, 4 * t + qa, false, cq[OP == 1 ? t : 0]);
     }
 #pragma unroll
     for (int t = 0; t < 2; t++) {
@@ -499,7 +548,8 @@ __global__ void __launch_bounds__(256) dft3_tile8_kernel(const DevPatch* __restr
 }
 
 template <typename T, typename TF, typename TO, int D>
-void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, bool zg, hipStream_t s)
+void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzero, bool zg, bool fill,
+              hipStream_t s)
 {
   const te_domain* d = pl->g->d;
   Layout L = make_layout(d->dim, d->ns, 1, d->np);
@@ -513,28 +563,28 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
   const T* mats = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_mats64 : (const void*)pl->d_mats32);
   const T* s2 = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_s2_64 : (const void*)pl->d_s2_32);
   const T* cf = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_coeffs64 : (const void*)pl->d_coeffs32);
-  if (D == 3 && pl->use_mfma && d->ns[0] == 16 && d->ns[1] == 16 && d->ns[2] == 16) {
-#define TE_D3(OP_, UZ_)                                                                                         \
-  hipLaunchKernelGGL((dft3_mfma_kernel<T, TF, TO, OP_, UZ_>), dim3(d->np), dim3(256), 0, s, d->d_patches,     \
-                     pl->d_ptype, mats, s2, f, u, cf, out, L, zg)
-    if (pl->op_kind == 0) {
-      if (uzero) TE_D3(0, true); else TE_D3(0, false);
-    } else {
-      if (uzero) TE_D3(1, true); else TE_D3(1, false);
-    }
+  if (D == 3 && dft3_mfma_supported(pl)) {
+    const bool big = d->ns[0] == 16;
+    const int groups = big ? d->np : (d->np + 3) / 4, grid = fill && !uzero ? xcd_grid(groups) : groups;
+#define TE_D3(OP_, UZ_, F_)                                                                                         \
+  do {                                                                                                              \
+    if (big)                                                                                                        \
+      hipLaunchKernelGGL((dft3_mfma_kernel<T, TF, TO, OP_, UZ_, F_>), dim3(grid), dim3(256), 0, s, d->d_patches,    \
+                         pl->d_ptype, mats, s2, f, u, cf, out, L, zg);                                              \
+    else                                                                                                            \
+      hipLaunchKernelGGL((dft3_tile8_kernel<T, TF, TO, OP_, UZ_, F_>), dim3(grid), dim3(256), 0, s, d->d_patches,   \
+                         pl->d_ptype, mats, s2, f, u, cf, out, L, zg);                                              \
+  } while (0)
+#define TE_D3O(OP_)                        \
+  do {                                     \
+    if (uzero) TE_D3(OP_, true, false);    \
+    else if (fill) TE_D3(OP_, false, true); \
+    else TE_D3(OP_, false, false);         \
+  } while (0)
+    if (pl->op_kind == 0) TE_D3O(0);
+    else TE_D3O(1);
+#undef TE_D3O
 #undef TE_D3
-    return;
-  }
-  if (D == 3 && pl->use_mfma && d->ns[0] == 8 && d->ns[1] == 8 && d->ns[2] == 8) {
-#define TE_D8(OP_, UZ_)                                                                                         \
-  hipLaunchKernelGGL((dft3_tile8_kernel<T, TF, TO, OP_, UZ_>), dim3((d->np + 3) / 4), dim3(256), 0, s,          \
-                     d->d_patches, pl->d_ptype, mats, s2, f, u, cf, out, d->np, zg)
-    if (pl->op_kind == 0) {
-      if (uzero) TE_D8(0, true); else TE_D8(0, false);
-    } else {
-      if (uzero) TE_D8(1, true); else TE_D8(1, false);
-    }
-#undef TE_D8
     return;
   }
   // patches per workgroup and threads per patch: the autotuner's choice for this shape
@@ -554,10 +604,11 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
 }
 
 template <typename T, typename TF, typename TO>
-void launch_t(const te_dft_plan* pl, const void* f, const void* u, void* out, bool uzero, bool zg, hipStream_t s)
+void launch_t(const te_dft_plan* pl, const void* f, const void* u, void* out, bool uzero, bool zg,
+              bool fill, hipStream_t s)
 {
-  if (pl->g->d->dim == 2) launch_d<T, TF, TO, 2>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, zg, s);
-  else launch_d<T, TF, TO, 3>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, zg, s);
+  if (pl->g->d->dim == 2) launch_d<T, TF, TO, 2>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, zg, fill, s);
+  else launch_d<T, TF, TO, 3>(pl, (const TF*)f, (const T*)u, (TO*)out, uzero, zg, fill, s);
 }
 
 // the fused sweeps of the generic kernel, 2D: gm 0 (ghosts read from u), 1 (computed here),
@@ -657,24 +708,34 @@ int launch_dft_fused(const te_dft_plan* pl, int dt, int dtf, int dto, const void
   return TE_OK;
 }
 
+bool dft3_mfma_supported(const te_dft_plan* pl)
+{
+  const te_domain* d = pl->g->d;
+  return pl->use_mfma && d->dim == 3 && (d->ns[0] == 8 || d->ns[0] == 16) && d->ns[1] == d->ns[0] &&
+         d->ns[2] == d->ns[0];
+}
+
 int launch_dft(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, const void* u, void* out, bool uzero,
-               hipStream_t s, bool zero_ghosts)
+               hipStream_t s, bool zero_ghosts, bool fill)
 {
   const te_domain* d = pl->g->d;
   if (d->np == 0) return TE_OK;
   // the 3D matrix-core kernels zero the ghosts themselves, where the patches start on 16 bytes
-  const bool own = pl->use_mfma && d->dim == 3 && (d->ns[0] == 8 || d->ns[0] == 16) && d->ns[1] == d->ns[0] &&
-                   d->ns[2] == d->ns[0] && uzero && f != out && (uintptr_t)out % 16 == 0;
+  const bool own = dft3_mfma_supported(pl) && uzero && f != out && (uintptr_t)out % 16 == 0;
+  if (fill && !uzero && (!dft3_mfma_supported(pl) || out == u)) {
+    set_error("internal: a 3D sweep that forms ghosts needs 8^3 or 16^3 patches and another buffer for its result");
+    return TE_ERR_ARG;
+  }
   const bool zg = zero_ghosts && own;
   if (zero_ghosts && !own) {
     int rc = launch_vec_op(d, dto, VOP_SET_WITH_GHOST, out, nullptr, nullptr, 0.0, 0, 0, 1, s);
     if (rc) return rc;
   }
   if (pl->use_mfma && dft_mfma_supported(pl)) return launch_dft_mfma(pl, dt, dtf, dto, f, u, out, uzero, s);
-  if (dt == TE_F64 && dtf == TE_F64 && dto == TE_F64) launch_t<double, double, double>(pl, f, u, out, uzero, zg, s);
-  else if (dt == TE_F32 && dtf == TE_F32 && dto == TE_F32) launch_t<float, float, float>(pl, f, u, out, uzero, zg, s);
-  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F32) launch_t<float, double, float>(pl, f, u, out, uzero, zg, s);
-  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F64) launch_t<float, double, double>(pl, f, u, out, uzero, zg, s);
+  if (dt == TE_F64 && dtf == TE_F64 && dto == TE_F64) launch_t<double, double, double>(pl, f, u, out, uzero, zg, fill, s);
+  else if (dt == TE_F32 && dtf == TE_F32 && dto == TE_F32) launch_t<float, float, float>(pl, f, u, out, uzero, zg, fill, s);
+  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F32) launch_t<float, double, float>(pl, f, u, out, uzero, zg, fill, s);
+  else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F64) launch_t<float, double, double>(pl, f, u, out, uzero, zg, fill, s);
   else {
     set_error("unsupported dtype combination for the DFT patch solver");
     return TE_ERR_UNSUPPORTED;
