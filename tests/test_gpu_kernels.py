@@ -640,3 +640,24 @@ def test_dft32_pair(level, op_kind, kind):
             du = R.DeviceArray.from_host(u0)
             (plan.apply if zero else plan.smooth)(R.DeviceArray.from_host(f0), du)
             assert relerr(mesh.interior(du.get(), 2), mesh.interior(uref, 2)) <= tol, (dtype, zero)
+
+
+@pytest.mark.parametrize("ns", [(4, 8), (8, 8), (10, 6), (20, 24), (32, 32), (40, 12)])
+@pytest.mark.parametrize("kind", [R.BILINEAR, R.BIQUADRATIC])
+@pytest.mark.parametrize("neumann", [False, True])
+def test_residual_restrict_sizes(ns, kind, neumann):
+    """Residual and restriction in one launch over the even sizes (a workgroup of 64 to 256
+    threads a patch) against the oracle's operator and restriction."""
+    lv = load("2d_uniform_8x8_refined_cross_mpi1.json", ns)[1][:2]
+    of, oc = (O.Domain(2, ns, v) for v in lv)
+    of.link_parents(oc)
+    df, dc = (R.Domain(2, ns, v) for v in lv)
+    link, g = R.LevelLink(df, dc), R.GhostFiller(df, kind, R.FACES)
+    for dtype, tol in [(R.F64, TOL64), (R.F32, TOL32)]:
+        t = R.np_dtype(dtype)
+        f0, u0 = random_field(of.shape(1), 51, t), random_field(of.shape(1), 52, t)
+        au = O.poisson_apply(of, u0.astype(np.float64), kind=kind, neumann=neumann)
+        want = O.restrict(of, oc, f0.astype(np.float64) - au)
+        fc = R.DeviceArray.from_host(np.zeros(oc.shape(1), t))
+        link.residual_restrict(g, R.DeviceArray.from_host(f0), R.DeviceArray.from_host(u0), fc, neumann=neumann)
+        assert relerr(mesh.interior(fc.get(), 2), mesh.interior(want, 2)) <= tol, dtype

@@ -6,7 +6,7 @@
 //   sweep      DFTPatchSolver::smooth (the interface terms of the ghosts computed from
 //              the neighbours' values, as dft_mfma_kernel does with ghosts on the fly;
 //              the first sweep of a level from u = 0 solves f alone);
-//   residual   r = f - A u with the ghost formulas of resid_restrict_2d, restricted into
+//   residual   r = f - A u with the ghost formulas of resid_restrict_16, restricted into
 //              the next level's f (LinearRestrictor, GMG/LinearRestrictor.h:101-191);
 //   interpolate u += P uc (DirectInterpolator, GMG/DirectInterpolator.h:60-91) into the
 //              level's other buffer, which the first post-smoothing sweep then reads
