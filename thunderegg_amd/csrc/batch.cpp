@@ -278,27 +278,29 @@ int build_group(Group& G, const std::vector<const te_domain* const*>& lv, const 
   return TE_OK;
 }
 
-// wait until the group's publish with sequence number G.seq has reached the host
-int wait_published(Group& G)
+// whether the group's publish with sequence number G.seq has reached the host (G.running is
+// then up to date); every 256th call (*spin counts them) also asks the stream, so that a failed
+// launch ends the wait
+int poll_published(Group& G, unsigned* spin, bool* done)
 {
   volatile double* m = G.mirror_h;
-  for (unsigned spin = 1;; spin++) {
-    if (m[0] == G.seq) break;
-    if ((spin & 255) == 0) {
-      hipError_t q = hipStreamQuery(G.s);
-      if (q == hipSuccess && m[0] == G.seq) break;
-      if (q == hipSuccess) {
-        set_error("batched BiCGStab: an iteration finished without publishing its state");
-        return TE_ERR_HIP;
-      }
-      if (q != hipErrorNotReady) {
-        set_error(std::string("batched BiCGStab iteration: ") + hipGetErrorString(q));
-        return TE_ERR_HIP;
-      }
+  *done = m[0] == G.seq;
+  if (!*done && (++*spin & 255) == 0) {
+    hipError_t q = hipStreamQuery(G.s);
+    *done = q == hipSuccess && m[0] == G.seq;
+    if (q == hipSuccess && !*done) {
+      set_error("batched BiCGStab: an iteration finished without publishing its state");
+      return TE_ERR_HIP;
+    }
+    if (q != hipSuccess && q != hipErrorNotReady) {
+      set_error(std::string("batched BiCGStab iteration: ") + hipGetErrorString(q));
+      return TE_ERR_HIP;
     }
   }
-  std::atomic_thread_fence(std::memory_order_acquire);
-  G.running = m[1];
+  if (*done) {
+    std::atomic_thread_fence(std::memory_order_acquire);
+    G.running = m[1];
+  }
   return TE_OK;
 }
 
@@ -542,22 +544,36 @@ int te_batch_bicgstab(te_batch* B, const double* const* b, double* const* x, int
     TE_RC(launch_batch_publish(G.scal, ng, G.ctl, G.mirror_d, G.s));
     G.seq += 1.0;
   }
-  for (Group& G : B->grp) TE_RC(wait_published(G));
-  // every problem's loop ends within max_it iterations (ST_DONE at the limit)
-  for (int it = 0; it <= max_it; it++) {
-    bool any = false;
-    for (Group& G : B->grp) {
-      if (G.running == 0.0) continue;
-      hipGraphExec_t gx = nullptr;
-      if (B->o.use_graph) TE_RC(iteration_graph(G, use_precond, &gx));
-      if (gx) TE_HIP(hipGraphLaunch(gx, G.s));
-      else TE_RC(iteration(G, use_precond));
-      G.seq += 1.0;
-      any = true;
+  // A group's next iteration is launched as soon as its own scalars have arrived, whatever the
+  // other groups are doing: the group with the most work never waits for the host to start the
+  // others' graphs.  Every problem's loop ends within max_it iterations (ST_DONE at the limit).
+  struct Flight {
+    bool up = true;  // published scalars are on their way (first those of the setup)
+    int launched = 0;
+    unsigned spin = 0;
+  };
+  std::vector<Flight> fl(B->grp.size());
+  for (bool any = true; any;) {
+    any = false;
+    for (size_t gi = 0; gi < B->grp.size(); gi++) {
+      Group& G = B->grp[gi];
+      Flight& F = fl[gi];
+      if (F.up) {
+        bool done = false;
+        TE_RC(poll_published(G, &F.spin, &done));
+        F.up = !done;
+      }
+      if (!F.up && G.running != 0.0 && F.launched <= max_it) {
+        hipGraphExec_t gx = nullptr;
+        if (B->o.use_graph) TE_RC(iteration_graph(G, use_precond, &gx));
+        if (gx) TE_HIP(hipGraphLaunch(gx, G.s));
+        else TE_RC(iteration(G, use_precond));
+        G.seq += 1.0;
+        F.launched++;
+        F.up = true;
+      }
+      any = any || F.up;
     }
-    if (!any) break;
-    for (Group& G : B->grp)
-      if (G.running != 0.0) TE_RC(wait_published(G));
   }
   std::vector<std::vector<double>> sc(B->grp.size());
   for (size_t gi = 0; gi < B->grp.size(); gi++) {

@@ -25,8 +25,8 @@ void set_error(const std::string& msg) { g_err = msg; }
 namespace {
 
 // result slots, cut from page-locked slabs: allocating one per domain would cost more than the
-// domain's tables (a batch makes thousands of domains).  A slab is freed when its last slot
-// comes back.
+// domain's tables (a batch makes thousands of domains).  A slab is freed when its last slot comes
+// back, but for one (16 KiB) kept for the next domain.
 constexpr int kSlotBytes = 64, kSlabSlots = 256;
 struct Slab {
   char* base;
@@ -62,7 +62,9 @@ void give_result(double* r)
     const long off = (char*)r - sl.base;
     if (off < 0 || off >= kSlotBytes * kSlabSlots) continue;
     sl.free.push_back((int)(off / kSlotBytes));
-    if (sl.free.size() == kSlabSlots) {
+    int empty = 0;
+    for (const Slab& o : g_slabs) empty += o.free.size() == kSlabSlots;
+    if (empty > 1) {  // this one and another
       (void)hipHostFree(sl.base);
       g_slabs.erase(g_slabs.begin() + (long)i);
     }
