@@ -661,3 +661,43 @@ def test_residual_restrict_sizes(ns, kind, neumann):
         fc = R.DeviceArray.from_host(np.zeros(oc.shape(1), t))
         link.residual_restrict(g, R.DeviceArray.from_host(f0), R.DeviceArray.from_host(u0), fc, neumann=neumann)
         assert relerr(mesh.interior(fc.get(), 2), mesh.interior(want, 2)) <= tol, dtype
+
+
+@pytest.mark.parametrize("ns", [(7, 7), (5, 9), (8, 8), (10, 12), (24, 24), (40, 6), (50, 50), (6, 6, 6), (4, 6, 8), (12, 12, 12),
+                                (16, 14, 18)])
+@pytest.mark.parametrize("neumann_mask", [0, 0b0110])
+@pytest.mark.parametrize("op_kind", [0, 1])
+def test_dft_generic_sizes(ns, neumann_mask, op_kind):
+    """The generic patch solve over odd, even, mixed and large sizes (padded and unpadded LDS, one
+    matrix for all axes or one per axis and patch, several patches a workgroup): sweep and
+    apply with its zeroed ghosts, in place and on vectors one value off, against the oracle."""
+    dim = len(ns)
+    odd = any(v % 2 for v in ns)
+    name = ("2d_uniform_4x4_mpi1.json" if odd else "2d_uniform_2x2_refined_nw_mpi1.json") if dim == 2 else (
+        "3d_refined_bnw_2x2x2_mpi1.json")
+    lv = load(name, ns)[1][0]
+    kind = R.TRILINEAR if dim == 3 else R.BIQUADRATIC
+    od, dd = O.Domain(dim, ns, lv), _dev(dim, ns, lv)
+    coeffs = None
+    if op_kind == 1:
+        X = mesh.cell_centers(lv, dim, ns)
+        coeffs = np.exp(np.sin(3 * X[..., 0]) * np.cos(2 * X[..., 1]))[:, None].copy()
+        O.fill_ghost(od, coeffs, kind=kind)
+    plan = R.DftPlan(R.GhostFiller(dd, kind, R.FACES), neumann_mask=neumann_mask, op_kind=op_kind,
+                     coeffs=R.DeviceArray.from_host(coeffs) if op_kind else None)
+    args = dict(kind=kind, neumann_mask=neumann_mask, op_kind=op_kind, coeffs=coeffs)
+    for dtype, tol in [(R.F64, 1e-12), (R.F32, 2e-5)]:
+        t = R.np_dtype(dtype)
+        f0, u0 = random_field(od.shape(1), 35, t), random_field(od.shape(1), 36, t)
+        uref, uz = u0.astype(np.float64), np.zeros(od.shape(1))
+        O.dft_smooth(od, f0.astype(np.float64), uref, **args)
+        O.dft_smooth(od, f0.astype(np.float64), uz, **args)
+        df, du = R.DeviceArray.from_host(f0), R.DeviceArray.from_host(u0)
+        plan.smooth(df, du)
+        assert relerr(mesh.interior(du.get(), dim), mesh.interior(uref, dim)) <= tol, dtype
+        big = R.DeviceArray.from_host(np.full(u0.size + 1, 7, t))
+        R.check(R.lib().te_dft_apply(plan.h, dtype, df.ptr, big.ptr + t().itemsize, None))
+        got = big.get()[1:].reshape(u0.shape)
+        assert relerr(mesh.interior(got, dim), mesh.interior(uz, dim)) <= tol, dtype
+        mesh.interior(got, dim)[...] = 0
+        assert not got.any()

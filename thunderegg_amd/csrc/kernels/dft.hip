@@ -1,6 +1,6 @@
 // Poisson::DFTPatchSolver::solveSinglePatch (Poisson/DFTPatchSolver.h:420-450) for
 // every patch of a level in one launch, generic (VALU) form for any n: a workgroup holds
-// PPW patches, TPP threads each (a launch variant chosen by the autotuner's table, tune.h).
+// PPW patches, TPP threads each (by a rule, or a variant of the autotuner's table, tune.h).
 // Each patch is staged in LDS; each axis transform y = M x (executePlan, :205-265) is a
 // dense n x n product over all lines of that axis; eigenvalues (:320-361) come from a
 // per-axis sin^2 table.
@@ -9,6 +9,8 @@
 // the output.  UZERO: u is known to be identically zero (the first smoothing
 // sweep of a freshly zeroed level), so the interface terms of
 // modifyRHSForInternalBoundaryConditions vanish and u is not read.
+#include <algorithm>
+
 #include "../te_internal.h"
 #include "dft.h"
 #include "blas.h"
@@ -20,143 +22,302 @@
 namespace te {
 namespace {
 
+// The launch's geometry: LDS pitches and the divisions by run-time sizes.
+struct DftGeom {
+  int px;      // row pitch of the staged patch (odd where it fits, so that a wave's lines spread over the banks)
+  int mp;      // pitch of a transposed matrix; a multiple of 4 (vec) where it fits
+  int nmat;    // matrices per direction and copy: one per axis, or one for all of equal sizes and types
+  bool vec, share;  // share: one copy for the whole workgroup (every patch has the same types)
+  FastDiv d0, d1, lines[3], na[3];
+};
+
 // GM (2D): 0 = the ghost values of u are read from u (filled beforehand); 1 = they are
-// computed here from the neighbours' cells (ghost2d, the filler's closed forms); 2 = the same
+// computed here from the neighbours' cells (ghost2d.h, the filler's closed forms); 2 = the same
 // on u + P uc (DirectInterpolator applied on the fly: uc is the coarser level's solution).
 // With GM != 0, out must not alias u.
+//
+// A task of an axis transform is one line and four of its outputs: per step of the product one
+// staged value and four matrix values (one wide LDS read, the same for a wave's lanes, which
+// take consecutive lines) feed four multiply-adds.  The last forward transform divides by the
+// eigenvalues as it writes, the last inverse one writes the result.  The interface terms are
+// formed first, a thread per side cell (in 2D from one ring-table record each).
+// Bound by LDS reads on large levels, by the chain of loads and barriers on small ones.
+// Measured against one output a thread and task, the terms formed cell by cell (apply from
+// zero with its zeroed ghosts / sweep with its ghosts, us): 1,024 patches of 24^2 in FP64
+// 43.4 -> 14.9 / 49.1 -> 21.5; 512 of 12^3 in FP32 37.0 -> 16.2 / 47.8 -> 28.9; 512 of 6^3 in
+// FP32 10.6 -> 8.3 / 13.2 -> 14.0; 1,024 of 7^2 7.8 -> 6.7 / 10.0 -> 10.4; 48 problems
+// together, a third of them on 8^2 patches, 12.2 -> 10.7 ms.
 template <typename T, typename TF, typename TO, int D, int OP, bool UZERO, int GM = 0, int KIND = 0, typename TC = T>
 __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
                                                   const T* __restrict__ mats, const T* __restrict__ s2tab,
-                                                  const TF* __restrict__ f, const T* __restrict__ u,
-                                                  const T* __restrict__ coeffs, TO* __restrict__ out, Layout L,
-                                                  int ppw, FusedArgs<T, TC> fa)
+                                                  const TF* __restrict__ f, const T* u, const T* __restrict__ coeffs,
+                                                  TO* out, Layout L, int ppw, FusedArgs<T, TC> fa,
+                                                  const int4* __restrict__ ring, DftGeom G, bool zero_ghosts)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1;
-  const int N = n0 * n1 * n2;
+  const int nn[3] = { n0, n1, n2 }, N = n0 * n1 * n2, NP = G.px * n1 * n2;
   const int nmax = n0 > n1 ? (n0 > n2 ? n0 : n2) : (n1 > n2 ? n1 : n2);
+  const int msz = nmax * G.mp, nr = UZERO ? 0 : D == 2 ? 2 * (n0 + n1) : 2 * (n1 * n2 + n0 * n2 + n0 * n1);
   // this thread's patch (sub-block of tpp threads) and its index t within it; the threads
   // of a patch past the last one take part in the barriers only
   const int tpp = blockDim.x / ppw, sub = threadIdx.x / tpp, t = threadIdx.x - sub * tpp;
   const bool live = blockIdx.x * ppw + sub < L.np;
   const int p = live ? blockIdx.x * ppw + sub : L.np - 1;
-  T* sm = reinterpret_cast<T*>(smem_raw) + (size_t)sub * (2 * N + 2 * D * nmax * nmax);
-  T* A = sm;
-  T* B = sm + N;
-  T* MF = sm + 2 * N;                 // forward matrices, D x nmax^2
-  T* MI = MF + D * nmax * nmax;       // inverse matrices
+  // LDS: the matrices (forward, then inverse; one copy or one per patch), then per patch two
+  // buffers, the second of which first holds the interface terms
+  T* M = reinterpret_cast<T*>(smem_raw) + (G.share ? 0 : sub * 2 * G.nmat * msz);
+  T* A = reinterpret_cast<T*>(smem_raw) + (G.share ? 1 : ppw) * 2 * G.nmat * msz + sub * (NP + (NP > nr ? NP : nr));
+  T* B = A + NP;
+  T* term = B;  // consumed before the first transform writes B
   const int* pt = ptype + p * 8;      // fwd type per axis [0..2], eig type per axis [3..5], zero mode [6]
   const DevPatch& P = dp[p];
-  const int nn[3] = { n0, n1, n2 };
-
-  for (int a = 0; a < D; a++) {
-    int na = nn[a];
-    int tf = pt[a];
-    int ti = tf == 0 ? 1 : (tf == 3 ? 4 : tf);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
-    for (int k = t; k < na * na; k += tpp) {
-      MF[a * nmax * nmax + k] = mats[(tf * 3 + a) * kDftMatStride + k];
-      MI[a * nmax * nmax + k] = mats[(ti * 3 + a) * kDftMatStride + k];
-    }
-  }
-  // f_copy = f, then modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson :168-186)
-  for (int o = t; o < N; o += tpp) {
-    int x = o % n0;
-    int y = (o / n0) % n1;
-    int z = D == 3 ? o / (n0 * n1) : 0;
-    int gi = lin(L, p, 0, x, y, z);
-    T v = T(f[gi]);
-    if (!UZERO) {
-      const int c3[3] = { x, y, z };
-      const int st[3] = { 1, L.sx, L.sy };
-      const int sbase = D == 2 ? 4 : 20;
-#pragma unroll
-      for (int a = 0; a < D; a++) {
-#pragma unroll
-        for (int up = 0; up < 2; up++) {
-          bool edge = up ? (c3[a] == nn[a] - 1) : (c3[a] == 0);
-          if (!edge || P.type[sbase + 2 * a + up] < 0) continue;
-          int gidx = up ? gi + st[a] : gi - st[a];
-          T ih2 = T(P.inv_h2[a]);
-          T ug, ub;  // the ghost and the boundary cell
-          if (GM == 0) {
-            ug = u[gidx];
-            ub = u[gi];
-          } else {
-            const UAcc<T, TC, GM == 2> U{ u, fa.uc, fa.parent, fa.porth, L };
-            const int sd = 2 * a + up;
-            ug = ghost2d<T, KIND>(side_info(P, sd), p, sd, a == 0 ? y : x, nn[a], nn[1 - a], U);
-            ub = U(p, x, y);
-          }
-          if (OP == 0) {
-            v -= (ug + ub) * ih2;
-          } else {
-            int cq = gi - p * L.ps;
-            int cg = up ? cq + st[a] : cq - st[a];
-            T cb = coeffs[p * L.cs + cq], cgv = coeffs[p * L.cs + cg];
-            v -= (ug + ub) * (cb + cgv) * (ih2 * T(0.5));
-          }
-        }
+  if (UZERO && zero_ghosts && live)  // the patch's results follow after the barriers
+    for (int k = t; k < L.cs; k += tpp) out[p * L.ps + k] = TO(0);
+  {
+    const int m0 = G.share ? threadIdx.x : t, step = G.share ? blockDim.x : tpp;
+    for (int a = 0; a < G.nmat; a++) {
+      const int tf = pt[a], ti = tf == 0 ? 1 : (tf == 3 ? 4 : tf);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
+      for (int i = m0; i < nn[a] * nn[a]; i += step) {
+        const int k = G.na[a](i), j = i - k * nn[a];
+        M[a * msz + j * G.mp + k] = mats[(tf * 3 + a) * kDftMatStride + i];
+        M[(G.nmat + a) * msz + j * G.mp + k] = mats[(ti * 3 + a) * kDftMatStride + i];
       }
     }
-    A[o] = v;
+  }
+  // f_copy = f
+  for (int o = t; o < N; o += tpp) {
+    const int row = G.d0(o), x = o - row * n0, z = D == 3 ? G.d1(row) : 0, y = row - z * n1;
+    A[row * G.px + x] = T(f[lin(L, p, 0, x, y, z)]);
+  }
+  // modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson :168-186), sides in the
+  // reference's order
+  if (!UZERO && D == 2) {
+    for (int g = t; g < nr; g += tpp) {
+      int s, tt;
+      const int ri = ring_index(p, g, n0, n1, &s, &tt);
+      const int a = s >> 1, up = s & 1, nt = a == 0 ? n1 : n0;
+      T v = T(0);
+      if (P.type[4 + s] >= 0) {
+        int bx, by;
+        side_xy(s, 0, tt, nn[a], &bx, &by);
+        const int bi = lin(L, p, 0, bx, by, 0), gi = bi + (up ? 1 : -1) * (a == 0 ? 1 : L.sx);
+        if (GM == 0) {
+          v = u[gi] + u[bi];
+        } else {
+          const int4 r = ring[ri];
+          const int par = GM == 2 ? fa.parent[p] : 0, o = GM == 2 ? fa.porth[p] : -1;
+          // u, or u + P uc with q's parent and orthant, at a cell of patch q
+          auto val = [&](int q, int qpar, int qo, int x, int y) {
+            T w = at(u, lin(L, q, 0, x, y, 0));
+            if (GM == 2) {
+              const int cx = qo >= 0 ? (x + ((qo & 1) ? n0 : 0)) / 2 : x, cy = qo >= 0 ? (y + ((qo & 2) ? n1 : 0)) / 2 : y;
+              w = T(w + T(at(fa.uc, lin(L, qpar, 0, cx, cy, 0))));
+            }
+            return w;
+          };
+          T gv[4] = { T(0), T(0), T(0), T(0) };
+          ghost2d_gather<KIND>(r.x, r.y, r.z, s, tt, nn[a], nt,
+                               [&](int k, int q, int x, int y) { gv[k] = val(q, r.w >> 3, (r.w & 7) - 1, x, y); });
+          const T ug = ghost2d_combine<T, KIND>(r.x, r.y, tt, nt,
+                                                [&](int k, int e) {
+                                                  int x, y;
+                                                  side_xy(s, k, e, nn[a], &x, &y);
+                                                  return val(p, par, o, x, y);
+                                                },
+                                                gv);
+          v = ug + val(p, par, o, bx, by);
+        }
+        const T ih2 = T(P.inv_h2[a]);
+        if (OP == 0) v = v * ih2;
+        else v = v * (coeffs[bi] + coeffs[gi]) * (ih2 * T(0.5));
+      }
+      term[g] = v;
+    }
+  }
+  // 3D face cell g of axis a: its side and cell (first free axis fastest)
+  auto face_cell = [&](int a, int g, int* up, int (&c3)[3]) {
+    const int f0 = a == 0 ? 1 : 0, f1 = a == 2 ? 1 : 2, cells = nn[f0] * nn[f1];
+    *up = g >= cells ? 1 : 0;
+    const int q = g - *up * cells, j = a == 0 ? G.d1(q) : G.d0(q);
+    c3[a] = *up ? nn[a] - 1 : 0;
+    c3[f0] = q - j * nn[f0];
+    c3[f1] = j;
+  };
+  auto faces = [&](int a) { return 2 * N / nn[a]; };
+  if (!UZERO && D == 3) {
+#pragma unroll
+    for (int a = 0; a < D; a++) {
+      const int g0 = a == 0 ? 0 : a == 1 ? faces(0) : faces(0) + faces(1);
+      const T ih2 = T(P.inv_h2[a]);
+      for (int g = t; g < faces(a); g += tpp) {
+        int up, c3[3];
+        face_cell(a, g, &up, c3);
+        T v = T(0);
+        if (P.type[20 + 2 * a + up] >= 0) {
+          const int bi = lin(L, p, 0, c3[0], c3[1], c3[2]), st = a == 0 ? 1 : (a == 1 ? L.sx : L.sy);
+          const int gi = up ? bi + st : bi - st;
+          v = u[gi] + u[bi];
+          if (OP == 0) v = v * ih2;
+          else v = v * (coeffs[bi] + coeffs[gi]) * (ih2 * T(0.5));
+        }
+        term[g0 + g] = v;
+      }
+    }
   }
   __syncthreads();
-  // forward transform along each axis (DST-II / DCT-II / DCT-IV / DST-IV)
+  if (!UZERO) {
+#pragma unroll
+    for (int a = 0; a < D; a++) {
+      if (D == 2) {
+        const int nt = a == 0 ? n1 : n0, g0 = a == 0 ? 0 : 2 * n1;
+        for (int g = t; g < 2 * nt; g += tpp) {
+          int s, tt, bx, by;
+          ring_cell(g0 + g, n0, n1, &s, &tt);
+          side_xy(s, 0, tt, nn[a], &bx, &by);
+          A[by * G.px + bx] -= term[g0 + g];
+        }
+      } else {
+        const int g0 = a == 0 ? 0 : a == 1 ? faces(0) : faces(0) + faces(1);
+        for (int g = t; g < faces(a); g += tpp) {
+          int up, c3[3];
+          face_cell(a, g, &up, c3);
+          A[c3[0] + G.px * (c3[1] + n1 * c3[2])] -= term[g0 + g];
+        }
+      }
+      __syncthreads();
+    }
+  }
+  T lam[D];
+#pragma unroll
+  for (int a = 0; a < D; a++) lam[a] = T(4.0 / (P.h[a] * P.h[a]));
+  T scale = T(1);
+#pragma unroll
+  for (int a = 0; a < D; a++) scale *= T(2.0) / T(nn[a]);
+  // one transform (DST-II / DCT-II / DCT-IV / DST-IV and their inverses) along axis a
+  auto transform = [&](int a, const T* Mt, const T* src, auto put) {
+    const int na = nn[a], sta = a == 0 ? 1 : (a == 1 ? G.px : G.px * n1), nl = (int)G.lines[a].d;
+    const int tasks = nl * ((na + 3) / 4);
+    for (int i = t; i < tasks; i += tpp) {
+      const int kb = G.lines[a](i), l = i - kb * nl, k0 = 4 * kb;
+      int base;
+      if (a == 0) {
+        base = l * G.px;
+      } else {
+        const int q = G.d0(l);
+        base = l - q * n0 + (a == 1 ? q * G.px * n1 : q * G.px);
+      }
+      T acc[4] = { T(0), T(0), T(0), T(0) };
+      if (G.vec) {
+        typedef T V4 __attribute__((ext_vector_type(4)));
+#pragma unroll 4
+        for (int j = 0; j < na; j++) {
+          const T v = src[base + j * sta];
+          const V4 m = *reinterpret_cast<const V4*>(Mt + j * G.mp + k0);
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[r] += m[r] * v;
+        }
+      } else {
+        int k[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) k[r] = k0 + r < na ? k0 + r : na - 1;
+        for (int j = 0; j < na; j++) {
+          const T v = src[base + j * sta];
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[r] += Mt[j * G.mp + k[r]] * v;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (k0 + r < na) put(l, k0 + r, base + (k0 + r) * sta, acc[r]);
+    }
+  };
   T* src = A;
   T* dst = B;
+#pragma unroll
   for (int a = 0; a < D; a++) {
-    int na = nn[a];
-    int sta = a == 0 ? 1 : (a == 1 ? n0 : n0 * n1);
-    const T* M = MF + a * nmax * nmax;
-    for (int o = t; o < N; o += tpp) {
-      int k = (o / sta) % na;
-      int base = o - k * sta;
-      T acc = T(0);
-      for (int j = 0; j < na; j++) acc += M[k * na + j] * src[base + j * sta];
-      dst[o] = acc;
-    }
+    transform(a, M + (G.nmat == 1 ? 0 : a) * msz, src, [&](int l, int k, int at_, T v) {
+      if (a == D - 1) {  // divide by the eigenvalues
+        const int y = D == 3 ? G.d0(l) : 0, x = l - y * n0;
+        const int k3[3] = { x, D == 3 ? y : k, k };
+        T eig = T(0);
+#pragma unroll
+        for (int b = 0; b < D; b++) eig -= lam[b] * s2tab[(pt[3 + b] * 3 + b) * kDftMatDim + k3[b]];
+        v = v / eig;
+        if (pt[6] && l == 0 && k == 0) v = T(0);  // all-Neumann patch without neighbours (:438-440)
+      }
+      dst[at_] = v;
+    });
     __syncthreads();
-    T* t = src;
+    T* sw = src;
     src = dst;
-    dst = t;
+    dst = sw;
   }
-  // divide by the eigenvalues
-  for (int o = t; o < N; o += tpp) {
-    int k3[3] = { o % n0, (o / n0) % n1, D == 3 ? o / (n0 * n1) : 0 };
-    T eig = T(0);
-    for (int a = 0; a < D; a++) {
-      double h = P.h[a];
-      eig -= T(4.0 / (h * h)) * s2tab[(pt[3 + a] * 3 + a) * kDftMatDim + k3[a]];
-    }
-    src[o] /= eig;
-  }
-  __syncthreads();
-  if (pt[6] && t == 0) src[0] = T(0);  // all-Neumann patch without neighbours (:438-440)
-  __syncthreads();
+#pragma unroll
   for (int a = 0; a < D; a++) {
-    int na = nn[a];
-    int sta = a == 0 ? 1 : (a == 1 ? n0 : n0 * n1);
-    const T* M = MI + a * nmax * nmax;
-    for (int o = t; o < N; o += tpp) {
-      int k = (o / sta) % na;
-      int base = o - k * sta;
-      T acc = T(0);
-      for (int j = 0; j < na; j++) acc += M[k * na + j] * src[base + j * sta];
-      dst[o] = acc;
-    }
-    __syncthreads();
-    T* t = src;
+    transform(a, M + (G.nmat + (G.nmat == 1 ? 0 : a)) * msz, src, [&](int l, int k, int at_, T v) {
+      if (a < D - 1) {
+        dst[at_] = v;
+      } else if (live) {
+        const int y = D == 3 ? G.d0(l) : k, x = D == 3 ? l - y * n0 : l;
+        out[lin(L, p, 0, x, y, D == 3 ? k : 0)] = TO(v * scale);
+      }
+    });
+    if (a < D - 1) __syncthreads();
+    T* sw = src;
     src = dst;
-    dst = t;
+    dst = sw;
   }
-  T scale = T(1);
-  for (int a = 0; a < D; a++) scale *= T(2.0) / T(nn[a]);
-  for (int o = t; o < N; o += tpp) {
-    int x = o % n0;
-    int y = (o / n0) % n1;
-    int z = D == 3 ? o / (n0 * n1) : 0;
-    if (live) out[lin(L, p, 0, x, y, z)] = TO(src[o] * scale);
+}
+
+// pitches, sharing and the launch's LDS bytes for ppw patches a workgroup
+size_t dft_geom(const te_dft_plan* pl, size_t esz, int ppw, bool terms, DftGeom* G)
+{
+  const te_domain* d = pl->g->d;
+  const int D = d->dim, n0 = d->ns[0], n1 = d->ns[1], n2 = D == 3 ? d->ns[2] : 1;
+  const int nmax = std::max(n0, std::max(n1, n2)), N = n0 * n1 * n2;
+  const bool cubic = n0 == n1 && (D == 2 || n2 == n0);
+  G->share = pl->mask == 0;
+  G->nmat = G->share && cubic ? 1 : D;
+  auto bytes = [&]() {
+    const size_t np = (size_t)G->px * n1 * n2;
+    return esz * ((size_t)(G->share ? 1 : ppw) * 2 * G->nmat * nmax * G->mp +
+                  (size_t)ppw * (np + std::max<size_t>(np, !terms ? 0 : D == 2 ? 2 * (n0 + n1) : 2 * (n1 * n2 + n0 * n2 + n0 * n1))));
+  };
+  G->px = n0 | 1;
+  G->mp = (nmax + 3) / 4 * 4;
+  G->vec = true;
+  if (bytes() > 65536) {  // large patches: unpadded
+    G->px = n0;
+    G->mp = nmax;
+    G->vec = nmax % 4 == 0;
   }
+  G->d0 = FastDiv(n0);
+  G->d1 = FastDiv(n1);
+  const int nn[3] = { n0, n1, n2 };
+  for (int a = 0; a < 3; a++) {
+    G->na[a] = FastDiv(nn[a]);
+    G->lines[a] = FastDiv(N / nn[a]);
+  }
+  return bytes();
+}
+
+// patches per workgroup and threads per patch: the autotuner's choice for this shape, or (variant
+// 0) a thread per four outputs of a transform, in powers of two from 32 to 256 threads (up to one
+// per cell while the level does not fill the CUs with 256 threads each), and as many patches as
+// make 256 threads and at most 48 KB of LDS
+DftGenericVariant dft_shape(const te_dft_plan* pl, size_t esz, bool terms)
+{
+  const te_domain* d = pl->g->d;
+  const int v = tune_variant(TUNE_DFT_GENERIC, d->dim, d->ns[0], esz == 8 ? TE_F64 : TE_F32);
+  if (v != 0) return dft_generic_variant(v);
+  const int N = d->ns[0] * d->ns[1] * (d->dim == 3 ? d->ns[2] : 1);
+  DftGenericVariant w{ 1, 32 };
+  while (w.tpp < 256 && (w.tpp * 4 < N || (w.tpp < N && (long)d->np * w.tpp < 256 * cu_count()))) w.tpp *= 2;
+  DftGeom G;
+  for (w.ppw = 256 / w.tpp; w.ppw > 1 && dft_geom(pl, esz, w.ppw, terms, &G) > 49152; w.ppw /= 2) {
+  }
+  return w;
 }
 
 // The same solve for 3D patches of 16^3 cells on the matrix cores.  Every axis transform is a
@@ -553,13 +714,6 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
 {
   const te_domain* d = pl->g->d;
   Layout L = make_layout(d->dim, d->ns, 1, d->np);
-  int nmax = 0;
-  int N = 1;
-  for (int a = 0; a < D; a++) {
-    nmax = d->ns[a] > nmax ? d->ns[a] : nmax;
-    N *= d->ns[a];
-  }
-  size_t shmem = sizeof(T) * (2 * (size_t)N + 2 * (size_t)D * nmax * nmax);
   const T* mats = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_mats64 : (const void*)pl->d_mats32);
   const T* s2 = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_s2_64 : (const void*)pl->d_s2_32);
   const T* cf = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_coeffs64 : (const void*)pl->d_coeffs32);
@@ -587,14 +741,14 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
 #undef TE_D3
     return;
   }
-  // patches per workgroup and threads per patch: the autotuner's choice for this shape
-  const DftGenericVariant v = dft_generic_variant(tune_variant(TUNE_DFT_GENERIC, D, d->ns[0], sizeof(T) == 8 ? TE_F64 : TE_F32));
+  const DftGenericVariant v = dft_shape(pl, sizeof(T), !uzero);
+  DftGeom G;
+  const size_t shmem = dft_geom(pl, sizeof(T), v.ppw, !uzero, &G);
   const int grid = (d->np + v.ppw - 1) / v.ppw;
-  shmem *= (size_t)v.ppw;
   const FusedArgs<T, T> fa{ nullptr, nullptr, nullptr };
 #define TE_DL(OP_, UZ_)                                                                                          \
   hipLaunchKernelGGL((dft_kernel<T, TF, TO, D, OP_, UZ_>), dim3(grid), dim3(v.ppw * v.tpp), shmem, s,          \
-                     d->d_patches, pl->d_ptype, mats, s2, f, u, cf, out, L, v.ppw, fa)
+                     d->d_patches, pl->d_ptype, mats, s2, f, u, cf, out, L, v.ppw, fa, nullptr, G, zg)
   if (pl->op_kind == 0) {
     if (uzero) TE_DL(0, true); else TE_DL(0, false);
   } else {
@@ -619,16 +773,14 @@ void launch_fused_t(const te_dft_plan* pl, const void* fv, const void* uv, void*
 {
   const te_domain* d = pl->g->d;
   Layout L = make_layout(2, d->ns, 1, d->np);
-  const int nmax = d->ns[0] > d->ns[1] ? d->ns[0] : d->ns[1];
-  const int N = d->ns[0] * d->ns[1];
-  size_t shmem = sizeof(T) * (2 * (size_t)N + 4 * (size_t)nmax * nmax);
   const T* mats = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_mats64 : (const void*)pl->d_mats32);
   const T* s2 = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_s2_64 : (const void*)pl->d_s2_32);
   const T* cf = (const T*)(sizeof(T) == 8 ? (const void*)pl->d_coeffs64 : (const void*)pl->d_coeffs32);
-  const DftGenericVariant v =
-    dft_generic_variant(tune_variant(TUNE_DFT_GENERIC, 2, d->ns[0], sizeof(T) == 8 ? TE_F64 : TE_F32));
+  const DftGenericVariant v = dft_shape(pl, sizeof(T), !uzero);
+  DftGeom G;
+  const size_t shmem = dft_geom(pl, sizeof(T), v.ppw, !uzero, &G);
   const int grid = (d->np + v.ppw - 1) / v.ppw;
-  shmem *= (size_t)v.ppw;
+  const int4* ring = (const int4*)(gm == 2 ? link->d_ring : d->d_ring);
   const FusedArgs<T, TC> fa{ (const TC*)ucv, link ? link->d_parent : nullptr, link ? link->d_orth : nullptr };
   const TF* f = (const TF*)fv;
   const T* u = (const T*)uv;
@@ -636,7 +788,7 @@ void launch_fused_t(const te_dft_plan* pl, const void* fv, const void* uv, void*
   const int kind = pl->g->kind;
 #define TE_DF(OP_, UZ_, GM_, K_)                                                                                 \
   hipLaunchKernelGGL((dft_kernel<T, TF, TO, 2, OP_, UZ_, GM_, K_, TC>), dim3(grid), dim3(v.ppw * v.tpp), shmem, \
-                     s, d->d_patches, pl->d_ptype, mats, s2, f, u, cf, out, L, v.ppw, fa)
+                     s, d->d_patches, pl->d_ptype, mats, s2, f, u, cf, out, L, v.ppw, fa, ring, G, false)
 #define TE_DFO(OP_)                                                        \
   do {                                                                     \
     if (uzero) TE_DF(OP_, true, 0, 0);                                     \
@@ -720,8 +872,9 @@ int launch_dft(const te_dft_plan* pl, int dt, int dtf, int dto, const void* f, c
 {
   const te_domain* d = pl->g->d;
   if (d->np == 0) return TE_OK;
-  // the 3D matrix-core kernels zero the ghosts themselves, where the patches start on 16 bytes
-  const bool own = dft3_mfma_supported(pl) && uzero && f != out && (uintptr_t)out % 16 == 0;
+  // the kernels of this file zero the ghosts themselves (the 3D matrix-core ones by 16-byte stores)
+  const bool own = uzero && f != out &&
+                   (dft3_mfma_supported(pl) ? (uintptr_t)out % 16 == 0 : !(pl->use_mfma && dft_mfma_supported(pl)));
   if (fill && !uzero && (!dft3_mfma_supported(pl) || out == u)) {
     set_error("internal: a 3D sweep that forms ghosts needs 8^3 or 16^3 patches and another buffer for its result");
     return TE_ERR_ARG;

@@ -73,14 +73,26 @@ __global__ void ghost_corners_2d(const DevPatch* __restrict__ dp, T* __restrict_
   }
 }
 
-// 3D faces: one workgroup per patch (fill_faces3), so that the patch's neighbour records are
-// wave-uniform and a cell's place on the face takes one division.
-template <typename T>
-__global__ void __launch_bounds__(256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L)
+// 3D faces: one workgroup per patch, so that the patch's neighbour records are wave-uniform and a
+// cell's place on the face takes one division.  SIDES (faces of at most 64 cells): a wave per
+// side; else each thread takes the same cell of all six sides (fill_faces3).
+template <typename T, bool SIDES>
+__global__ void __launch_bounds__(SIDES ? 384 : 256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L)
 {
   const int p = xcd_item(blockIdx.x, gridDim.x);
   if (p >= L.np) return;
-  fill_faces3<T>(L, dp[p], u, p, threadIdx.x, blockDim.x);
+  const DevPatch& P = dp[p];
+  if (!SIDES) {
+    fill_faces3<T>(L, P, u, p, threadIdx.x, blockDim.x);
+    return;
+  }
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), k = threadIdx.x & 63;
+  const int type = P.type[20 + s], ni = L.n[s < 2 ? 1 : 0], nj = L.n[s < 4 ? 2 : 1], j = k / ni;
+  if (type < 0 || k >= ni * nj) return;
+  for (int c = 0; c < L.ncomp; c++) {
+    const T G = face_ghost3<T>(L, type, P.orth[20 + s], P.nbr[20 + s], u, p, c, s, k - j * ni, j);
+    at(u, side_cell3(L, p, c, s, -1, k - j * ni, j)) = G;
+  }
 }
 
 // 3D edge e (Face<3,1>): free axis = e >> 2; fixed sides in axis order with
@@ -200,9 +212,11 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, hipStrea
   } else {
     int face = 0;  // cells of the largest face: a thread each, up to 256
     for (int a = 0; a < 3; a++) face = std::max(face, d->ns[a] * d->ns[(a + 1) % 3]);
-    if (faces)
-      hipLaunchKernelGGL((ghost_faces_3d<T>), dim3(xcd_grid(d->np)), dim3(std::min(256, (face + 63) / 64 * 64)), 0, s,
-                         d->d_patches, u, L);
+    if (faces && face <= 64)
+      hipLaunchKernelGGL((ghost_faces_3d<T, true>), dim3(xcd_grid(d->np)), dim3(384), 0, s, d->d_patches, u, L);
+    else if (faces)
+      hipLaunchKernelGGL((ghost_faces_3d<T, false>), dim3(xcd_grid(d->np)), dim3(std::min(256, (face + 63) / 64 * 64)),
+                         0, s, d->d_patches, u, L);
     if (g->fill_type != TE_FACES) {
       int tmax = d->ns[0];
       for (int a = 1; a < 3; a++) tmax = d->ns[a] > tmax ? d->ns[a] : tmax;
