@@ -559,3 +559,34 @@ def test_vcycle3d_refined_fused(name, n, op_kind, neumann, sweeps, monkeypatch):
         if op_kind == 0 and not neumann:
             ol = O.Levels([O.Domain(dim, ns, lv) for lv in levels], filler_kind=R.TRILINEAR, smoother_kind=0)
             assert relerr(got, mesh.interior(ol.vcycle(f.copy(), pre=pre, post=post, coarse=coarse), dim)) <= tol
+
+
+def test_vcycle3d_partly_covered_coarse_patch():
+    """A coarse patch with seven of its eight children (a notch in the finer level): the coarse
+    cells without a child get zero from the restriction, in every cycle, as in the oracle."""
+    ns = (8, 8, 8)
+    levels = solver.uniform_levels(3, 1, ns)
+    fine = levels[0]
+    gone = fine["id"][-1]
+    fine = fine[:-1].copy()
+    hit = (fine["nbr_ids"] == gone).any(axis=2) & (fine["nbr_type"] != mesh.NBR_NONE)
+    fine["nbr_type"][hit] = mesh.NBR_NONE
+    fine["nbr_ids"][hit] = -1
+    fine["nbr_ranks"][hit] = -1
+    coarse = levels[1].copy()
+    kids = coarse["child_ids"]
+    coarse["child_ranks"][kids == gone] = -1
+    kids[kids == gone] = -1
+    levels = [fine, coarse] + [lv.copy() for lv in levels[2:]]
+    f = random_field(mesh.padded_shape(len(fine), 3, ns), 3)
+    want = None
+    for prec, tol in ((R.F64, 1e-12), (R.F32, 2e-5)):
+        g = solver.GMG(3, ns, levels, filler_kind=R.TRILINEAR, precision=prec)
+        got = mesh.interior(g.vcycle(f), 3)
+        if want is None:
+            ol = O.Levels([O.Domain(3, ns, lv) for lv in levels], filler_kind=R.TRILINEAR, smoother_kind=0)
+            want = mesh.interior(ol.vcycle(f.copy(), pre=1, post=1, coarse=1), 3)
+        assert relerr(got, want) <= tol
+        # scratch that an earlier right-hand side left behind must not reach the result
+        g.vcycle(1e6 * f)
+        assert relerr(mesh.interior(g.vcycle(f), 3), want) <= tol

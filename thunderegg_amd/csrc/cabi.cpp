@@ -386,6 +386,8 @@ int te_level_link_create(const te_domain* fine, const te_domain* coarse, te_leve
     }
     child[(size_t)cp * 8 + nchild[cp]++] = i;  // fine local order = increasing
   }
+  for (int c = 0; c < coarse->np; c++)
+    l->covered = l->covered && (nchild[c] == (1 << fine->dim) || (nchild[c] == 1 && orth[child[(size_t)c * 8]] < 0));
   hipError_t e = hipSuccess;
   size_t nf = std::max(fine->np, 1), nc = std::max(coarse->np, 1);
   e = hipMalloc(&l->d_parent, sizeof(int32_t) * nf);

@@ -46,7 +46,8 @@ int launch_resid_restrict(const te_ghost_filler* g, const te_level_link* link, i
                           const void* coeffs, int dt, int dtf, const void* f, const void* u, int dtc, void* fc,
                           hipStream_t s);
 // Cycle::restrict in 3D (kernels/stencil.hip): fc = restriction of f - A u with u's ghosts formed in
-// the launch; 8^3 or 16^3 patches, a regular link.  fc's ghost cells are not written.
+// the launch; 8^3 or 16^3 patches, a regular link that covers the coarse level (a coarse cell
+// without a child would not be written).  fc's ghost cells are not written.
 bool resid_restrict3_supported(const te_ghost_filler* g, const te_level_link* link);
 int launch_resid_restrict3(const te_ghost_filler* g, const te_level_link* link, int op_kind, int neumann,
                            const void* coeffs, int dt, int dtf, const void* f, const void* u, int dtc, void* fc,

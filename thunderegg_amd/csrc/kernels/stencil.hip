@@ -309,7 +309,7 @@ bool resid_restrict3_supported(const te_ghost_filler* g, const te_level_link* li
 {
   const te_domain* d = g->d;
   return d->dim == 3 && (d->ns[0] == 8 || d->ns[0] == 16) && d->ns[1] == d->ns[0] && d->ns[2] == d->ns[0] &&
-         link->regular && link->fine == d;
+         link->regular && link->covered && link->fine == d;
 }
 
 int launch_resid_restrict3(const te_ghost_filler* g, const te_level_link* link, int op_kind, int neumann,
@@ -318,7 +318,7 @@ int launch_resid_restrict3(const te_ghost_filler* g, const te_level_link* link, 
 {
   if (g->d->np == 0) return TE_OK;
   if (!resid_restrict3_supported(g, link)) {
-    set_error("internal: 3D residual / restriction needs 8^3 or 16^3 patches and a regular link");
+    set_error("internal: 3D residual / restriction needs 8^3 or 16^3 patches and a regular, covered link");
     return TE_ERR_UNSUPPORTED;
   }
   if (dt == TE_F64 && dtf == TE_F64 && dtc == TE_F64)

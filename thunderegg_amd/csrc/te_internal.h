@@ -183,6 +183,8 @@ struct te_level_link {
   // even cells per side, and every coarse patch has either one copied child or children of
   // distinct orthants: each coarse cell then lies under one child
   bool regular = true;
+  // every coarse patch has a copied child or one per orthant: no coarse cell is without a child
+  bool covered = true;
 };
 
 namespace te {
