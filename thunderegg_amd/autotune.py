@@ -1,9 +1,8 @@
 """Autotuner for the DFT patch-solve launches.
 
-For every patch shape the solvers run with the DFT smoother -- 2D n = 8, 16, 32 and 3D
-n = 8, in FP32 and FP64 -- it times each launch variant of the kernel that shape uses
-(tune.h: patches per workgroup x threads per patch for the VALU kernel, the workgroup count
-of the 2D matrix-core kernel) on a uniform level of about 4-16 thousand patches, with HIP
+For 2D patches of n = 8 and 16, in FP32 and FP64, it times each launch variant of the DFT
+patch solve (tune.h: patches per workgroup x threads per patch for the VALU kernel, the
+workgroup count of the 2D matrix-core kernel) on a uniform level of 16,384 patches, with HIP
 events (te_tune_time_dft), checks that the variant's result has the same bits as the hand
 default's, and writes the table the library loads on first use (tune_table.txt beside
 libthunderegg_amd.so).  A variant replaces the default only when it is faster by more than
@@ -29,8 +28,9 @@ from .solver import uniform_levels
 HERE = os.path.dirname(os.path.abspath(__file__))
 DEFAULT_OUT = os.path.join(HERE, "tune_table.txt")
 
-# (dim, n, uniform level): about 4-16 thousand patches each
-SHAPES = [(2, 8, 7), (2, 16, 7), (2, 32, 6), (3, 8, 4)]
+# (dim, n, uniform level) of 16,384 patches each; 2D 32^2 and 3D 8^3 patches have kernels of one
+# launch shape (dft32_kernel, dft3_tile8_kernel), nothing to choose
+SHAPES = [(2, 8, 7), (2, 16, 7)]
 # the 3D compact cycle (16^3 patches): its finest-level sweeps on a uniform level
 C3_LEVEL = 4
 

@@ -20,6 +20,7 @@
 namespace te {
 namespace {
 
+// variant 0 is the launch's own rule (dft_shape); its entry here is not used
 constexpr DftGenericVariant kGeneric[] = { { 1, 256 }, { 1, 128 }, { 1, 64 }, { 2, 128 },
                                            { 4, 64 },  { 2, 64 },  { 8, 32 } };
 constexpr int kGenericCount = sizeof(kGeneric) / sizeof(kGeneric[0]);
