@@ -701,3 +701,71 @@ def test_dft_generic_sizes(ns, neumann_mask, op_kind):
         assert relerr(mesh.interior(got, dim), mesh.interior(uz, dim)) <= tol, dtype
         mesh.interior(got, dim)[...] = 0
         assert not got.any()
+
+
+@pytest.mark.parametrize("n", [8, 16])
+@pytest.mark.parametrize("off", [0, 1])
+def test_star3_tile(n, off):
+    """The LDS operator of large 3D levels (more patches than CUs, 8^3 and 16^3; refined, so that
+    every face type occurs) against the ghost fill followed by the operator: the bits of u, and
+    the result but for contracted products (a few roundings of its largest term)."""
+    ns = (n,) * 3
+    forest = solver.Forest(3, 2)
+    forest.refine((np.arange(64) % 3 != 0).astype(np.uint8))
+    forest.balance()
+    lv = forest.build_domains(ns)[0]
+    assert len(lv) > 256 and len(lv) % 8 != 0 and all((lv["nbr_type"][:, 20:] == k).any() for k in (-1, 0, 1, 2))
+    dd, L = R.Domain(3, ns, lv), R.lib()
+    g = R.GhostFiller(dd, R.TRILINEAR, R.FACES)
+    shape = mesh.padded_shape(len(lv), 3, ns, 2)
+    size = int(np.prod(shape))
+    ih2 = 1.0 / lv["spacings"].min() ** 2
+    for dtype in (R.F64, R.F32):
+        t = R.np_dtype(dtype)
+        u0, f0 = random_field((size + off,), 83, t), random_field((size + off,), 84, t)
+        cf = R.DeviceArray.from_host(np.exp(random_field(mesh.padded_shape(len(lv), 3, ns), 85, t)).astype(t))
+        beta = float(np.abs(cf.get()).max())
+        for op, neumann in ((0, 0), (0, 1), (1, 0)):
+            u1, u2, f = (R.DeviceArray.from_host(v) for v in (u0, u0, f0))
+            a1, a2, r1 = (R.DeviceArray.from_host(np.full(size + off, 7, t)) for _ in range(3))
+            p = [d.ptr + off * t().itemsize for d in (u1, u2, f, a1, a2, r1)]
+            R.check(L.te_ghost_fill(g.h, dtype, p[0], 2, None))
+            if op == 0:
+                R.check(L.te_star_apply_patches(g.h, dtype, neumann, p[0], p[3], 2, None))
+                R.check(L.te_star_apply(g.h, dtype, neumann, p[1], p[4], 2, None))
+            else:
+                R.check(L.te_varstar_apply(g.h, dtype, cf.ptr, p[1], p[4], 2, None))
+            assert np.array_equal(u1.get(), u2.get())
+            tol = 8 * np.finfo(t).eps * 12 * ih2 * float(np.abs(u0).max()) * (beta if op else 1.0)
+            got = a2.get()[off:].reshape(shape)
+            if op == 0:
+                assert np.abs(got - a1.get()[off:].reshape(shape)).max() <= tol
+            else:
+                U = u1.get()[off:].reshape(shape).astype(np.float64)
+                B = cf.get().astype(np.float64)[:, :1]
+                M, C0 = mesh.interior(U, 3), mesh.interior(B, 3)
+                want = np.zeros(M.shape)
+                for a in range(3):
+                    h2 = (1.0 / lv["spacings"][:, a] ** 2).reshape(-1, 1, 1, 1, 1)
+                    ax = 4 - a
+                    sl = [slice(None), slice(None)] + [slice(1, -1)] * 3
+                    sl_l, sl_u = list(sl), list(sl)
+                    sl_l[ax], sl_u[ax] = slice(0, -2), slice(2, None)
+                    UL, UU = U[tuple(sl_l)].copy(), U[tuple(sl_u)].copy()
+                    first, last = [slice(None)] * 5, [slice(None)] * 5
+                    first[ax], last[ax] = 0, -1
+                    pl, pu = lv["nbr_type"][:, 20 + 2 * a] < 0, lv["nbr_type"][:, 21 + 2 * a] < 0
+                    UL[tuple(first)][pl] = -M[tuple(first)][pl]
+                    UU[tuple(last)][pu] = -M[tuple(last)][pu]
+                    CL, CU = B[tuple(sl_l)], B[tuple(sl_u)]
+                    want += ((CU + C0) * (UU - M) - (CL + C0) * (M - UL)) * (0.5 * h2)
+                assert np.abs(mesh.interior(got, 3) - want).max() <= tol
+            u2.upload(u0)
+            R.check(L.te_residual(g.h, dtype, op, neumann, cf.ptr if op else None, p[2], p[1], p[5], 2, None))
+            assert np.array_equal(u1.get(), u2.get())
+            want = f0.astype(np.float64)[off:].reshape(shape) - got.astype(np.float64)
+            r = r1.get()[off:].reshape(shape)
+            assert np.abs(mesh.interior(r, 3) - mesh.interior(want, 3)).max() <= tol + np.finfo(t).eps * float(np.abs(f0).max())
+            for v in (r, got):
+                mesh.interior(v, 3)[...] = 0
+                assert not v.any()  # ghost cells of the output are zero

@@ -154,12 +154,114 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) star_kernel(const DevPatc
   }
 }
 
+// The ghost fill and the stencil of 3D patches of N^3 cells through LDS, on levels of more patches
+// than CUs: a workgroup stages its patch as it lies in memory (padded, 16-byte loads), puts the
+// face ghosts into it (and into u for the caller) and each thread forms 16 bytes of the padded
+// result at a time, its z and y neighbours by wide LDS reads.  star_kernel above reads each cell
+// seven times through the vector L1 and its stencil waits for the ghosts' stores; here it waits
+// for LDS only.  Bound by memory.  Operator / residual with the ghost fill, star_kernel -> this
+// one, us: 2,535 patches of 16^3 (refined octree, FP32) 62 / 70 -> 39 / 43 (a torch copy of the
+// vector takes 17); 4,096 of 16^3 in FP32 69 / 104 -> 56 / 83, VarPoisson in FP64 348 / 377 ->
+// 213 / 224; 4,096 of 8^3 in FP32 21.6 / 23 -> 12.3 / 14.3, in FP64 32 / 32 -> 20 / 24; 512 of
+// 8^3 6.7 -> 5.5.  Not for 16^3 Poisson in FP64 (149 / 175 against 149 / 186: three workgroups of
+// 46 KB a CU) and VarPoisson in FP32 (161 / 182 against 170 / 184: bound by the coefficients' reads).
+template <typename T, typename TF, typename TO, int OP, int N>
+__global__ void __launch_bounds__(N == 16 ? 256 : 64) star3_tile_kernel(const DevPatch* __restrict__ dp, T* u,
+                                                                        const T* __restrict__ cf,
+                                                                        const TF* __restrict__ fin,
+                                                                        TO* __restrict__ out, Layout L, int neumann)
+{
+  constexpr int SX = N + 2, SY = SX * SX, PS = SX * SY, NT = N == 16 ? 256 : 64;
+  constexpr int W = 16 / sizeof(T);  // values a group
+  static_assert(PS % W == 0 && SY % W == 0 && N * N == NT, "whole groups; a cell of each face per thread");
+  __shared__ __align__(16) T tile[PS];
+  const int p = xcd_item(blockIdx.x, gridDim.x);
+  if (p >= L.np) return;
+  const DevPatch& P = dp[p];
+  const int t = threadIdx.x, fi = t % N, fj = t / N;
+  const T ih2[3] = { T(P.inv_h2[0]), T(P.inv_h2[1]), T(P.inv_h2[2]) };
+  typedef T VecT __attribute__((ext_vector_type(W), aligned(sizeof(T))));
+  typedef TF VecF __attribute__((ext_vector_type(W), aligned(sizeof(TF))));
+  typedef TO VecO __attribute__((ext_vector_type(W), aligned(sizeof(TO))));
+  for (int c = 0; c < L.ncomp; c++) {
+    const int base = p * L.ps + c * L.cs, cbase = p * L.cs;
+    if (c) __syncthreads();  // the last component's reads of the tile
+    T G[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+      if (P.type[20 + s] >= 0) {
+        G[s] = face_ghost3<T>(L, P.type[20 + s], P.orth[20 + s], P.nbr[20 + s], u, p, c, s, fi, fj);
+      } else {
+        const T b = at(u, side_cell3(L, p, c, s, 0, fi, fj));
+        G[s] = (OP == 0 && neumann) ? b : -b;
+      }
+    }
+    for (int k = t; k < PS / W; k += NT)
+      *reinterpret_cast<VecT*>(tile + W * k) = *reinterpret_cast<const VecT*>(&at(u, base + W * k));
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+      tile[side_cell3(L, 0, 0, s, -1, fi, fj)] = G[s];
+      if (P.type[20 + s] >= 0) at(u, side_cell3(L, p, c, s, -1, fi, fj)) = G[s];
+    }
+    __syncthreads();
+    for (int k = t; k < PS / W; k += NT) {
+      VecO res;
+      const int q0 = W * k;
+#pragma unroll
+      for (int j = 0; j < W; j++) res[j] = TO(0);
+      if (q0 >= SY && q0 < PS - SY) {  // whole groups lie in or out of the ghost planes
+        VecF fv;
+        if (fin) fv = *reinterpret_cast<const VecF*>(&at(fin, base + q0));
+#pragma unroll
+        for (int j = 0; j < W; j++) {  // rows' ghosts too (every neighbour lies in the tile), set to zero below
+          const int q = q0 + j, y = q / SX % SX, x = q % SX;
+          const T mid = tile[q];
+          T acc = T(0);
+          const int st[3] = { 1, SX, SY };
+#pragma unroll
+          for (int a = 0; a < 3; a++) {
+            const T lower = tile[q - st[a]], upper = tile[q + st[a]];
+            if (OP == 0) {
+              acc += (upper - T(2) * mid + lower) * ih2[a];
+            } else {
+              const int ci = cbase + q;
+              const T cm = at(cf, ci), cl = at(cf, ci - st[a]), cu = at(cf, ci + st[a]);
+              acc += ((cu + cm) * (upper - mid) - (cl + cm) * (mid - lower)) * (ih2[a] * T(0.5));
+            }
+          }
+          const bool in = x >= 1 && x <= N && y >= 1 && y <= N;
+          res[j] = in ? (fin ? TO(T(fv[j]) - acc) : TO(acc)) : TO(0);
+        }
+      }
+      *reinterpret_cast<VecO*>(&at(out, base + q0)) = res;
+    }
+  }
+}
+
 template <typename T, typename TF, typename TO, int D, int OP>
 void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* out, int ncomp, int neumann, bool fill,
                 hipStream_t s)
 {
   const te_domain* d = g->d;
   Layout L = make_layout(d->dim, d->ns, ncomp, d->np);
+  // star3_tile_kernel's levels: those that fill the CUs, of the patch sizes it is written for; 16^3
+  // patches only where it is the faster one (its comment)
+  if constexpr (D == 3) {
+    const bool cube = L.n[1] == L.n[0] && L.n[2] == L.n[0];
+    if (fill && d->np > 256 && cube && L.n[0] == 8) {
+      hipLaunchKernelGGL((star3_tile_kernel<T, TF, TO, OP, 8>), dim3(xcd_grid(d->np)), dim3(64), 0, s, d->d_patches,
+                         u, cf, fin, out, L, neumann);
+      return;
+    }
+    if constexpr ((OP == 0) == (sizeof(T) == 4)) {
+      if (fill && d->np > 256 && cube && L.n[0] == 16) {
+        hipLaunchKernelGGL((star3_tile_kernel<T, TF, TO, OP, 16>), dim3(xcd_grid(d->np)), dim3(256), 0, s,
+                           d->d_patches, u, cf, fin, out, L, neumann);
+        return;
+      }
+    }
+  }
   const bool pairs = L.n[0] % 2 == 0 && (uintptr_t)u % (2 * sizeof(T)) == 0 && (uintptr_t)fin % (2 * sizeof(TF)) == 0 &&
                      (uintptr_t)out % (2 * sizeof(TO)) == 0;
   const int V = pairs ? 2 : 1, per = (L.n[0] + 2) / V;
