@@ -769,3 +769,77 @@ def test_star3_tile(n, off):
             for v in (r, got):
                 mesh.interior(v, 3)[...] = 0
                 assert not v.any()  # ghost cells of the output are zero
+
+
+@pytest.mark.parametrize("ns,level,ncomp,dtype", [
+    ((16, 16, 16), 5, 3, R.F64), ((16, 16, 16), 5, 8, R.F32), ((12, 12, 12), 5, 8, R.F64), ((64, 64), 7, 8, R.F64)])
+def test_vectors_past_4_gib(ns, level, ncomp, dtype):
+    """Vectors of several components whose bytes pass 2^32: the ghost fill, the operator and the
+    residual of every component have the bits of the same calls on that component alone.  Only the
+    last patches and those 4 GiB before them (where an offset cut to 32 bits would land) hold data."""
+    _print_case("past-4-gib", ns, level, ncomp, dtype)
+    dim, L, t = len(ns), R.lib(), R.np_dtype(dtype)
+    lv = solver.uniform_levels(dim, level, ns)[0]
+    dd = R.Domain(dim, ns, lv)
+    g = R.GhostFiller(dd, R.TRILINEAR if dim == 3 else R.BILINEAR, R.FACES)
+    np_, cs, sz, k = len(lv), int(np.prod([n + 2 for n in ns])), t().itemsize, 64
+    ps = cs * ncomp
+    assert (np_ - k) * ps * sz > 1 << 32
+    back = (np_ - k) - (((1 << 32) // sz + ps - 1) // ps)
+    blocks = [(back, k + 2), (np_ - k, k)]
+
+    def fresh(nc, data):
+        d = R.DeviceArray(dd.shape(nc), t)
+        d.zero()
+        for (p, n), v in zip(blocks, data):
+            v = np.ascontiguousarray(v)
+            R.check(L.te_memcpy_h2d(d.ptr + p * cs * nc * sz, v.ctypes.data, v.nbytes))
+        return d
+
+    def got(d, nc):
+        out = []
+        for p, n in blocks:
+            v = np.empty((n,) + dd.shape(nc)[1:], t)
+            R.check(L.te_memcpy_d2h(v.ctypes.data, d.ptr + p * cs * nc * sz, v.nbytes))
+            out.append(v)
+        return out
+
+    u0, f0 = ([random_field((n,) + dd.shape(ncomp)[1:], s + i, t) for i, (p, n) in enumerate(blocks)] for s in (91, 95))
+    f = fresh(ncomp, f0)
+    out = R.DeviceArray(dd.shape(ncomp), t)
+    results = []
+    for call in ("fill", "apply", "residual"):
+        u = fresh(ncomp, u0)
+        if call == "fill":
+            g.fill_ghost(u)
+        elif call == "apply":
+            g.star_apply(u, out)
+        else:
+            g.residual(f, u, out)
+        results.append((got(u, ncomp), None if call == "fill" else got(out, ncomp),
+                        None if call == "fill" else dd.two_norm(out)))
+        u.free()
+    f.free()
+    out.free()
+    squares = [0.0, 0.0]
+    out = R.DeviceArray(dd.shape(1), t)
+    for c in range(ncomp):
+        f = fresh(1, [v[:, c:c + 1] for v in f0])
+        for i, call in enumerate(("fill", "apply", "residual")):
+            u = fresh(1, [v[:, c:c + 1] for v in u0])
+            if call == "fill":
+                g.fill_ghost(u)
+            elif call == "apply":
+                g.star_apply(u, out)
+            else:
+                g.residual(f, u, out)
+            for want, have in zip(got(u, 1), results[i][0]):
+                assert np.array_equal(want[:, 0], have[:, c]), (call, c)
+            if call != "fill":
+                for want, have in zip(got(out, 1), results[i][1]):
+                    assert np.array_equal(want[:, 0], have[:, c]), (call, c)
+                squares[i - 1] += dd.two_norm(out) ** 2
+            u.free()
+        f.free()
+    for i in (0, 1):  # and nothing was written elsewhere: the whole results' norms agree
+        assert abs(results[i + 1][2] - np.sqrt(squares[i])) <= 1e-12 * results[i + 1][2]

@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(SIDES ? 384 : 256) ghost_faces_3d(const DevPat
   if (type < 0 || k >= ni * nj) return;
   for (int c = 0; c < L.ncomp; c++) {
     const T G = face_ghost3<T>(L, type, P.orth[20 + s], P.nbr[20 + s], u, p, c, s, k - j * ni, j);
-    at(u, side_cell3(L, p, c, s, -1, k - j * ni, j)) = G;
+    at(component(L, u, p, c), side_cell3(L, 0, 0, s, -1, k - j * ni, j)) = G;
   }
 }
 

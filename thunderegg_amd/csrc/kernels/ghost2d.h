@@ -347,8 +347,7 @@ __device__ __forceinline__ void fill_ring_cell(const int4& r, int s, int t, T* u
   side_xy(s, 0, t, na, &bx, &by);
   const int gx = a == 0 ? (up ? n0 : -1) : bx, gy = a == 0 ? by : (up ? n1 : -1);
   for (int c = 0; c < L.ncomp; c++) {
-    T* uc = u + c * L.cs;
-    auto U = [&](int q, int x, int y) { return at(uc, q * L.ps + (y + 1) * L.sx + x + 1); };
+    auto U = [&](int q, int x, int y) { return at(component(L, u, q, c), (y + 1) * L.sx + x + 1); };
     T v[4] = { T(0), T(0), T(0), T(0) };
     ghost2d_gather<KIND>(r.x, r.y, r.z, s, t, na, nt, [&](int k, int q, int x, int y) { v[k] = U(q, x, y); });
     const T G = ghost2d_combine<T, KIND>(r.x, r.y, t, nt,
@@ -358,7 +357,7 @@ __device__ __forceinline__ void fill_ring_cell(const int4& r, int s, int t, T* u
                                            return U(p, x, y);
                                          },
                                          v);
-    at(uc, p * L.ps + (gy + 1) * L.sx + gx + 1) = G;
+    at(component(L, u, p, c), (gy + 1) * L.sx + gx + 1) = G;
   }
 }
 

@@ -24,7 +24,9 @@ __device__ __forceinline__ T face_ghost3(const Layout& L, int type, int orth, co
                                          int s, int i, int j)
 {
   const int a = s >> 1, ni = L.n[a == 0 ? 1 : 0], nj = L.n[a == 2 ? 1 : 2];
-  auto U = [&](int qq, int side, int ii, int jj) { return at(u, side_cell3(L, qq, c, side, 0, ii, jj)); };
+  auto U = [&](int qq, int side, int ii, int jj) {
+    return at(component(L, u, qq, c), side_cell3(L, 0, 0, side, 0, ii, jj));
+  };
   if (type == 0) return U(q[0], s ^ 1, i, j);
   T G = T(0);
   if (type == 1) {
@@ -75,7 +77,7 @@ __device__ __forceinline__ void fill_faces3(const Layout& L, const DevPatch& P, 
       for (int s = 0; s < 6; s++) {
         if (k >= cells[s]) continue;
         const int ni = L.n[s < 2 ? 1 : 0], j = k / ni;
-        at(u, side_cell3(L, p, c, s, -1, k - j * ni, j)) = G[s];
+        at(component(L, u, p, c), side_cell3(L, 0, 0, s, -1, k - j * ni, j)) = G[s];
       }
     }
 }

@@ -67,9 +67,10 @@ inline Layout make_layout(int dim, const int* n, int ncomp, int np)
   return L;
 }
 
-// base[idx] for idx >= 0 with the byte offset formed in 32 bits (vectors and tables stay
-// below 2 GiB, checked when domains are created), so a load or store can address from the
-// kernel argument's scalar base plus a 32-bit vector offset instead of a 64-bit vector address.
+// base[idx] for idx >= 0 with the byte offset formed in 32 bits (tables and vectors of one
+// component stay below 2 GiB, checked when domains are created), so a load or store can address
+// from a scalar base plus a 32-bit vector offset instead of a 64-bit vector address.  Vectors of
+// several components reach 16 GiB: there the base is one component of one patch (component).
 template <typename T>
 __device__ __forceinline__ const T& at(const T* base, int idx)
 {
@@ -79,6 +80,13 @@ template <typename T>
 __device__ __forceinline__ T& at(T* base, int idx)
 {
   return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (unsigned)idx * (unsigned)sizeof(T));
+}
+
+// component c of patch p: all its padded values lie within 32-bit offsets of it
+template <typename T>
+__device__ __forceinline__ T* component(const Layout& L, T* u, int p, int c)
+{
+  return u + (p * L.ps + c * L.cs);
 }
 
 // x / d for 0 <= x < 2^31 and a fixed d >= 1 as one high product and a shift
