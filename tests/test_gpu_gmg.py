@@ -232,6 +232,36 @@ def test_patch_bicgstab_shapes(ns, op_kind, neumann):
         assert iters.get().max() <= max_it and iters.get().min() > 0
 
 
+@pytest.mark.parametrize("n", [8, 16])
+@pytest.mark.parametrize("op_kind", [0, 1])
+def test_patch_bicgstab_one_wave(n, op_kind):
+    """The one-wave strips, whose lanes exchange their strips' ends through LDS without a workgroup
+    barrier, on a level with several waves a SIMD: a few iterations do the oracle's arithmetic up
+    to the order of sums, so any exchange that came too early or late shows at once.  The bounds
+    lie above rounding (the operator's condition number, at most 2 (2 n / pi)^2 times the
+    coefficients' ratio of about 20, times the type's epsilon: 1e-12 and 5e-4) and far below a wrong
+    neighbour value's effect."""
+    _print_case("patch-bicgstab-one-wave", n, op_kind)
+    ns = (n, n)
+    lv = solver.uniform_levels(2, 6, ns)[0]
+    od, dd = O.Domain(2, ns, lv), R.Domain(2, ns, lv)
+    g = R.GhostFiller(dd, R.BILINEAR, R.FACES)
+    f0, u0 = random_field(od.shape(1), 45), random_field(od.shape(1), 46)
+    coeffs = np.exp(0.3 * random_field(od.shape(1), 47)) if op_kind else None
+    if op_kind:
+        O.fill_ghost(od, coeffs, kind=R.BILINEAR)
+    for dtype, bound in ((np.float64, 1e-10), (np.float32, 1e-3)):
+        dc = R.DeviceArray.from_host(coeffs.astype(dtype)) if op_kind else None
+        for its in (1, 2, 4):
+            uref = u0.copy()
+            O.bicgstab_smooth(od, f0.copy(), uref, kind=R.BILINEAR, op_kind=op_kind, neumann=False, coeffs=coeffs,
+                              max_it=its, tol=1e-12)
+            du = R.DeviceArray.from_host(u0.astype(dtype))
+            g.patch_bicgstab_smooth(R.DeviceArray.from_host(f0.astype(dtype)), du, op_kind=op_kind, coeffs=dc,
+                                    max_it=its, tol=1e-12, continue_on_breakdown=True)
+            assert relerr(mesh.interior(du.get(), 2), mesh.interior(uref, 2)) <= bound, (dtype, its)
+
+
 def test_varpoisson_gmg():
     _print_case("varpoisson-gmg")
     ns = (16, 16)

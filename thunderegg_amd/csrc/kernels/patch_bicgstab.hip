@@ -17,7 +17,7 @@
 //  - square 2D patches of 8, 16 and 32 cells a side run patch_bicgstab_tile, whose threads own
 //    strips of a column: x neighbours come from the adjacent lanes, y neighbours from registers,
 //    only the strip ends cross LDS, and VarPoisson's face weights stay in registers; 8 and 16
-//    are one wave without any barrier.  Every other shape runs patch_bicgstab_kernel, whose
+//    are one wave without any barrier (wave_sync orders their LDS exchanges).  Every other shape runs patch_bicgstab_kernel, whose
 //    operand passes through a padded LDS patch.
 // Measured against one 256-thread workgroup per patch for every shape, with cross-lane shuffles,
 // the operand in LDS and the cells' places worked out in every apply: 64 patches of 32^2 in FP64
@@ -26,6 +26,7 @@
 // 256: 1.1 to 1.3 times slower (more cells per thread; more waves to sum).
 #include "../te_internal.h"
 #include "blas.h"
+#include "ghost2d.h"
 
 namespace te {
 namespace {
@@ -64,7 +65,8 @@ __device__ __forceinline__ double wave_sum63(double v)
 
 // sums over the workgroup of NV values per thread, returned to every thread; `buf` alternates
 // between the two halves of `red` from call to call, so that a call's writes cannot meet the
-// previous call's reads and one barrier suffices (the one before it orders the call before)
+// previous call's reads and one barrier suffices (the one before it orders the call before).
+// Every call orders the LDS accesses before it before those after it, in one wave too.
 template <int NV, int NT>
 __device__ __forceinline__ void wg_sums(double (&v)[NV], double (*red)[3 * (NT / 64)], int& buf)
 {
@@ -76,6 +78,7 @@ __device__ __forceinline__ void wg_sums(double (&v)[NV], double (*red)[3 * (NT /
     for (int j = 0; j < NV; j++)
       v[j] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v[j]), 63),
                               __builtin_amdgcn_readlane(__double2loint(v[j]), 63));
+    wave_sync();
     return;
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
