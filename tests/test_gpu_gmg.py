@@ -1,6 +1,8 @@
 """GPU parity of the multigrid path against the oracle: the per-patch BiCGStab
 smoother, the V-cycle (GMG::Cycle::apply) and the V-cycle-preconditioned
 BiCGStab solve, FP64 and mixed precision, through the C ABI."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -557,6 +559,37 @@ def test_cycles_and_solves_on_several_streams(ns, level, pre):
         assert np.array_equal(mesh.interior(x.get(), dim), mesh.interior(solved, dim))
         for u, want in zip(us, alone):
             assert np.array_equal(mesh.interior(u.get(), dim), mesh.interior(want, dim))
+
+
+@pytest.mark.parametrize("ns,level", [((16, 16, 16), 4), ((16, 16), 6)])
+def test_first_cycle_on_a_nonblocking_stream(ns, level):
+    """The first cycle of a new hierarchy, enqueued at once on a stream that the null stream does
+    not order: the hierarchy's clearing of its vectors and flags is over when it is created, so the
+    result has the bits of a later cycle."""
+    dim = len(ns)
+    levels = solver.uniform_levels(dim, level, ns)
+    o = dict(filler_kind=R.TRILINEAR if dim == 3 else R.BILINEAR, precision=R.F32, pre_sweeps=2, post_sweeps=1)
+    hip = ctypes.CDLL(R.LIB_PATH)  # its HIP runtime
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0  # hipStreamNonBlocking
+    f = u = None
+    for rep in range(3):
+        g = solver.GMG(dim, ns, levels, **o)
+        if f is None:
+            f = R.DeviceArray.from_host(random_field(g.shape, 73))
+            u = R.DeviceArray(g.shape)
+            u.zero()
+            R.sync()
+            del g
+            g = solver.GMG(dim, ns, levels, **o)
+        R.check(R.lib().te_gmg_vcycle(g.h, f.ptr, u.ptr, stream.value))
+        R.sync(stream.value)
+        first = mesh.interior(u.get(), dim)
+        R.check(R.lib().te_gmg_vcycle(g.h, f.ptr, u.ptr, stream.value))
+        R.sync(stream.value)
+        assert np.array_equal(first, mesh.interior(u.get(), dim)), rep
+        del g
+    assert hip.hipStreamDestroy(stream) == 0
 
 
 @pytest.mark.parametrize("name,n", [("3d_mid_refine_4x4x4_mpi1.json", 8), ("3d_refined_bnw_2x2x2_mpi1.json", 16),

@@ -924,6 +924,9 @@ int te::gmg_create(const te_domain* const* levels, int num_levels, const te_gmg_
       std::memset(g->mirror_h, 0, sizeof(double) * 16);
       e = hipHostGetDevicePointer((void**)&g->mirror_d, g->mirror_h, 0);
     }
+    // the memsets above run on the null stream, which does not order a caller's non-blocking stream
+    // (te_gmg_vcycle runs on its caller's)
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(g->s);
     if (e != hipSuccess) {
       set_error(std::string("te_gmg_create: ") + hipGetErrorString(e));
