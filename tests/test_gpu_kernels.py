@@ -771,6 +771,59 @@ def test_star3_tile(n, off):
                 assert not v.any()  # ghost cells of the output are zero
 
 
+@pytest.mark.parametrize("ns", [(32, 32), (64, 64), (33, 70), (256, 128), (1024, 6), (6, 1024), (16, 16, 16), (32, 32, 32),
+                                (40, 24, 6), (128, 2, 2), (4, 4, 128), (2, 64, 64), (64, 64, 2)])
+def test_patches_of_many_cells(ns):
+    """Few patches of many cells, each shared by several wavefronts or workgroups (runs of rows, of
+    slices, of a patch's values, of its faces' cells; faces in a launch of their own): ghost fill,
+    operators, residual, restriction and interpolation against the oracle."""
+    _print_case("many-cells", ns)
+    dim, odd = len(ns), any(v % 2 for v in ns)
+    name = "3d_refined_bnw_2x2x2_mpi1.json" if dim == 3 else "2d_uniform_2x2_mpi1.json" if odd else "2d_uniform_2x2_refined_nw_mpi1.json"
+    lv = load(name, ns)[1][:2]
+    kind = R.TRILINEAR if dim == 3 else R.BILINEAR
+    of, oc = (O.Domain(dim, ns, v) for v in lv)
+    of.link_parents(oc)
+    df, dc = (R.Domain(dim, ns, v) for v in lv)
+    link, g = R.LevelLink(df, dc), R.GhostFiller(df, kind, R.FACES)
+    beta = np.exp(0.3 * random_field(of.shape(1), 70))
+    O.fill_ghost(of, beta, kind=kind)
+    for dtype, t64, t32 in ((R.F64, TOL64, None), (R.F32, None, 5e-6)):
+        t, tol = R.np_dtype(dtype), t64 or t32
+        u0, f0, c0 = (random_field(o.shape(2), s, t).astype(np.float64) for o, s in ((of, 71), (of, 72), (oc, 73)))
+        filled = u0.copy()
+        O.fill_ghost(of, filled, kind=kind)
+        du = R.DeviceArray.from_host(u0.astype(t))
+        g.fill_ghost(du)
+        assert relerr(du.get(), filled) <= tol
+        b = beta.astype(t).astype(np.float64)
+        for op, neumann in ((0, False), (0, True), (1, False)):
+            dcf = R.DeviceArray.from_host(b.astype(t)) if op else None
+            du.upload(u0)
+            dr, da = (R.DeviceArray.from_host(np.full(u0.shape, 7, t)) for _ in range(2))
+            g.residual(R.DeviceArray.from_host(f0.astype(t)), du, dr, op_kind=op, neumann=neumann, coeffs=dcf)
+            assert relerr(du.get(), filled) <= tol
+            du.upload(u0)
+            g.varstar_apply(dcf, du, da) if op else g.star_apply(du, da, neumann=neumann)
+            assert relerr(du.get(), filled) <= tol
+            for c in range(2):
+                one = np.ascontiguousarray(u0[:, c:c + 1])
+                want = O.varpoisson_apply(of, b, one, kind=kind) if op else O.poisson_apply(of, one, kind=kind, neumann=neumann)
+                assert relerr(da.get()[:, c:c + 1], want) <= tol
+                r = np.zeros(want.shape)
+                mesh.interior(r, dim)[...] = mesh.interior(f0[:, c:c + 1] - want, dim)
+                assert relerr(dr.get()[:, c:c + 1], r) <= tol
+        fref = f0.copy()
+        O.interpolate(oc, of, c0, fref)
+        dfv, dcv = R.DeviceArray.from_host(f0.astype(t)), R.DeviceArray.from_host(c0.astype(t))
+        link.interpolate(dcv, dfv)
+        assert relerr(dfv.get(), fref) <= (TOL64 if t64 else TOL32)
+        if not odd:
+            dfv.upload(f0)
+            link.restrict(dfv, dcv)
+            assert relerr(dcv.get(), O.restrict(of, oc, f0)) <= (TOL64 if t64 else TOL32)
+
+
 @pytest.mark.parametrize("ns,level,ncomp,dtype", [
     ((16, 16, 16), 5, 3, R.F64), ((16, 16, 16), 5, 8, R.F32), ((12, 12, 12), 5, 8, R.F64), ((64, 64), 7, 8, R.F64)])
 def test_vectors_past_4_gib(ns, level, ncomp, dtype):

@@ -85,6 +85,14 @@ int cu_count()
   return v;
 }
 
+int patch_split(int np, long items, int pass, int waves, long most)
+{
+  const long full = 16L * cu_count();
+  int s = 0;
+  while ((items >> s) > 2L * pass && ((long)np << s) * waves < full && (2L << s) <= most && s < 16) s++;
+  return s;
+}
+
 int resident_blocks(const void* kernel, int block, size_t shmem)
 {
   static std::mutex mu;

@@ -73,17 +73,22 @@ __global__ void ghost_corners_2d(const DevPatch* __restrict__ dp, T* __restrict_
   }
 }
 
-// 3D faces: one workgroup per patch, so that the patch's neighbour records are wave-uniform and a
-// cell's place on the face takes one division.  SIDES (faces of at most 64 cells): a wave per
-// side; else each thread takes the same cell of all six sides (fill_faces3).
+// 3D faces: a workgroup per patch or part of its faces' cells, so that the patch's neighbour records
+// are wave-uniform and a cell's place on the face takes one division.  SIDES (faces of at most 64
+// cells): a wave per side; else each thread takes the same cell of all six sides (fill_faces3).
 template <typename T, bool SIDES>
-__global__ void __launch_bounds__(SIDES ? 384 : 256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L)
+__global__ void __launch_bounds__(SIDES ? 384 : 256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L,
+                                                                    int split)
 {
-  const int p = xcd_item(blockIdx.x, gridDim.x);
+  const int unit = xcd_item(blockIdx.x, gridDim.x), p = unit >> split;
   if (p >= L.np) return;
   const DevPatch& P = dp[p];
   if (!SIDES) {
-    fill_faces3<T>(L, P, u, p, threadIdx.x, blockDim.x);
+    int first[6], last[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+      last[s] = split_range(L.n[s < 2 ? 1 : 0] * L.n[s < 4 ? 2 : 1], split, unit & ((1 << split) - 1), &first[s]);
+    fill_faces3<T>(L, P, u, p, threadIdx.x, blockDim.x, first, last);
     return;
   }
   const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), k = threadIdx.x & 63;
@@ -186,7 +191,7 @@ __global__ void ghost_lowdim_3d(const DevPatch* __restrict__ dp, T* __restrict__
 }
 
 template <typename T>
-int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, hipStream_t s)
+int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, bool lowdim, hipStream_t s)
 {
   const te_domain* d = g->d;
   if (d->np == 0) return TE_OK;
@@ -202,7 +207,7 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, hipStrea
     else
       hipLaunchKernelGGL((ghost_ring_2d<T, TE_BIQUADRATIC>), dim3(grid), dim3(B), 0, s, (const int4*)d->d_ring, u,
                          L);
-    if (g->fill_type == TE_CORNERS) {
+    if (lowdim && g->fill_type == TE_CORNERS) {
       int cg = (d->np * 4 + B - 1) / B;
       if (g->kind == TE_BILINEAR)
         hipLaunchKernelGGL((ghost_corners_2d<T, TE_BILINEAR>), dim3(cg), dim3(B), 0, s, d->d_patches, u, L);
@@ -213,11 +218,13 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, hipStrea
     int face = 0;  // cells of the largest face: a thread each, up to 256
     for (int a = 0; a < 3; a++) face = std::max(face, d->ns[a] * d->ns[(a + 1) % 3]);
     if (faces && face <= 64)
-      hipLaunchKernelGGL((ghost_faces_3d<T, true>), dim3(xcd_grid(d->np)), dim3(384), 0, s, d->d_patches, u, L);
-    else if (faces)
-      hipLaunchKernelGGL((ghost_faces_3d<T, false>), dim3(xcd_grid(d->np)), dim3(std::min(256, (face + 63) / 64 * 64)),
-                         0, s, d->d_patches, u, L);
-    if (g->fill_type != TE_FACES) {
+      hipLaunchKernelGGL((ghost_faces_3d<T, true>), dim3(xcd_grid(d->np)), dim3(384), 0, s, d->d_patches, u, L, 0);
+    else if (faces) {
+      const int block = std::min(256, (face + 63) / 64 * 64), split = patch_split(d->np, face, block, block / 64, face);
+      hipLaunchKernelGGL((ghost_faces_3d<T, false>), dim3(xcd_grid(d->np << split)), dim3(block), 0, s, d->d_patches, u,
+                         L, split);
+    }
+    if (lowdim && g->fill_type != TE_FACES) {
       int tmax = d->ns[0];
       for (int a = 1; a < 3; a++) tmax = d->ns[a] > tmax ? d->ns[a] : tmax;
       long tl = (long)d->np * (12 * tmax + 8);
@@ -234,16 +241,23 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, hipStrea
 
 int launch_ghost_fill(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s)
 {
-  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, true, s);
-  return ghost_fill_t<float>(g, (float*)u, ncomp, true, s);
+  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, true, true, s);
+  return ghost_fill_t<float>(g, (float*)u, ncomp, true, true, s);
+}
+
+// the face ghosts alone
+int launch_ghost_fill_faces(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s)
+{
+  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, true, false, s);
+  return ghost_fill_t<float>(g, (float*)u, ncomp, true, false, s);
 }
 
 // the edge and corner ghosts alone (nothing for fill type Faces)
 int launch_ghost_fill_lowdim(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s)
 {
   if (g->fill_type == TE_FACES) return TE_OK;
-  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, false, s);
-  return ghost_fill_t<float>(g, (float*)u, ncomp, false, s);
+  if (dtype == TE_F64) return ghost_fill_t<double>(g, (double*)u, ncomp, false, true, s);
+  return ghost_fill_t<float>(g, (float*)u, ncomp, false, true, s);
 }
 
 }  // namespace te

@@ -52,31 +52,32 @@ __device__ __forceinline__ T face_ghost3(const Layout& L, int type, int orth, co
   return G;
 }
 
-// The face ghosts of patch p, by the nt threads t = 0 .. nt - 1: each thread
-// takes the same cell of all six sides, so that their loads are in flight together.
+// The face ghosts first[s] <= k < last[s] of each side s of patch p (k: the face's cells, first
+// free axis fastest), by the nt threads t = 0 .. nt - 1: each thread takes a cell of all six sides
+// at a time, so that their loads are in flight together.
 template <typename T>
-__device__ __forceinline__ void fill_faces3(const Layout& L, const DevPatch& P, T* u, int p, int t, int nt)
+__device__ __forceinline__ void fill_faces3(const Layout& L, const DevPatch& P, T* u, int p, int t, int nt,
+                                            const int (&first)[6], const int (&last)[6])
 {
   int cells[6], most = 0;
 #pragma unroll
   for (int s = 0; s < 6; s++) {
-    const int a = s >> 1;
-    cells[s] = P.type[20 + s] < 0 ? 0 : L.n[a == 0 ? 1 : 0] * L.n[a == 2 ? 1 : 2];
+    cells[s] = P.type[20 + s] < 0 ? 0 : last[s] - first[s];
     most = cells[s] > most ? cells[s] : most;
   }
   for (int c = 0; c < L.ncomp; c++)
-    for (int k = t; k < most; k += nt) {
+    for (int i = t; i < most; i += nt) {
       T G[6];
 #pragma unroll
       for (int s = 0; s < 6; s++) {
-        if (k >= cells[s]) continue;
-        const int ni = L.n[s < 2 ? 1 : 0], j = k / ni;
+        if (i >= cells[s]) continue;
+        const int ni = L.n[s < 2 ? 1 : 0], k = first[s] + i, j = k / ni;
         G[s] = face_ghost3<T>(L, P.type[20 + s], P.orth[20 + s], P.nbr[20 + s], u, p, c, s, k - j * ni, j);
       }
 #pragma unroll
       for (int s = 0; s < 6; s++) {
-        if (k >= cells[s]) continue;
-        const int ni = L.n[s < 2 ? 1 : 0], j = k / ni;
+        if (i >= cells[s]) continue;
+        const int ni = L.n[s < 2 ? 1 : 0], k = first[s] + i, j = k / ni;
         at(component(L, u, p, c), side_cell3(L, 0, 0, s, -1, k - j * ni, j)) = G[s];
       }
     }

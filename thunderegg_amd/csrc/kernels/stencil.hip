@@ -5,6 +5,8 @@
 // of the output are written 0 (f.setWithGhost(0), PatchOperator.h:136), interior cells get
 // the stencil.  Physical-boundary ghosts of u are applied inline
 // (enforceBoundaryConditions, :115-144): -u (Dirichlet) or +u (Neumann).
+#include <algorithm>
+
 #include "../te_internal.h"
 #include "dft.h"
 #include "ghost2d.h"
@@ -15,44 +17,67 @@ namespace {
 
 constexpr int kNoFill = -1;
 
-// One patch per workgroup (3D) or per wavefront (2D), so that its neighbour records and spacings
-// are wave-uniform and a cell's place takes one or two multiply-shift divisions.  FILL (a
-// te_filler_kind): the patch's own side ghosts first, written to u for the caller; they depend
-// on interior cells only, so no patch waits for another's, and the stencil then reads them back
-// from this workgroup's cache.  The stencil runs over the padded patch in groups of V = 2
+// One patch, or a run of its slices (3D) or rows (2D), per workgroup (3D) or wavefront (2D), so that
+// its neighbour records and spacings are wave-uniform and a cell's place takes one or two
+// multiply-shift divisions.  FILL (a te_filler_kind): the side ghosts next to the unit's cells
+// first, written to u for the caller; they depend on interior cells only, so no unit waits for
+// another's, and the stencil then reads them back from this workgroup's cache.  The stencil runs over the padded patch in groups of V = 2
 // values (rows of even length start on them): one 16-byte (FP64) or 8-byte access per row
 // neighbour and for the output, kStarItems groups in flight a thread.  Patches go to the XCDs in
 // contiguous eighths (xcd_item), which takes 9 to 10 us off both cases below: the ghost phase
 // reads most of the neighbours' lines.
-// A u with ghosts, two launches of one thread per cell before / this one: 2,535 patches of 16^3
-// (refined octree, FP32) 117 / 45 us, of which the stencil alone 74 / 26 (a copy of the padded
-// vector takes 23); 19,543 patches of 16^2 (refined quadtree, FP64) 56 / 30 us.
+// A u with ghosts, two launches of one thread per cell before / this one, vectors rotated so that
+// the caches do not keep them: 4,096 patches of 16^3 in FP64 240 / 157 us (a copy of the padded
+// vector 110), VarPoisson in FP32 209 / 133; 65,536 patches of 16^2 in FP64 (one set of vectors)
+// 203 / 104, VarPoisson 248 / 143; few patches: 64 of 32^2 8.0 / 4.4, 4 of 1024^2 59 / 27.
 // Marching each thread along z (three rows' loads together) was 3 to 4 us slower in 3D.
 constexpr int kStarItems = 2;
+// 3D faces (z) of more cells are filled by a launch of their own where a patch is split: one unit
+// would fill such a face alone (64^3: 16 passes of its threads; 32^3: 4)
+constexpr int kFusedFace = 1024;
 
 template <typename T, typename TF, typename TO, int D, int OP, int FILL, int V>
-__global__ void __launch_bounds__(D == 2 ? 256 : 1024) star_kernel(const DevPatch* __restrict__ dp, const int4* __restrict__ ring, T* u,
+__global__ void __launch_bounds__(256) star_kernel(const DevPatch* __restrict__ dp, const int4* __restrict__ ring, T* u,
                                                    const T* __restrict__ cf, const TF* __restrict__ fin,
                                                    TO* __restrict__ out, Layout L, int neumann, FastDiv per_row,
-                                                   FastDiv rows)
+                                                   FastDiv rows, int split)
 {
   constexpr bool WAVE = D == 2;
   const int b = xcd_item(blockIdx.x, gridDim.x);
-  const int p = WAVE ? __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6)) : b;
+  const int unit = WAVE ? __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6)) : b;
+  const int p = unit >> split, part = unit & ((1 << split) - 1);
   if (p >= L.np) return;
   const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
+  const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1;
+  const int per = (n0 + 2) / V;
   const DevPatch& P = dp[p];
-  if (FILL != kNoFill) {
+  int first, last;  // the unit's groups
+  if (FILL == kNoFill) {
+    last = split_range(per * (n1 + 2) * (D == 3 ? n2 + 2 : 1), split, part, &first);
+  } else {
+    // whole rows (2D) or slices (3D), lo <= r < hi of the interior ones
+    const int nr = D == 3 ? n2 : n1, group = D == 3 ? per * (n1 + 2) : per;
+    last = split_range(nr + 2, split, part, &first);
+    const int lo = max(first, 1) - 1, hi = min(last, nr + 1) - 1;
+    const bool low = lo == 0 && hi > lo, high = hi == nr && hi > lo;
+    first *= group;
+    last *= group;
     if (D == 2) {
-      const int nr = 2 * (L.n[0] + L.n[1]);
-      for (int g = t; g < nr; g += 64) {
+      // ring cells: west and east of the rows, then south and north where they are the unit's
+      const int m = max(hi - lo, 0), sides = 2 * m + (low ? n0 : 0) + (high ? n0 : 0);
+      for (int i = t; i < sides; i += 64) {
+        int g = i - 2 * m + 2 * n1 + (low ? 0 : n0);
+        if (i < m) g = lo + i;
+        else if (i < 2 * m) g = n1 + lo + i - m;
         int s, tt;
-        const int4 r = ring[ring_index(p, g, L.n[0], L.n[1], &s, &tt)];
+        const int4 r = ring[ring_index(p, g, n0, n1, &s, &tt)];
         if (r.x >= 0) fill_ring_cell<T, FILL == TE_BILINEAR ? TE_BILINEAR : TE_BIQUADRATIC>(r, s, tt, u, L, p);
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // one wave wrote what it reads below
     } else {
-      fill_faces3<T>(L, P, u, p, t, nt);
+      const int f0[6] = { lo * n1, lo * n1, lo * n0, lo * n0, 0, 0 };
+      const int f1[6] = { hi * n1, hi * n1, hi * n0, hi * n0, low ? n0 * n1 : 0, high ? n0 * n1 : 0 };
+      fill_faces3<T>(L, P, u, p, t, nt, f0, f1);
       __syncthreads();
     }
   }
@@ -66,27 +91,38 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) star_kernel(const DevPatc
     phys[2 * a + 1] = P.type[SB + 2 * a + 1] < 0;
   }
   const T bs = (OP == 0 && neumann) ? T(1) : T(-1);
-  const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1;
-  const int per = (n0 + 2) / V, items = per * (n1 + 2) * (D == 3 ? n2 + 2 : 1);
   for (int c = 0; c < L.ncomp; c++) {
     const int base = p * L.ps + c * L.cs, cbase = p * L.cs;
-    for (int i0 = t; i0 < items; i0 += kStarItems * nt) {
-      // row neighbours of a group: below / above along y and z; single values left and right of it
-      T m[kStarItems][V], yl[kStarItems][V], yu[kStarItems][V], zl[kStarItems][V], zu[kStarItems][V];
-      T lf[kStarItems], rt[kStarItems];
+    for (int i0 = first + t; i0 < last; i0 += kStarItems * nt) {
+      // a group and its row neighbours: below / above along y and z; single values left and right of it
+      struct Cells {
+        T m[V], yl[V], yu[V], zl[V], zu[V], lf, rt;
+      };
+      Cells U[kStarItems], C[OP == 1 ? kStarItems : 1];  // u, and the coefficients
       TF fv[kStarItems][V];
       int xx[kStarItems], yy[kStarItems], zz[kStarItems];
       bool in[kStarItems];
       auto load = [](auto& dst, const auto* src) {
         typedef typename std::remove_const<typename std::remove_reference<decltype(*src)>::type>::type E;
         if (V == 2) {
-          typedef E E2 __attribute__((ext_vector_type(2)));
+          typedef E E2 __attribute__((ext_vector_type(2), aligned(sizeof(E))));
           const E2 v = *reinterpret_cast<const E2*>(src);
           dst[0] = v[0];
           dst[V - 1] = v[1];
         } else {
           dst[0] = *src;
         }
+      };
+      auto cells = [&](Cells& d, const T* q) {
+        load(d.m, q);
+        load(d.yl, q - L.sx);
+        load(d.yu, q + L.sx);
+        if (D == 3) {
+          load(d.zl, q - L.sy);
+          load(d.zu, q + L.sy);
+        }
+        d.lf = q[-1];
+        d.rt = q[V];
       };
 #pragma unroll
       for (int k = 0; k < kStarItems; k++) {
@@ -95,48 +131,43 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) star_kernel(const DevPatc
         zz[k] = D == 3 ? rows(row) : 1;
         yy[k] = D == 3 ? row - zz[k] * (n1 + 2) : row;
         xx[k] = V * (i - row * per) - 1;
-        in[k] = i < items && yy[k] >= 1 && yy[k] <= n1 && zz[k] >= 1 && zz[k] <= n2;
+        in[k] = i < last && yy[k] >= 1 && yy[k] <= n1 && zz[k] >= 1 && zz[k] <= n2;
         if (V == 1) in[k] = in[k] && xx[k] >= 0 && xx[k] < n0;
         if (!in[k]) continue;
-        const T* q = u + base + V * i;
-        load(m[k], q);
-        load(yl[k], q - L.sx);
-        load(yu[k], q + L.sx);
-        if (D == 3) {
-          load(zl[k], q - L.sy);
-          load(zu[k], q + L.sy);
-        }
-        lf[k] = q[-1];
-        rt[k] = q[V];
+        cells(U[k], u + base + V * i);
+        if (OP == 1) cells(C[OP == 1 ? k : 0], cf + cbase + V * i);
         if (fin) load(fv[k], fin + base + V * i);
       }
 #pragma unroll
       for (int k = 0; k < kStarItems; k++) {
         const int i = i0 + k * nt;
-        if (i >= items) continue;
+        if (i >= last) continue;
         TO res[V];
 #pragma unroll
         for (int j = 0; j < V; j++) {
           res[j] = TO(0);
           const int x = xx[k] + j;
           if (!in[k] || x < 0 || x >= n0) continue;
-          const T mid = m[k][j];
+          const Cells& u_ = U[k];
+          const Cells& c_ = C[OP == 1 ? k : 0];
+          const T mid = u_.m[j];
           const T bc = bs * mid;
           T acc = T(0);
-          auto axis = [&](int a, T lower, T upper, int cells, int at0, int st) {
+          auto axis = [&](int a, T lower, T upper, T cl, T cu, int cells, int at0) {
             if (at0 == 0 && phys[2 * a]) lower = bc;
             if (at0 == cells - 1 && phys[2 * a + 1]) upper = bc;
             if (OP == 0) {
               acc += (upper - T(2) * mid + lower) * ih2[a];
             } else {
-              const int ci = cbase + V * i + j;
-              const T cm = at(cf, ci), cl = at(cf, ci - st), cu = at(cf, ci + st);
+              const T cm = c_.m[j];
               acc += ((cu + cm) * (upper - mid) - (cl + cm) * (mid - lower)) * (ih2[a] * T(0.5));
             }
           };
-          axis(0, j == 0 ? lf[k] : m[k][0], j == V - 1 ? rt[k] : m[k][V - 1], n0, x, 1);
-          axis(1, yl[k][j], yu[k][j], n1, yy[k] - 1, L.sx);
-          if (D == 3) axis(D - 1, zl[k][j], zu[k][j], n2, zz[k] - 1, L.sy);
+          auto left = [&](const Cells& q) { return j == 0 ? q.lf : q.m[0]; };
+          auto right = [&](const Cells& q) { return j == V - 1 ? q.rt : q.m[V - 1]; };
+          axis(0, left(u_), right(u_), left(c_), right(c_), n0, x);
+          axis(1, u_.yl[j], u_.yu[j], c_.yl[j], c_.yu[j], n1, yy[k] - 1);
+          if (D == 3) axis(D - 1, u_.zl[j], u_.zu[j], c_.zl[j], c_.zu[j], n2, zz[k] - 1);
           res[j] = fin ? TO(T(fv[k][j]) - acc) : TO(acc);
         }
         TO* o = out + base + V * i;
@@ -160,11 +191,12 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) star_kernel(const DevPatc
 // result at a time, its z and y neighbours by wide LDS reads.  star_kernel above reads each cell
 // seven times through the vector L1 and its stencil waits for the ghosts' stores; here it waits
 // for LDS only.  Bound by memory.  Operator / residual with the ghost fill, star_kernel -> this
-// one, us: 2,535 patches of 16^3 (refined octree, FP32) 62 / 70 -> 39 / 43 (a torch copy of the
-// vector takes 17); 4,096 of 16^3 in FP32 69 / 104 -> 56 / 83, VarPoisson in FP64 348 / 377 ->
-// 213 / 224; 4,096 of 8^3 in FP32 21.6 / 23 -> 12.3 / 14.3, in FP64 32 / 32 -> 20 / 24; 512 of
-// 8^3 6.7 -> 5.5.  Not for 16^3 Poisson in FP64 (149 / 175 against 149 / 186: three workgroups of
-// 46 KB a CU) and VarPoisson in FP32 (161 / 182 against 170 / 184: bound by the coefficients' reads).
+// one, us, vectors rotated so that the caches do not keep them: 2,500 patches of 16^3 (refined
+// octree, FP32) 60 / 75 -> 51 / 62 (a copy of the padded vector 25); 4,096 of 16^3 in FP32 91 / 111
+// -> 79 / 91, VarPoisson in FP64 226 / 236 -> 213 / 224; 4,096 of 8^3 in FP32 23.7 / 23.8 -> 13.0 /
+// 14.7, in FP64 33 / 41 -> 20 / 29; 512 of 8^3 6.9 -> 5.2.  Not for 16^3 Poisson in FP64 (157 / 178
+// against 163 / 189: three workgroups of 46 KB a CU) and VarPoisson in FP32 (133 / 142 against 152 /
+// 157: its coefficients are read cell by cell here).
 template <typename T, typename TF, typename TO, int OP, int N>
 __global__ void __launch_bounds__(N == 16 ? 256 : 64) star3_tile_kernel(const DevPatch* __restrict__ dp, T* u,
                                                                         const T* __restrict__ cf,
@@ -243,7 +275,7 @@ __global__ void __launch_bounds__(N == 16 ? 256 : 64) star3_tile_kernel(const De
 }
 
 template <typename T, typename TF, typename TO, int D, int OP>
-void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* out, int ncomp, int neumann, bool fill,
+int launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* out, int ncomp, int neumann, bool fill,
                 hipStream_t s)
 {
   const te_domain* d = g->d;
@@ -252,16 +284,17 @@ void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* 
   // patches only where it is the faster one (its comment)
   if constexpr (D == 3) {
     const bool cube = L.n[1] == L.n[0] && L.n[2] == L.n[0];
-    if (fill && d->np > 256 && cube && L.n[0] == 8) {
+    const bool tile = fill && cube && d->np > cu_count();
+    if (tile && L.n[0] == 8) {
       hipLaunchKernelGGL((star3_tile_kernel<T, TF, TO, OP, 8>), dim3(xcd_grid(d->np), ncomp), dim3(64), 0, s,
                          d->d_patches, u, cf, fin, out, L, neumann);
-      return;
+      return TE_OK;
     }
     if constexpr ((OP == 0) == (sizeof(T) == 4)) {
-      if (fill && d->np > 256 && cube && L.n[0] == 16) {
+      if (tile && L.n[0] == 16) {
         hipLaunchKernelGGL((star3_tile_kernel<T, TF, TO, OP, 16>), dim3(xcd_grid(d->np), ncomp), dim3(256), 0, s,
                            d->d_patches, u, cf, fin, out, L, neumann);
-        return;
+        return TE_OK;
       }
     }
   }
@@ -269,11 +302,20 @@ void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* 
                      (uintptr_t)out % (2 * sizeof(TO)) == 0;
   const int V = pairs ? 2 : 1, per = (L.n[0] + 2) / V;
   const int items = per * (L.n[1] + 2) * (D == 3 ? L.n[2] + 2 : 1);
-  const int block = D == 2 ? 256 : patch_block(items / kStarItems, d->np);
-  const int grid = xcd_grid(D == 2 ? (d->np + 3) / 4 : d->np);
+  const int block = D == 2 ? 256 : std::min(256, (items / kStarItems + 63) / 64 * 64);
+  // the unit: a wave in 2D, the workgroup in 3D
+  const int threads = D == 2 ? 64 : block, pass = threads * kStarItems;
+  int split = patch_split(d->np, items, pass, threads / 64, fill ? (D == 3 ? L.n[2] : L.n[1]) + 2 : items);
+  if (fill && D == 3 && split > 0 && L.n[0] * L.n[1] > kFusedFace) {
+    int rc = launch_ghost_fill_faces(g, sizeof(T) == 8 ? TE_F64 : TE_F32, u, ncomp, s);
+    if (rc) return rc;
+    fill = false;
+    split = patch_split(d->np, items, pass, threads / 64, items);
+  }
+  const int units = d->np << split, grid = xcd_grid(D == 2 ? (units + 3) / 4 : units);
 #define TE_ST(F_, V_)                                                                                               \
   hipLaunchKernelGGL((star_kernel<T, TF, TO, D, OP, F_, V_>), dim3(grid), dim3(block), 0, s, d->d_patches,          \
-                     (const int4*)d->d_ring, u, cf, fin, out, L, neumann, FastDiv(per), FastDiv(L.n[1] + 2))
+                     (const int4*)d->d_ring, u, cf, fin, out, L, neumann, FastDiv(per), FastDiv(L.n[1] + 2), split)
 #define TE_SF(F_)          \
   do {                     \
     if (V == 2) TE_ST(F_, 2); \
@@ -285,19 +327,19 @@ void launch_one(const te_ghost_filler* g, T* u, const T* cf, const TF* fin, TO* 
   else TE_SF((D == 2 ? TE_BIQUADRATIC : kNoFill));
 #undef TE_SF
 #undef TE_ST
+  return TE_OK;
 }
 
 template <typename T, typename TF, typename TO>
-void launch_dim(const te_ghost_filler* g, int op_kind, T* u, const T* cf, const TF* fin, TO* out, int ncomp,
+int launch_dim(const te_ghost_filler* g, int op_kind, T* u, const T* cf, const TF* fin, TO* out, int ncomp,
                 int neumann, bool fill, hipStream_t s)
 {
   if (g->d->dim == 2) {
-    if (op_kind == 0) launch_one<T, TF, TO, 2, 0>(g, u, cf, fin, out, ncomp, neumann, fill, s);
-    else launch_one<T, TF, TO, 2, 1>(g, u, cf, fin, out, ncomp, neumann, fill, s);
-  } else {
-    if (op_kind == 0) launch_one<T, TF, TO, 3, 0>(g, u, cf, fin, out, ncomp, neumann, fill, s);
-    else launch_one<T, TF, TO, 3, 1>(g, u, cf, fin, out, ncomp, neumann, fill, s);
+    if (op_kind == 0) return launch_one<T, TF, TO, 2, 0>(g, u, cf, fin, out, ncomp, neumann, fill, s);
+    return launch_one<T, TF, TO, 2, 1>(g, u, cf, fin, out, ncomp, neumann, fill, s);
   }
+  if (op_kind == 0) return launch_one<T, TF, TO, 3, 0>(g, u, cf, fin, out, ncomp, neumann, fill, s);
+  return launch_one<T, TF, TO, 3, 1>(g, u, cf, fin, out, ncomp, neumann, fill, s);
 }
 
 // Cycle::restrict (GMG/Cycle.h:57-65) of 3D patches of N^3 cells in one launch: a workgroup stages
@@ -450,23 +492,25 @@ int launch_star(const te_ghost_filler* g, int dt, int dtf, int dto, int op_kind,
                 const void* fin, void* u, void* out, int ncomp, bool fill, hipStream_t s)
 {
   if (g->d->np == 0) return TE_OK;
+  int rc = TE_OK;
   if (fill) {
-    int rc = launch_ghost_fill_lowdim(g, dt, u, ncomp, s);
+    rc = launch_ghost_fill_lowdim(g, dt, u, ncomp, s);
     if (rc) return rc;
   }
   if (dt == TE_F64 && dtf == TE_F64 && dto == TE_F64)
-    launch_dim<double, double, double>(g, op_kind, (double*)u, (const double*)coeffs, (const double*)fin, (double*)out,
+    rc = launch_dim<double, double, double>(g, op_kind, (double*)u, (const double*)coeffs, (const double*)fin, (double*)out,
                                        ncomp, neumann, fill, s);
   else if (dt == TE_F32 && dtf == TE_F32 && dto == TE_F32)
-    launch_dim<float, float, float>(g, op_kind, (float*)u, (const float*)coeffs, (const float*)fin, (float*)out, ncomp,
+    rc = launch_dim<float, float, float>(g, op_kind, (float*)u, (const float*)coeffs, (const float*)fin, (float*)out, ncomp,
                                     neumann, fill, s);
   else if (dt == TE_F32 && dtf == TE_F64 && dto == TE_F32)
-    launch_dim<float, double, float>(g, op_kind, (float*)u, (const float*)coeffs, (const double*)fin, (float*)out,
+    rc = launch_dim<float, double, float>(g, op_kind, (float*)u, (const float*)coeffs, (const double*)fin, (float*)out,
                                      ncomp, neumann, fill, s);
   else {
     set_error("unsupported dtype combination for the star stencil");
     return TE_ERR_UNSUPPORTED;
   }
+  if (rc) return rc;
   TE_HIP(hipGetLastError());
   return TE_OK;
 }

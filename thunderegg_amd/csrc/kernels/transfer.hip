@@ -11,6 +11,8 @@
 //  - DirectInterpolator (GMG/DirectInterpolator.h:60-91): fine[i] += coarse[(i+s)/2].
 // Children of a coarse patch are visited in increasing fine local index and fine
 // cells in x-fastest order, the order in which the reference accumulates them.
+#include <algorithm>
+
 #include "../te_internal.h"
 #include "ghost2d.h"
 
@@ -177,23 +179,27 @@ __device__ __forceinline__ void store_at(T* q, Get get)
   }
 }
 
-// One patch per workgroup (3D) or wavefront (2D) in both kernels below, so that the link's
-// records are wave-uniform, and pairs of values along rows (even cells per side).
+// One patch, or a run of its values, per workgroup (3D) or wavefront (2D) in both kernels below, so
+// that the link's records are wave-uniform, and pairs of values along rows (even cells per side).
+// Bound by memory on large levels.  One thread per cell with its place found by divisions -> these,
+// us, FP64, restriction / interpolation: 4,096 fine patches of 16^3 81 / 90 -> 29 / 56; 65,536 of
+// 16^2 79 / 76 -> 30 / 59; 64 of 64^2 4.7 / 4.2 -> 4.1 / 4.1 (16 / 9.5 with one wave a patch).
 
 // Restriction where every coarse cell has one child over it (te_level_link::regular): a thread
 // forms the two coarse cells of an aligned pair, each from 2^(D - 1) accesses of two fine cells,
 // in the order of the general kernel above.
 template <typename TI, typename TO, int D>
-__global__ void __launch_bounds__(D == 2 ? 256 : 1024) restrict_regular_kernel(const int32_t* __restrict__ child,
+__global__ void __launch_bounds__(256) restrict_regular_kernel(const int32_t* __restrict__ child,
                                                                const int32_t* __restrict__ orth,
                                                                const TI* __restrict__ fine, TO* __restrict__ coarse,
-                                                               Layout L, int np_coarse, FastDiv per_row, FastDiv rows)
+                                                               Layout L, int np_coarse, FastDiv per_row, FastDiv rows,
+                                                               int split)
 {
   constexpr bool WAVE = D == 2;
   __shared__ int tabs[4][8], copies[4];  // the child of each octant (-1: none), or a copied child in entry 0
   const int b = xcd_item(blockIdx.x, gridDim.x);
   const int w = WAVE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-  const int p = WAVE ? b * 4 + w : b;
+  const int unit = WAVE ? b * 4 + w : b, p = unit >> split;
   const bool live = p < np_coarse;
   const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
   // the link's records of the patch by one lane each (entries past the last child are -1)
@@ -209,10 +215,12 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) restrict_regular_kernel(c
   const bool copy = copies[w] != 0;
   if (!live) return;
   const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1, h0 = n0 / 2, h1 = n1 / 2, h2 = n2 / 2;
-  const int per = (n0 + 2) / 2, items = per * (n1 + 2) * (D == 3 ? n2 + 2 : 1);
+  const int per = (n0 + 2) / 2;
+  int first;
+  const int last = split_range(per * (n1 + 2) * (D == 3 ? n2 + 2 : 1), split, unit & ((1 << split) - 1), &first);
   const TI wt = TI(1.0 / (1 << D));
   for (int c = 0; c < L.ncomp; c++) {
-    for (int i = t; i < items; i += nt) {
+    for (int i = first + t; i < last; i += nt) {
       const int row = per_row(i);
       const int Z = D == 3 ? rows(row) - 1 : 0, Y = D == 3 ? row - (Z + 1) * (n1 + 2) - 1 : row - 1;
       const int X0 = 2 * (i - row * per) - 1;
@@ -255,33 +263,38 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) restrict_regular_kernel(c
   }
 }
 
+constexpr int kInterpItems = 2;  // pairs in flight a thread
+
 // DirectInterpolator: fine += the coarse cell over it, over the interior rows of each fine patch
 template <typename TC, typename TF, int D, int V>
-__global__ void __launch_bounds__(D == 2 ? 256 : 1024) interp_kernel(const int32_t* __restrict__ parent,
+__global__ void __launch_bounds__(256) interp_kernel(const int32_t* __restrict__ parent,
                                                      const int32_t* __restrict__ orth, const TC* __restrict__ coarse,
-                                                     TF* __restrict__ fine, Layout L, FastDiv per_row, FastDiv rows)
+                                                     TF* __restrict__ fine, Layout L, FastDiv per_row, FastDiv rows,
+                                                     int split)
 {
   constexpr bool WAVE = D == 2;
-  constexpr int U = 2;  // pairs in flight a thread
+  constexpr int U = kInterpItems;
   const int b = xcd_item(blockIdx.x, gridDim.x);
-  const int p = WAVE ? __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6)) : b;
+  const int unit = WAVE ? __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6)) : b, p = unit >> split;
   if (p >= L.np) return;
   const int t = WAVE ? threadIdx.x & 63 : threadIdx.x, nt = WAVE ? 64 : blockDim.x;
   const int n0 = L.n[0], n1 = L.n[1], n2 = D == 3 ? L.n[2] : 1;
-  const int per = V == 2 ? n0 / 2 + 1 : n0, items = per * n1 * n2;
+  const int per = V == 2 ? n0 / 2 + 1 : n0;
+  int first;
+  const int last = split_range(per * n1 * n2, split, unit & ((1 << split) - 1), &first);
   const int cp = parent[p], o = orth[p], sh = o < 0 ? 0 : 1;
   const int s0 = sh && (o & 1) ? n0 : 0, s1 = sh && (o & 2) ? n1 : 0, s2 = sh && (o & 4) ? n2 : 0;
   for (int c = 0; c < L.ncomp; c++) {
     const TC* cb = coarse + cp * L.ps + c * L.cs;
     TF* fb = fine + p * L.ps + c * L.cs;
-    for (int i0 = t; i0 < items; i0 += U * nt) {
+    for (int i0 = first + t; i0 < last; i0 += U * nt) {
       TF fv[U][V];
       TC cv[U][V];
       int off[U], x0[U];
 #pragma unroll
       for (int k = 0; k < U; k++) {
         const int i = i0 + k * nt;
-        if (i >= items) continue;
+        if (i >= last) continue;
         const int row = per_row(i), z = D == 3 ? rows(row) : 0, y = row - z * n1;
         x0[k] = V == 2 ? 2 * (i - row * per) - 1 : i - row * per;
         const int up = D == 3 ? L.sy : 0;
@@ -297,7 +310,7 @@ __global__ void __launch_bounds__(D == 2 ? 256 : 1024) interp_kernel(const int32
 #pragma unroll
       for (int k = 0; k < U; k++) {
         const int i = i0 + k * nt;
-        if (i >= items) continue;
+        if (i >= last) continue;
 #pragma unroll
         for (int j = 0; j < V; j++) fv[k][j] = TF(fv[k][j] + TF(cv[k][j]));
         if (V == 1 || (x0[k] >= 0 && x0[k] + 1 < n0)) store_at<TF, V>(fb + off[k], [&](int j) { return fv[k][j]; });
@@ -318,13 +331,14 @@ void restrict_t(const te_level_link* l, const TI* fine, TO* coarse, int ncomp, b
   if (!ex && l->regular) {
     const int per = (L.n[0] + 2) / 2, rows = L.n[1] + 2;
     const int items = per * rows * (c->dim == 3 ? L.n[2] + 2 : 1);
+    const int block = c->dim == 2 ? 256 : std::min(256, (items + 63) / 64 * 64), unit = c->dim == 2 ? 64 : block;
+    const int split = patch_split(c->np, items, unit, unit / 64, items), units = c->np << split;
     if (c->dim == 2)
-      hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 2>), dim3(xcd_grid((c->np + 3) / 4)), dim3(256), 0, s,
-                         l->d_child, l->d_orth, fine, coarse, L, c->np, FastDiv(per), FastDiv(rows));
+      hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 2>), dim3(xcd_grid((units + 3) / 4)), dim3(block), 0, s,
+                         l->d_child, l->d_orth, fine, coarse, L, c->np, FastDiv(per), FastDiv(rows), split);
     else
-      hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 3>), dim3(xcd_grid(c->np)),
-                         dim3(patch_block(items, c->np)), 0, s, l->d_child, l->d_orth, fine, coarse, L, c->np,
-                         FastDiv(per), FastDiv(rows));
+      hipLaunchKernelGGL((restrict_regular_kernel<TI, TO, 3>), dim3(xcd_grid(units)), dim3(block), 0, s, l->d_child,
+                         l->d_orth, fine, coarse, L, c->np, FastDiv(per), FastDiv(rows), split);
     return;
   }
   const int B = 256;
@@ -350,11 +364,13 @@ void interp_t(const te_level_link* l, const TC* coarse, TF* fine, int ncomp, hip
   Layout L = make_layout(f->dim, f->ns, ncomp, f->np);
   const int V = L.n[0] % 2 == 0 ? 2 : 1, per = V == 2 ? L.n[0] / 2 + 1 : L.n[0];
   const int items = per * L.n[1] * (f->dim == 3 ? L.n[2] : 1);
-  const int grid = xcd_grid(f->dim == 2 ? (f->np + 3) / 4 : f->np);
-  const int block = f->dim == 2 ? 256 : patch_block(items, f->np);
+  const int block = f->dim == 2 ? 256 : std::min(256, (items / kInterpItems + 63) / 64 * 64);
+  const int unit = f->dim == 2 ? 64 : block;
+  const int split = patch_split(f->np, items, unit * kInterpItems, unit / 64, items), units = f->np << split;
+  const int grid = xcd_grid(f->dim == 2 ? (units + 3) / 4 : units);
 #define TE_IP(D_, V_)                                                                                              \
   hipLaunchKernelGGL((interp_kernel<TC, TF, D_, V_>), dim3(grid), dim3(block), 0, s, l->d_parent, l->d_orth, coarse, \
-                     fine, L, FastDiv(per), FastDiv(L.n[1]))
+                     fine, L, FastDiv(per), FastDiv(L.n[1]), split)
   if (f->dim == 2) {
     if (V == 2) TE_IP(2, 2);
     else TE_IP(2, 1);

@@ -110,14 +110,14 @@ struct FastDiv {
 // dealt round-robin over the 8) takes the x-th contiguous eighth of n items: patches are in
 // Morton order, so most neighbours are then read through the same L2.  n or more: no item.
 __host__ __device__ inline int xcd_grid(int n) { return (n + 7) / 8 * 8; }
-// Threads of a workgroup that works on one patch: up to 256, or up to 1024 on levels with no more
-// patches than CUs, whose launch lasts as long as one patch's chain of loads and stores.
-inline int patch_block(int items, int np)
-{
-  const int cap = np <= 256 ? 1024 : 256, want = (items + 63) / 64 * 64;
-  return want < cap ? want : cap;
-}
 __device__ __forceinline__ int xcd_item(int b, int grid) { return (b & 7) * (grid >> 3) + (b >> 3); }
+
+// part k of n items in 2^split equal parts: [*first, the return value)
+__device__ __forceinline__ int split_range(int n, int split, int k, int* first)
+{
+  *first = (int)(((long)n * k) >> split);
+  return (int)(((long)n * (k + 1)) >> split);
+}
 
 // The interior cells of a padded vector as items of V consecutive padded values: row after row
 // (ghost rows left out), each row the V-wide groups that cover its cells.  V = 2 (even n[0],
@@ -208,6 +208,14 @@ std::vector<int32_t> ring_table(const te_domain* d, const int32_t* parent, const
 
 // compute units of the current device (queried once per device)
 int cu_count();
+// Each of np patches is shared by 2^s units (workgroups or wavefronts) of `waves` waves, `pass` of
+// its `items` work items a pass: s grows while a unit would take more than two passes and the
+// launch has fewer than 16 waves a CU, and not past `most` units.  A patch that one wave walks
+// alone takes as long as its cells: the operator on 4 patches of 1024^2 (FP64) 3,460 us as one wave
+// a patch, 27 shared; 8 of 64^3 148 and 17; 64 of 32^2 7.0 and 4.4.  Not more waves, nor fewer (the
+// same for 1,024 patches of 128^2 in FP32 at 8 / 16 / 32 waves a CU: 41 / 30 / 34 us; 512 of 16^3 in
+// FP64: 17 / 16 / 20; only 16 patches of 1024^2 gain from more, 96 / 80).
+int patch_split(int np, long items, int pass, int waves, long most);
 // workgroups of `block` threads and `shmem` dynamic LDS bytes of `kernel` resident at once
 // on the whole current device (occupancy query, cached)
 int resident_blocks(const void* kernel, int block, size_t shmem);
@@ -220,6 +228,7 @@ bool timer_has_domain(const te_timer* t, int domain_id);
 
 // ---- launchers (defined in kernels/*.hip) ----
 int launch_ghost_fill(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s);
+int launch_ghost_fill_faces(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s);
 int launch_ghost_fill_lowdim(const te_ghost_filler* g, int dtype, void* u, int ncomp, hipStream_t s);
 // out = A u, or fin - A u where fin is given.  fill: u's ghosts are filled first (as
 // launch_ghost_fill) in the same launch; otherwise they are read as they are.
