@@ -824,6 +824,35 @@ def test_patches_of_many_cells(ns):
             assert relerr(dcv.get(), O.restrict(of, oc, f0)) <= (TOL64 if t64 else TOL32)
 
 
+@pytest.mark.parametrize("ns", [(2, 2, 2), (2, 2, 8), (4, 2, 4), (4, 4, 6), (8, 8, 8), (4, 16, 6), (12, 6, 10)])
+@pytest.mark.parametrize("big", [False, True])
+def test_ghost_fill_3d_forms(ns, big):
+    """Every form of the 3D face fill (faces of at most 16 cells, of at most 64, of more; few
+    patches and many, every neighbour type): FP64 and FP32 against the oracle, two components."""
+    _print_case("ghost3d-forms", ns, big)
+    if big:
+        forest = solver.Forest(3, 3)
+        forest.refine((np.arange(512) % 5 == 0).astype(np.uint8))
+        forest.balance()
+        lv = forest.build_domains(ns)[0]
+        assert len(lv) * 6 > 4096 and all((lv["nbr_type"][:, 20:] == k).any() for k in (-1, 0, 1, 2))
+    else:
+        lv = load("3d_refined_bnw_2x2x2_mpi1.json", ns)[1][0]
+    od, dd = O.Domain(3, ns, lv), R.Domain(3, ns, lv)
+    g = R.GhostFiller(dd, R.TRILINEAR, R.FACES)
+    for dtype, tol in ((R.F64, TOL64), (R.F32, TOL32)):
+        u0 = random_field(od.shape(2), 74, R.np_dtype(dtype))
+        ref = u0.astype(np.float64)
+        O.fill_ghost(od, ref, kind=R.TRILINEAR)
+        du, df = R.DeviceArray.from_host(u0), R.DeviceArray(dd.shape(2), R.np_dtype(dtype))
+        g.fill_ghost(du)
+        got = du.get()
+        assert relerr(got, ref) <= tol
+        du.upload(u0)
+        g.star_apply(du, df)  # the operator's own fill
+        assert np.array_equal(du.get(), got)
+
+
 @pytest.mark.parametrize("ns,level,ncomp,dtype", [
     ((16, 16, 16), 5, 3, R.F64), ((16, 16, 16), 5, 8, R.F32), ((12, 12, 12), 5, 8, R.F64), ((64, 64), 7, 8, R.F64)])
 def test_vectors_past_4_gib(ns, level, ncomp, dtype):

@@ -73,30 +73,55 @@ __global__ void ghost_corners_2d(const DevPatch* __restrict__ dp, T* __restrict_
   }
 }
 
-// 3D faces: a workgroup per patch or part of its faces' cells, so that the patch's neighbour records
-// are wave-uniform and a cell's place on the face takes one division.  SIDES (faces of at most 64
-// cells): a wave per side; else each thread takes the same cell of all six sides (fill_faces3).
-template <typename T, bool SIDES>
-__global__ void __launch_bounds__(SIDES ? 384 : 256) ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L,
-                                                                    int split)
+// 3D faces, so that a wave's patch (and side) and with it the neighbour records are uniform and a
+// cell's place on the face takes one division (FP64, one thread per ghost cell of all patches -> the form):
+//  FACES_SMALL, faces of at most 16 cells: a wave per patch, the six faces' cells in a row
+//    (fill_faces3_small; 32,768 patches of 4^3: 36 -> 26 us, 48 as FACES_SIDES);
+//  FACES_SIDES, up to 64 cells: a workgroup per patch, a wave per side (4,096 of 8^3: 23 -> 12);
+//  FACES_PARTS, more, on levels that leave the card partly idle: as FACES_SIDES, the patch's faces shared by
+//    several workgroups (512 of 16^3: 11.8 -> 6.8, 8.0 as FACES_ALL; 64 of 64^3: 13.6 -> 12.6, 54;
+//    8 of 128^3: 6.8 -> 5.1, 107).  Up to one patch a CU they are dealt to the XCDs in turn:
+//    contiguous eighths take 15.3 us for 64 of 64^3, but 6.8 against 9.9 for 512 of 16^3;
+//  FACES_ALL, more, on the other levels: a workgroup per patch, each thread a cell of all six sides
+//    (fill_faces3), so that one workgroup reads a neighbour's lines (4,096 of 16^3: 76 -> 62).
+enum FaceForm { FACES_SMALL, FACES_SIDES, FACES_PARTS, FACES_ALL };
+
+template <typename T, int FORM>
+__global__ void __launch_bounds__(FORM == FACES_SIDES || FORM == FACES_PARTS ? 384 : 256)
+  ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L, int split, bool in_turn)
 {
-  const int unit = xcd_item(blockIdx.x, gridDim.x), p = unit >> split;
+  const int b = FORM == FACES_PARTS && in_turn ? blockIdx.x : xcd_item(blockIdx.x, gridDim.x);
+  if (FORM == FACES_SMALL) {
+    const int q = __builtin_amdgcn_readfirstlane(b * 4 + (threadIdx.x >> 6));
+    if (q < L.np) fill_faces3_small<T>(L, dp[q], u, q, threadIdx.x & 63, 64, largest_face(L));
+    return;
+  }
+  const int p = FORM == FACES_PARTS ? b >> split : b;
   if (p >= L.np) return;
   const DevPatch& P = dp[p];
-  if (!SIDES) {
-    int first[6], last[6];
+  if (FORM == FACES_ALL) {
+    int first[6] = { 0, 0, 0, 0, 0, 0 }, last[6];
 #pragma unroll
-    for (int s = 0; s < 6; s++)
-      last[s] = split_range(L.n[s < 2 ? 1 : 0] * L.n[s < 4 ? 2 : 1], split, unit & ((1 << split) - 1), &first[s]);
+    for (int s = 0; s < 6; s++) last[s] = L.n[s < 2 ? 1 : 0] * L.n[s < 4 ? 2 : 1];
     fill_faces3<T>(L, P, u, p, threadIdx.x, blockDim.x, first, last);
     return;
   }
-  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), k = threadIdx.x & 63;
-  const int type = P.type[20 + s], ni = L.n[s < 2 ? 1 : 0], nj = L.n[s < 4 ? 2 : 1], j = k / ni;
-  if (type < 0 || k >= ni * nj) return;
-  for (int c = 0; c < L.ncomp; c++) {
-    const T G = face_ghost3<T>(L, type, P.orth[20 + s], P.nbr[20 + s], u, p, c, s, k - j * ni, j);
-    at(component(L, u, p, c), side_cell3(L, 0, 0, s, -1, k - j * ni, j)) = G;
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int type = P.type[20 + s], ni = L.n[s < 2 ? 1 : 0], nj = L.n[s < 4 ? 2 : 1];
+  if (type < 0) return;
+  auto fill = [&](int k) {
+    const int j = k / ni;
+    for (int c = 0; c < L.ncomp; c++) {
+      const T G = face_ghost3<T>(L, type, P.orth[20 + s], P.nbr[20 + s], u, p, c, s, k - j * ni, j);
+      at(component(L, u, p, c), side_cell3(L, 0, 0, s, -1, k - j * ni, j)) = G;
+    }
+  };
+  if (FORM == FACES_SIDES) {
+    if (lane < ni * nj) fill(lane);
+  } else {
+    int first;
+    const int last = split_range(ni * nj, split, b & ((1 << split) - 1), &first);
+    for (int k = first + lane; k < last; k += 64) fill(k);
   }
 }
 
@@ -215,15 +240,22 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, bool low
         hipLaunchKernelGGL((ghost_corners_2d<T, TE_BIQUADRATIC>), dim3(cg), dim3(B), 0, s, d->d_patches, u, L);
     }
   } else {
-    int face = 0;  // cells of the largest face: a thread each, up to 256
-    for (int a = 0; a < 3; a++) face = std::max(face, d->ns[a] * d->ns[(a + 1) % 3]);
-    if (faces && face <= 64)
-      hipLaunchKernelGGL((ghost_faces_3d<T, true>), dim3(xcd_grid(d->np)), dim3(384), 0, s, d->d_patches, u, L, 0);
-    else if (faces) {
-      const int block = std::min(256, (face + 63) / 64 * 64), split = patch_split(d->np, face, block, block / 64, face);
-      hipLaunchKernelGGL((ghost_faces_3d<T, false>), dim3(xcd_grid(d->np << split)), dim3(block), 0, s, d->d_patches, u,
-                         L, split);
+    const int face = largest_face(L);
+    const int split = patch_split(d->np, face, 64, 2, face);  // of FACES_PARTS: short waves, so 48 of them a CU
+#define TE_GF(FORM_, UNITS_, BLOCK_)                                                                                \
+  hipLaunchKernelGGL((ghost_faces_3d<T, FORM_>), dim3(xcd_grid(UNITS_)), dim3(BLOCK_), 0, s, d->d_patches, u, L, split, \
+                     d->np <= cu_count())
+    if (!faces) {
+    } else if (face <= kSmallFace) {
+      TE_GF(FACES_SMALL, (d->np + 3) / 4, B);
+    } else if (face <= 64) {
+      TE_GF(FACES_SIDES, d->np, 384);
+    } else if (d->np * 6L < 16L * cu_count()) {
+      TE_GF(FACES_PARTS, d->np << split, 384);
+    } else {
+      TE_GF(FACES_ALL, d->np, std::min(B, (face + 63) / 64 * 64));
     }
+#undef TE_GF
     if (lowdim && g->fill_type != TE_FACES) {
       int tmax = d->ns[0];
       for (int a = 1; a < 3; a++) tmax = d->ns[a] > tmax ? d->ns[a] : tmax;

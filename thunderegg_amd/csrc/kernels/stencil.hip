@@ -77,7 +77,9 @@ __global__ void __launch_bounds__(256) star_kernel(const DevPatch* __restrict__ 
     } else {
       const int f0[6] = { lo * n1, lo * n1, lo * n0, lo * n0, 0, 0 };
       const int f1[6] = { hi * n1, hi * n1, hi * n0, hi * n0, low ? n0 * n1 : 0, high ? n0 * n1 : 0 };
-      fill_faces3<T>(L, P, u, p, t, nt, f0, f1);
+      const int face = largest_face(L);
+      if (face <= kSmallFace && split == 0) fill_faces3_small<T>(L, P, u, p, t, nt, face);
+      else fill_faces3<T>(L, P, u, p, t, nt, f0, f1);
       __syncthreads();
     }
   }
