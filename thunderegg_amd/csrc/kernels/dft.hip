@@ -28,6 +28,7 @@ struct DftGeom {
   int mp;      // pitch of a transposed matrix; a multiple of 4 (vec) where it fits
   int nmat;    // matrices per direction and copy: one per axis, or one for all of equal sizes and types
   bool vec, share;  // share: one copy for the whole workgroup (every patch has the same types)
+  bool one;         // a thread per cell: one output a task, the cell's interface terms formed by its thread
   FastDiv d0, d1, lines[3], na[3];
 };
 
@@ -40,12 +41,16 @@ struct DftGeom {
 // staged value and four matrix values (one wide LDS read, the same for a wave's lanes, which
 // take consecutive lines) feed four multiply-adds.  The last forward transform divides by the
 // eigenvalues as it writes, the last inverse one writes the result.  The interface terms are
-// formed first, a thread per side cell (in 2D from one ring-table record each).
+// formed first, a thread per side cell (in 2D from one ring-table record each).  Where the patch
+// has a thread per cell (G.one, small levels) a task is one output, and a thread forms the terms
+// of its own cell from the filled ghosts: the launch then lasts as long as one thread's chain,
+// and four outputs, a barrier per axis and terms apart make that longer (16 patches of 8^2 in FP64
+// 7.8 us, 5.3 so; 8 of 4^3 9.7, 6.4).
 // Bound by LDS reads on large levels, by the chain of loads and barriers on small ones.
-// Measured against one output a thread and task, the terms formed cell by cell (apply from
-// zero with its zeroed ghosts / sweep with its ghosts, us): 1,024 patches of 24^2 in FP64
-// 43.4 -> 14.9 / 49.1 -> 21.5; 512 of 12^3 in FP32 37.0 -> 16.2 / 47.8 -> 28.9; 512 of 6^3 in
-// FP32 10.6 -> 8.3 / 13.2 -> 14.0; 1,024 of 7^2 7.8 -> 6.7 / 10.0 -> 10.4; 48 problems
+// Measured against one output a thread and task everywhere, the terms formed cell by cell (apply
+// from zero with its zeroed ghosts / sweep on filled ghosts, us): 1,024 patches of 24^2 in FP64
+// 44 -> 14.7 / 41.6 -> 14.9; 512 of 12^3 in FP32 36.6 -> 15.5 / 34.0 -> 17.9; 512 of 6^3 in
+// FP32 10.3 -> 6.7 / 8.6 -> 7.5; 1,024 of 7^2 7.9 -> 5.3 / 7.1 -> 6.0; 48 problems
 // together, a third of them on 8^2 patches, 12.2 -> 10.7 ms.
 template <typename T, typename TF, typename TO, int D, int OP, bool UZERO, int GM = 0, int KIND = 0, typename TC = T>
 __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ dp, const int* __restrict__ ptype,
@@ -70,29 +75,60 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
   T* A = reinterpret_cast<T*>(smem_raw) + (G.share ? 1 : ppw) * 2 * G.nmat * msz + sub * (NP + (NP > nr ? NP : nr));
   T* B = A + NP;
   T* term = B;  // consumed before the first transform writes B
-  const int* pt = ptype + p * 8;      // fwd type per axis [0..2], eig type per axis [3..5], zero mode [6]
+  // transform and eigenvalue types per axis, zero mode; without Neumann sides (share) DST-II, Dirichlet
+  int tf[D], te[D], zero_mode = 0;
+#pragma unroll
+  for (int a = 0; a < D; a++) {
+    tf[a] = 3;
+    te[a] = 2;
+  }
+  if (!G.share) {
+    const int* pt = ptype + p * 8;
+#pragma unroll
+    for (int a = 0; a < D; a++) {
+      tf[a] = pt[a];
+      te[a] = pt[3 + a];
+    }
+    zero_mode = pt[6];
+  }
   const DevPatch& P = dp[p];
   if (UZERO && zero_ghosts && live)  // the patch's results follow after the barriers
     for (int k = t; k < L.cs; k += tpp) out[p * L.ps + k] = TO(0);
   {
     const int m0 = G.share ? threadIdx.x : t, step = G.share ? blockDim.x : tpp;
-    for (int a = 0; a < G.nmat; a++) {
-      const int tf = pt[a], ti = tf == 0 ? 1 : (tf == 3 ? 4 : tf);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
+#pragma unroll
+    for (int a = 0; a < D; a++) {
+      if (a >= G.nmat) break;
+      const int ti = tf[a] == 0 ? 1 : (tf[a] == 3 ? 4 : tf[a]);  // DCT_II->DCT_III, DST_II->DST_III, IV types self-inverse
       for (int i = m0; i < nn[a] * nn[a]; i += step) {
         const int k = G.na[a](i), j = i - k * nn[a];
-        M[a * msz + j * G.mp + k] = mats[(tf * 3 + a) * kDftMatStride + i];
+        M[a * msz + j * G.mp + k] = mats[(tf[a] * 3 + a) * kDftMatStride + i];
         M[(G.nmat + a) * msz + j * G.mp + k] = mats[(ti * 3 + a) * kDftMatStride + i];
       }
     }
   }
-  // f_copy = f
+  // f_copy = f, then modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson
+  // :168-186), sides in the reference's order: here (a thread per cell), or term by term below
+  const bool here = !UZERO && GM == 0 && G.one;
   for (int o = t; o < N; o += tpp) {
     const int row = G.d0(o), x = o - row * n0, z = D == 3 ? G.d1(row) : 0, y = row - z * n1;
-    A[row * G.px + x] = T(f[lin(L, p, 0, x, y, z)]);
+    const int c = lin(L, p, 0, x, y, z), c3[3] = { x, y, z };
+    T v = T(f[c]);
+    if (here) {
+#pragma clang fp contract(off)  // a term is rounded before it is subtracted, as below: the same bits for every launch shape
+      const T ub = u[c], cb = OP == 1 ? coeffs[c] : T(0);
+#pragma unroll
+      for (int s = 0; s < 2 * D; s++) {
+        const int a = s >> 1, st = a == 0 ? 1 : (a == 1 ? L.sx : L.sy), g = s & 1 ? c + st : c - st;
+        if (c3[a] != (s & 1 ? nn[a] - 1 : 0) || P.type[(D == 2 ? 4 : 20) + s] < 0) continue;
+        const T ih2 = T(P.inv_h2[a]), w = u[g] + ub;
+        if (OP == 0) v -= w * ih2;
+        else v -= w * (cb + coeffs[g]) * (ih2 * T(0.5));
+      }
+    }
+    A[row * G.px + x] = v;
   }
-  // modifyRHSForInternalBoundaryConditions (Poisson :165-180, VarPoisson :168-186), sides in the
-  // reference's order
-  if (!UZERO && D == 2) {
+  if (!UZERO && !here && D == 2) {
     for (int g = t; g < nr; g += tpp) {
       int s, tt;
       const int ri = ring_index(p, g, n0, n1, &s, &tt);
@@ -145,7 +181,7 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
     c3[f1] = j;
   };
   auto faces = [&](int a) { return 2 * N / nn[a]; };
-  if (!UZERO && D == 3) {
+  if (!UZERO && !here && D == 3) {
 #pragma unroll
     for (int a = 0; a < D; a++) {
       const int g0 = a == 0 ? 0 : a == 1 ? faces(0) : faces(0) + faces(1);
@@ -166,7 +202,7 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
     }
   }
   __syncthreads();
-  if (!UZERO) {
+  if (!UZERO && !here) {
 #pragma unroll
     for (int a = 0; a < D; a++) {
       if (D == 2) {
@@ -195,11 +231,12 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
 #pragma unroll
   for (int a = 0; a < D; a++) scale *= T(2.0) / T(nn[a]);
   // one transform (DST-II / DCT-II / DCT-IV / DST-IV and their inverses) along axis a
-  auto transform = [&](int a, const T* Mt, const T* src, auto put) {
+  // (pre(l, k0): task (l, k0)'s values for its outputs, loaded before its product)
+  auto transform = [&](int a, const T* Mt, const T* src, auto pre, auto put) {
     const int na = nn[a], sta = a == 0 ? 1 : (a == 1 ? G.px : G.px * n1), nl = (int)G.lines[a].d;
-    const int tasks = nl * ((na + 3) / 4);
+    const int tasks = G.one ? nl * na : nl * ((na + 3) / 4);
     for (int i = t; i < tasks; i += tpp) {
-      const int kb = G.lines[a](i), l = i - kb * nl, k0 = 4 * kb;
+      const int kb = G.lines[a](i), l = i - kb * nl, k0 = G.one ? kb : 4 * kb;
       int base;
       if (a == 0) {
         base = l * G.px;
@@ -207,7 +244,14 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
         const int q = G.d0(l);
         base = l - q * n0 + (a == 1 ? q * G.px * n1 : q * G.px);
       }
+      const auto e = pre(l, k0);
       T acc[4] = { T(0), T(0), T(0), T(0) };
+      if (G.one) {
+#pragma unroll 4
+        for (int j = 0; j < na; j++) acc[0] += Mt[j * G.mp + k0] * src[base + j * sta];
+        put(l, k0, base + k0 * sta, acc[0], e, 0);
+        continue;
+      }
       if (G.vec) {
         typedef T V4 __attribute__((ext_vector_type(4)));
 #pragma unroll 4
@@ -229,25 +273,43 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
       }
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        if (k0 + r < na) put(l, k0 + r, base + (k0 + r) * sta, acc[r]);
+        if (k0 + r < na) put(l, k0 + r, base + (k0 + r) * sta, acc[r], e, r);
     }
+  };
+  // the eigenvalues (:320-361) of a task's outputs of the last forward transform
+  struct Eig {
+    T v[4];
+  };
+  auto eigen = [&](int l, int k0) {
+    const int y = D == 3 ? G.d0(l) : 0, x = l - y * n0;
+    const T sx = s2tab[te[0] * 3 * kDftMatDim + x], sy = D == 3 ? s2tab[(te[1] * 3 + 1) * kDftMatDim + y] : T(0);
+    T sl[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++)  // loaded together (a load under each output's bound would wait for the one before)
+      sl[r] = s2tab[(te[D - 1] * 3 + D - 1) * kDftMatDim + (k0 + r < nn[D - 1] ? k0 + r : nn[D - 1] - 1)];
+    Eig e;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      T eig = T(0);
+      eig -= lam[0] * sx;
+      if (D == 3) eig -= lam[1] * sy;
+      eig -= lam[D - 1] * sl[r];
+      e.v[r] = eig;
+    }
+    return e;
   };
   T* src = A;
   T* dst = B;
 #pragma unroll
   for (int a = 0; a < D; a++) {
-    transform(a, M + (G.nmat == 1 ? 0 : a) * msz, src, [&](int l, int k, int at_, T v) {
-      if (a == D - 1) {  // divide by the eigenvalues
-        const int y = D == 3 ? G.d0(l) : 0, x = l - y * n0;
-        const int k3[3] = { x, D == 3 ? y : k, k };
-        T eig = T(0);
-#pragma unroll
-        for (int b = 0; b < D; b++) eig -= lam[b] * s2tab[(pt[3 + b] * 3 + b) * kDftMatDim + k3[b]];
-        v = v / eig;
-        if (pt[6] && l == 0 && k == 0) v = T(0);  // all-Neumann patch without neighbours (:438-440)
-      }
-      dst[at_] = v;
-    });
+    transform(a, M + (G.nmat == 1 ? 0 : a) * msz, src, [&](int l, int k0) { return a < D - 1 ? Eig{} : eigen(l, k0); },
+              [&](int l, int k, int at_, T v, const Eig& e, int r) {
+                if (a == D - 1) {
+                  v = v / e.v[r];
+                  if (zero_mode && l == 0 && k == 0) v = T(0);  // all-Neumann patch without neighbours (:438-440)
+                }
+                dst[at_] = v;
+              });
     __syncthreads();
     T* sw = src;
     src = dst;
@@ -255,14 +317,15 @@ __global__ void __launch_bounds__(256) dft_kernel(const DevPatch* __restrict__ d
   }
 #pragma unroll
   for (int a = 0; a < D; a++) {
-    transform(a, M + (G.nmat + (G.nmat == 1 ? 0 : a)) * msz, src, [&](int l, int k, int at_, T v) {
-      if (a < D - 1) {
-        dst[at_] = v;
-      } else if (live) {
-        const int y = D == 3 ? G.d0(l) : k, x = D == 3 ? l - y * n0 : l;
-        out[lin(L, p, 0, x, y, D == 3 ? k : 0)] = TO(v * scale);
-      }
-    });
+    transform(a, M + (G.nmat + (G.nmat == 1 ? 0 : a)) * msz, src, [](int, int) { return 0; },
+              [&](int l, int k, int at_, T v, int, int) {
+                if (a < D - 1) {
+                  dst[at_] = v;
+                } else if (live) {
+                  const int y = D == 3 ? G.d0(l) : k, x = D == 3 ? l - y * n0 : l;
+                  out[lin(L, p, 0, x, y, D == 3 ? k : 0)] = TO(v * scale);
+                }
+              });
     if (a < D - 1) __syncthreads();
     T* sw = src;
     src = dst;
@@ -302,18 +365,21 @@ size_t dft_geom(const te_dft_plan* pl, size_t esz, int ppw, bool terms, DftGeom*
   return bytes();
 }
 
+inline int patch_cells(const te_domain* d) { return d->ns[0] * d->ns[1] * (d->dim == 3 ? d->ns[2] : 1); }
+
 // patches per workgroup and threads per patch: the autotuner's choice for this shape, or (variant
 // 0) a thread per four outputs of a transform, in powers of two from 32 to 256 threads (up to one
-// per cell while the level does not fill the CUs with 256 threads each), and as many patches as
-// make 256 threads and at most 48 KB of LDS
+// per cell while the level does not fill the CUs with 512 threads each), and as many patches as
+// make 256 threads and at most 48 KB of LDS.  The sweep at 256 / 512 / 1,024 threads a CU: 512
+// patches of 6^3 in FP32 9.9 / 7.5 / 7.5 us, 4,096 of 10^2 in FP64 9.9 / 9.9 / 11.7
 DftGenericVariant dft_shape(const te_dft_plan* pl, size_t esz, bool terms)
 {
   const te_domain* d = pl->g->d;
   const int v = tune_variant(TUNE_DFT_GENERIC, d->dim, d->ns[0], esz == 8 ? TE_F64 : TE_F32);
   if (v != 0) return dft_generic_variant(v);
-  const int N = d->ns[0] * d->ns[1] * (d->dim == 3 ? d->ns[2] : 1);
+  const int N = patch_cells(d);
   DftGenericVariant w{ 1, 32 };
-  while (w.tpp < 256 && (w.tpp * 4 < N || (w.tpp < N && (long)d->np * w.tpp < 256 * cu_count()))) w.tpp *= 2;
+  while (w.tpp < 256 && (w.tpp * 4 < N || (w.tpp < N && (long)d->np * w.tpp < 512 * cu_count()))) w.tpp *= 2;
   DftGeom G;
   for (w.ppw = 256 / w.tpp; w.ppw > 1 && dft_geom(pl, esz, w.ppw, terms, &G) > 49152; w.ppw /= 2) {
   }
@@ -744,6 +810,7 @@ void launch_d(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uzer
   const DftGenericVariant v = dft_shape(pl, sizeof(T), !uzero);
   DftGeom G;
   const size_t shmem = dft_geom(pl, sizeof(T), v.ppw, !uzero, &G);
+  G.one = patch_cells(d) <= v.tpp;
   const int grid = (d->np + v.ppw - 1) / v.ppw;
   const FusedArgs<T, T> fa{ nullptr, nullptr, nullptr };
 #define TE_DL(OP_, UZ_)                                                                                          \
@@ -779,6 +846,7 @@ void launch_fused_t(const te_dft_plan* pl, const void* fv, const void* uv, void*
   const DftGenericVariant v = dft_shape(pl, sizeof(T), !uzero);
   DftGeom G;
   const size_t shmem = dft_geom(pl, sizeof(T), v.ppw, !uzero, &G);
+  G.one = patch_cells(d) <= v.tpp;
   const int grid = (d->np + v.ppw - 1) / v.ppw;
   const int4* ring = (const int4*)(gm == 2 ? link->d_ring : d->d_ring);
   const FusedArgs<T, TC> fa{ (const TC*)ucv, link ? link->d_parent : nullptr, link ? link->d_orth : nullptr };
