@@ -642,6 +642,45 @@ def test_dft32_pair(level, op_kind, kind):
             assert relerr(mesh.interior(du.get(), 2), mesh.interior(uref, 2)) <= tol, (dtype, zero)
 
 
+@pytest.mark.parametrize("op_kind", [0, 1])
+@pytest.mark.parametrize("kind", [R.BILINEAR, R.BIQUADRATIC])
+def test_dft32_levels_past_the_card(op_kind, kind):
+    """The 32^2 patch solve on a refined level of more patches than the card holds workgroups for
+    (each then walks several in FP64): from zero, in place on filled ghosts, and on u plus the coarser
+    level's correction, against the oracle."""
+    _print_case("dft32-loop", op_kind, kind)
+    ns = (32, 32)
+    forest = solver.Forest(2, 6)
+    forest.refine((np.arange(4096) % 41 == 0).astype(np.uint8))
+    forest.balance()
+    lv = forest.build_domains(ns)[:2]
+    assert len(lv[0]) > 4096 and all((lv[0]["nbr_type"][:, 4:] == k).any() for k in (-1, 0, 1, 2))
+    (od, oc), (dd, dc) = ([cls(2, ns, v) for v in lv] for cls in (O.Domain, R.Domain))
+    od.link_parents(oc)
+    link, g = R.LevelLink(dd, dc), R.GhostFiller(dd, kind, R.FACES)
+    coeffs = np.exp(0.3 * random_field(od.shape(1), 38)) if op_kind else None
+    if op_kind:
+        O.fill_ghost(od, coeffs, kind=kind)
+    plan = R.DftPlan(g, op_kind=op_kind, coeffs=R.DeviceArray.from_host(coeffs) if op_kind else None)
+    for dtype, tol in [(R.F64, 1e-12), (R.F32, 2e-5)]:
+        t = R.np_dtype(dtype)
+        f0, u0 = random_field(od.shape(1), 33, t), random_field(od.shape(1), 34, t)
+        c0 = random_field(oc.shape(1), 35, t)
+        df, dout = R.DeviceArray.from_host(f0), R.DeviceArray.from_host(np.zeros_like(u0))
+        for mode in ("apply", "smooth", "interp"):
+            uref = np.zeros(od.shape(1)) if mode == "apply" else u0.astype(np.float64)
+            if mode == "interp":
+                O.interpolate(oc, od, c0.astype(np.float64), uref)
+            O.dft_smooth(od, f0.astype(np.float64), uref, kind=kind, op_kind=op_kind, coeffs=coeffs)
+            du = R.DeviceArray.from_host(u0)
+            if mode == "interp":
+                plan.smooth_interp(link, df, du, R.DeviceArray.from_host(c0), dout)
+            else:
+                getattr(plan, mode)(df, du)
+            got = (dout if mode == "interp" else du).get()
+            assert relerr(mesh.interior(got, 2), mesh.interior(uref, 2)) <= tol, (dtype, mode)
+
+
 @pytest.mark.parametrize("ns", [(4, 8), (8, 8), (10, 6), (20, 24), (32, 32), (40, 12)])
 @pytest.mark.parametrize("kind", [R.BILINEAR, R.BIQUADRATIC])
 @pytest.mark.parametrize("neumann", [False, True])

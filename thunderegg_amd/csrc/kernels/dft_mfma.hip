@@ -344,9 +344,15 @@ void launch_n16(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uz
 // The matrices' operands live in registers (48 a lane).  The interface terms come first, one of
 // the 128 side cells per thread, and are subtracted in the operand layout, west / east then
 // south / north (Poisson/StarPatchOperator.h:165-180).
+// LOOP: a workgroup walks its patches with the operands loaded once; without it a patch a
+// workgroup, whose operand loads (24 KB of L2 a wave in FP64) are issued behind the patch's own.
 // Against one wave a patch: 48 problems of up to 2,400 patches, a third of them 32^2, solved together
-// (mixed): 15.3 -> 13.1 ms.
-template <typename T, typename TF, typename TO, typename TC, int OP, bool UZERO, int GM, int KIND>
+// (mixed): 15.3 -> 13.1 ms.  The solve on filled ghosts, one wave a patch / two, a patch a workgroup /
+// LOOP, us: 64 patches in FP64 10.0 / 6.3 / 7.6; 1,024 15.6 / 17.3 / 19.4; 4,096 40 / 54 / 41; 16,384
+// 189 / 197 / 141; 16,384 in FP32 97 / 82 / 69.  Hence LOOP in FP64 from two patches a resident
+// workgroup on.  Not in FP32, where the operands are half as many bytes: it takes the places of the
+// launches beside it (the 48 problems, on three streams, 1.2 to 1.8 % slower with it).
+template <typename T, typename TF, typename TO, typename TC, int OP, bool UZERO, int GM, int KIND, bool LOOP>
 __global__ void __launch_bounds__(128) dft32_kernel(const DevPatch* __restrict__ dp, const T* __restrict__ mats,
                                                     const T* __restrict__ s2tab, const TF* __restrict__ f, const T* u,
                                                     const T* __restrict__ coeffs, TO* out, int np, FusedArgs<T, TC> fa,
@@ -356,139 +362,150 @@ __global__ void __launch_bounds__(128) dft32_kernel(const DevPatch* __restrict__
   typedef typename Mf<T>::V V;
   __shared__ __align__(16) T X[n * LD];
   __shared__ T term[UZERO ? 1 : 4 * n];
-  const int p = xcd_item(blockIdx.x, gridDim.x);
-  if (p >= np) return;
   const int J = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const DevPatch& P = dp[p];
-  const int base = p * PS + SX + 1;  // cell (0, 0)
-  // F[I][K][s]: row 16 I + c, column 16 K + 4 g + s
-  T F[2][2][4];
-#pragma unroll
-  for (int I = 0; I < 2; I++)
-#pragma unroll
-    for (int K = 0; K < 2; K++) load_row4(f, base + (16 * I + c) * SX + 16 * K + 4 * g, F[I][K]);
-  if (!UZERO) {
-    const int s = threadIdx.x >> 5, t = threadIdx.x & 31, ph = s >> 1, up = s & 1;
-    int bx, by;
-    side_xy(s, 0, t, n, &bx, &by);
-    const int bi = base + by * SX + bx, gi = bi + (up ? 1 : -1) * (ph == 0 ? 1 : SX);
-    T v = T(0);
-    if (GM == 0) {
-      if (P.type[4 + s] >= 0) v = u[gi] + u[bi];
-    } else {
-      const int4 r = ring[(p * 4 + s) * 2 + (2 * t >= n ? 1 : 0)];
-      // u, or u + P uc: parent and orthant of patch q
-      auto val = [&](int q, int par, int o, int x, int y) {
-        T a = at(u, q * PS + (y + 1) * SX + x + 1);
-        if (GM == 2) {
-          const int cx = o >= 0 ? (x + ((o & 1) ? n : 0)) / 2 : x, cy = o >= 0 ? (y + ((o & 2) ? n : 0)) / 2 : y;
-          a = T(a + T(at(fa.uc, par * PS + (cy + 1) * SX + cx + 1)));
-        }
-        return a;
-      };
-      if (r.x >= 0) {
-        const int par = GM == 2 ? fa.parent[p] : 0, o = GM == 2 ? fa.porth[p] : -1;
-        T gv[4] = { T(0), T(0), T(0), T(0) };
-        ghost2d_gather<KIND>(r.x, r.y, r.z, s, t, n, n,
-                             [&](int k, int q, int x, int y) { gv[k] = val(q, r.w >> 3, (r.w & 7) - 1, x, y); });
-        const T ug = ghost2d_combine<T, KIND>(r.x, r.y, t, n,
-                                              [&](int k, int tt) {
-                                                int x, y;
-                                                side_xy(s, k, tt, n, &x, &y);
-                                                return val(p, par, o, x, y);
-                                              },
-                                              gv);
-        v = ug + val(p, par, o, bx, by);
-      }
-    }
-    const T ih2 = T(P.inv_h2[ph]);
-    if (OP == 0) v = v * ih2;
-    else if (P.type[4 + s] >= 0) v = v * (coeffs[bi] + coeffs[gi]) * (ih2 * T(0.5));
-    term[s * n + t] = v;  // 0 on physical sides
-  }
+  const XcdRange xr = LOOP ? xcd_range(blockIdx.x, gridDim.x, np, 1) : XcdRange{ xcd_item(blockIdx.x, gridDim.x), 0, np };
+  int p = xr.first;
+  if (p >= xr.end) return;
   // the matrices as operands: lane (c, g), step s holds element (16 B + c, K index)
   auto mat = [&](int ty, int i, int k) { return mats[(ty * 3) * kDftMatStride + i * n + k]; };  // axis 0; 3: DST-II, 4: DST-III
   T SB[2][4], S3B[2][4], SA[2][2][4], S3A[2][2][4];
-#pragma unroll
-  for (int K = 0; K < 2; K++)
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      SB[K][s] = mat(3, 16 * J + c, 16 * K + 4 * g + s);
-      S3B[K][s] = mat(4, 16 * J + c, 16 * K + 4 * g + s);
-#pragma unroll
-      for (int I = 0; I < 2; I++) {
-        SA[I][K][s] = mat(3, 16 * I + c, 16 * K + Mf<T>::row(s, g));
-        S3A[I][K][s] = mat(4, 16 * I + c, 16 * K + Mf<T>::row(s, g));
-      }
-    }
-  if (!UZERO) {
-    __syncthreads();
-#pragma unroll
-    for (int I = 0; I < 2; I++) {
-      if (g == 0) F[I][0][0] -= term[16 * I + c];
-      if (g == 3) F[I][1][3] -= term[n + 16 * I + c];
-    }
+  auto operands = [&]() {
 #pragma unroll
     for (int K = 0; K < 2; K++)
 #pragma unroll
       for (int s = 0; s < 4; s++) {
-        if (c == 0) F[0][K][s] -= term[2 * n + 16 * K + 4 * g + s];
-        if (c == 15) F[1][K][s] -= term[3 * n + 16 * K + 4 * g + s];
+        SB[K][s] = mat(3, 16 * J + c, 16 * K + 4 * g + s);
+        S3B[K][s] = mat(4, 16 * J + c, 16 * K + 4 * g + s);
+#pragma unroll
+        for (int I = 0; I < 2; I++) {
+          SA[I][K][s] = mat(3, 16 * I + c, 16 * K + Mf<T>::row(s, g));
+          S3A[I][K][s] = mat(4, 16 * I + c, 16 * K + Mf<T>::row(s, g));
+        }
       }
-  }
-  V Y[2], Z[2];
+  };
+  if (LOOP) operands();
+  for (;;) {
+    const DevPatch& P = dp[p];
+    const int base = p * PS + SX + 1;  // cell (0, 0)
+    // F[I][K][s]: row 16 I + c, column 16 K + 4 g + s
+    T F[2][2][4];
 #pragma unroll
-  for (int I = 0; I < 2; I++) {
-    V acc = { 0, 0, 0, 0 };
+    for (int I = 0; I < 2; I++)
 #pragma unroll
-    for (int K = 0; K < 2; K++)
-#pragma unroll
-      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(F[I][K][s], SB[K][s], acc);
-    Y[I] = acc;
-  }
-  const T lx = T(4.0 / (P.h[0] * P.h[0])), ly = T(4.0 / (P.h[1] * P.h[1]));
-  const T* s2 = s2tab + (2 * 3 + 0) * kDftMatDim;
-  const T s2x = s2[16 * J + c];
-#pragma unroll
-  for (int I = 0; I < 2; I++) {
-    V acc = { 0, 0, 0, 0 };
-#pragma unroll
-    for (int K = 0; K < 2; K++)
-#pragma unroll
-      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(SA[I][K][s], Y[K][s], acc);
-    // divide by the eigenvalues -4/hx^2 s2[kx] - 4/hy^2 s2[ky] (getEigenValues, :320-361)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      T eig = T(0);
-      eig -= lx * s2x;
-      eig -= ly * s2[16 * I + Mf<T>::row(r, g)];
-      // FP32: the hardware reciprocal (1 ulp) instead of a correctly rounded division
-      if (sizeof(T) == 4) acc[r] = acc[r] * T(__builtin_amdgcn_rcpf(float(eig)));
-      else acc[r] = acc[r] / eig;
+      for (int K = 0; K < 2; K++) load_row4(f, base + (16 * I + c) * SX + 16 * K + 4 * g, F[I][K]);
+    if (!UZERO) {
+      const int s = threadIdx.x >> 5, t = threadIdx.x & 31, ph = s >> 1, up = s & 1;
+      int bx, by;
+      side_xy(s, 0, t, n, &bx, &by);
+      const int bi = base + by * SX + bx, gi = bi + (up ? 1 : -1) * (ph == 0 ? 1 : SX);
+      T v = T(0);
+      if (GM == 0) {
+        if (P.type[4 + s] >= 0) v = u[gi] + u[bi];
+      } else {
+        const int4 r = ring[(p * 4 + s) * 2 + (2 * t >= n ? 1 : 0)];
+        // u, or u + P uc: parent and orthant of patch q
+        auto val = [&](int q, int par, int o, int x, int y) {
+          T a = at(u, q * PS + (y + 1) * SX + x + 1);
+          if (GM == 2) {
+            const int cx = o >= 0 ? (x + ((o & 1) ? n : 0)) / 2 : x, cy = o >= 0 ? (y + ((o & 2) ? n : 0)) / 2 : y;
+            a = T(a + T(at(fa.uc, par * PS + (cy + 1) * SX + cx + 1)));
+          }
+          return a;
+        };
+        if (r.x >= 0) {
+          const int par = GM == 2 ? fa.parent[p] : 0, o = GM == 2 ? fa.porth[p] : -1;
+          T gv[4] = { T(0), T(0), T(0), T(0) };
+          ghost2d_gather<KIND>(r.x, r.y, r.z, s, t, n, n,
+                               [&](int k, int q, int x, int y) { gv[k] = val(q, r.w >> 3, (r.w & 7) - 1, x, y); });
+          const T ug = ghost2d_combine<T, KIND>(r.x, r.y, t, n,
+                                                [&](int k, int tt) {
+                                                  int x, y;
+                                                  side_xy(s, k, tt, n, &x, &y);
+                                                  return val(p, par, o, x, y);
+                                                },
+                                                gv);
+          v = ug + val(p, par, o, bx, by);
+        }
+      }
+      const T ih2 = T(P.inv_h2[ph]);
+      if (OP == 0) v = v * ih2;
+      else if (P.type[4 + s] >= 0) v = v * (coeffs[bi] + coeffs[gi]) * (ih2 * T(0.5));
+      term[s * n + t] = v;  // 0 on physical sides
     }
-    Z[I] = acc;
-  }
+    if (!LOOP) operands();
+    if (!UZERO) {
+      __syncthreads();
 #pragma unroll
-  for (int I = 0; I < 2; I++) {
-    V acc = { 0, 0, 0, 0 };
+      for (int I = 0; I < 2; I++) {
+        if (g == 0) F[I][0][0] -= term[16 * I + c];
+        if (g == 3) F[I][1][3] -= term[n + 16 * I + c];
+      }
 #pragma unroll
-    for (int K = 0; K < 2; K++)
+      for (int K = 0; K < 2; K++)
 #pragma unroll
-      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(S3A[I][K][s], Z[K][s], acc);
+        for (int s = 0; s < 4; s++) {
+          if (c == 0) F[0][K][s] -= term[2 * n + 16 * K + 4 * g + s];
+          if (c == 15) F[1][K][s] -= term[3 * n + 16 * K + 4 * g + s];
+        }
+    }
+    V Y[2], Z[2];
 #pragma unroll
-    for (int r = 0; r < 4; r++) X[(16 * I + Mf<T>::row(r, g)) * LD + 16 * J + c] = acc[r];
-  }
-  __syncthreads();
-  const T scale = T(4.0 / double(n * n));  // prod over axes of 2/n (:442-449)
+    for (int I = 0; I < 2; I++) {
+      V acc = { 0, 0, 0, 0 };
 #pragma unroll
-  for (int I = 0; I < 2; I++) {
-    V acc = { 0, 0, 0, 0 };
+      for (int K = 0; K < 2; K++)
 #pragma unroll
-    for (int K = 0; K < 2; K++)
+        for (int s = 0; s < 4; s++) acc = Mf<T>::mma(F[I][K][s], SB[K][s], acc);
+      Y[I] = acc;
+    }
+    const T lx = T(4.0 / (P.h[0] * P.h[0])), ly = T(4.0 / (P.h[1] * P.h[1]));
+    const T* s2 = s2tab + (2 * 3 + 0) * kDftMatDim;
+    const T s2x = s2[16 * J + c];
 #pragma unroll
-      for (int s = 0; s < 4; s++) acc = Mf<T>::mma(X[(16 * I + c) * LD + 16 * K + 4 * g + s], S3B[K][s], acc);
+    for (int I = 0; I < 2; I++) {
+      V acc = { 0, 0, 0, 0 };
 #pragma unroll
-    for (int r = 0; r < 4; r++) at(out, base + (16 * I + Mf<T>::row(r, g)) * SX + 16 * J + c) = TO(acc[r] * scale);
+      for (int K = 0; K < 2; K++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc = Mf<T>::mma(SA[I][K][s], Y[K][s], acc);
+      // divide by the eigenvalues -4/hx^2 s2[kx] - 4/hy^2 s2[ky] (getEigenValues, :320-361)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        T eig = T(0);
+        eig -= lx * s2x;
+        eig -= ly * s2[16 * I + Mf<T>::row(r, g)];
+        // FP32: the hardware reciprocal (1 ulp) instead of a correctly rounded division
+        if (sizeof(T) == 4) acc[r] = acc[r] * T(__builtin_amdgcn_rcpf(float(eig)));
+        else acc[r] = acc[r] / eig;
+      }
+      Z[I] = acc;
+    }
+#pragma unroll
+    for (int I = 0; I < 2; I++) {
+      V acc = { 0, 0, 0, 0 };
+#pragma unroll
+      for (int K = 0; K < 2; K++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc = Mf<T>::mma(S3A[I][K][s], Z[K][s], acc);
+#pragma unroll
+      for (int r = 0; r < 4; r++) X[(16 * I + Mf<T>::row(r, g)) * LD + 16 * J + c] = acc[r];
+    }
+    __syncthreads();
+    const T scale = T(4.0 / double(n * n));  // prod over axes of 2/n (:442-449)
+#pragma unroll
+    for (int I = 0; I < 2; I++) {
+      V acc = { 0, 0, 0, 0 };
+#pragma unroll
+      for (int K = 0; K < 2; K++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc = Mf<T>::mma(X[(16 * I + c) * LD + 16 * K + 4 * g + s], S3B[K][s], acc);
+#pragma unroll
+      for (int r = 0; r < 4; r++) at(out, base + (16 * I + Mf<T>::row(r, g)) * SX + 16 * J + c) = TO(acc[r] * scale);
+    }
+    if (!LOOP) break;
+    p += xr.step;
+    if (p >= xr.end) break;
+    __syncthreads();  // this patch's reads of X and the terms
   }
 }
 
@@ -503,9 +520,20 @@ void launch_n32(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uz
   FusedArgs<T, TC> fa{ uc, link ? link->d_parent : nullptr, link ? link->d_orth : nullptr };
   const int4* ring = (const int4*)(gm == 2 ? link->d_ring : d->d_ring);
   const int kind = pl->g->kind;
-#define TE_M32(OP_, UZ_, GM_, K_)                                                                                    \
-  hipLaunchKernelGGL((dft32_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_>), dim3(xcd_grid(d->np)), dim3(128), 0, s,       \
+#define TE_M32L(OP_, UZ_, GM_, K_, LOOP_, G_)                                                                        \
+  hipLaunchKernelGGL((dft32_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_, LOOP_>), dim3(G_), dim3(128), 0, s,             \
                      d->d_patches, mats, s2, f, u, cf, out, d->np, fa, ring)
+#define TE_M32(OP_, UZ_, GM_, K_)                                                                                    \
+  do {                                                                                                               \
+    if constexpr (sizeof(T) == 8) {                                                                                  \
+      const int r = resident_blocks((const void*)dft32_kernel<T, TF, TO, TC, OP_, UZ_, GM_, K_, true>, 128, 0);      \
+      if (d->np >= 2 * r) {                                                                                          \
+        TE_M32L(OP_, UZ_, GM_, K_, true, r);                                                                         \
+        break;                                                                                                       \
+      }                                                                                                              \
+    }                                                                                                                \
+    TE_M32L(OP_, UZ_, GM_, K_, false, xcd_grid(d->np));                                                              \
+  } while (0)
 #define TE_M32G(OP_)                                                             \
   if (uzero) TE_M32(OP_, true, 0, 0);                                            \
   else if (gm == 0) TE_M32(OP_, false, 0, 0);                                    \
@@ -520,6 +548,7 @@ void launch_n32(const te_dft_plan* pl, const TF* f, const T* u, TO* out, bool uz
   }
 #undef TE_M32G
 #undef TE_M32
+#undef TE_M32L
 }
 
 template <typename T, typename TF, typename TO, typename TC>
