@@ -70,7 +70,6 @@ __global__ void __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? (PF ? (GM == 0 ?
   // in a padded tile first, so the ghost formulas read their self terms from LDS
   constexpr bool TILE = GM != 0;
   T* Tl = s2 + n + kWaves * n * ld + kWaves * 4 * n + wave * (n + 2) * (n + 2);
-  UAcc<T, TC, GM == 2> U{ u, fa.uc, fa.parent, fa.porth, L };
 
   for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
     const int row = k / n, col = k - row * n;
@@ -108,7 +107,7 @@ __global__ void __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? (PF ? (GM == 0 ?
   // (ring table: lane = ring cell, side lane / n, cell lane % n), then, once those have
   // arrived (mid-iteration), its coarse-level values and the neighbour values of every
   // lane's ghost cell (ghost2d_gather; with GM_INTERP each as u and coarse u separately)
-    T un[TILE ? FPL : 1];
+  T un[TILE ? FPL : 1];
   TC ucn[TILE ? FPL : 1];
   int on = -1, parn = 0;
   int4 rn = make_int4(-1, 0, -1, 0), rc = rn;  // ring records of the next / current patch
@@ -160,7 +159,7 @@ __global__ void __launch_bounds__(64 * kWaves, sizeof(T) == 4 ? (PF ? (GM == 0 ?
       }
     });
   };
-  auto tput = [&]() {  // the values UAcc would return, staged from the registers
+  auto tput = [&]() {  // u, or u + P uc, staged from the registers
 #pragma unroll
     for (int k = 0; k < (TILE ? FPL : 1); k++) {
       const int q = lane + 64 * k, y = q / n, x = q - y * n;

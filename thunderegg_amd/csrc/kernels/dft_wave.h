@@ -42,30 +42,6 @@ __device__ __forceinline__ void load_row4(const TS* base, int idx, T (&r)[4])
   }
 }
 
-// u (+ injection of the coarser level's uc) at interior cell (x, y) of patch q
-template <typename T, typename TC, bool INTERP>
-struct UAcc {
-  const T* u;
-  const TC* uc;
-  const int32_t* parent;
-  const int32_t* porth;
-  Layout L;
-  __device__ __forceinline__ T operator()(int q, int x, int y) const
-  {
-    T v = u[q * L.ps + (y + 1) * L.sx + x + 1];
-    if (INTERP) {
-      int o = porth[q];
-      int cx = x, cy = y;
-      if (o >= 0) {
-        cx = (x + ((o & 1) ? L.n[0] : 0)) / 2;
-        cy = (y + ((o & 2) ? L.n[1] : 0)) / 2;
-      }
-      v = T(v + T(uc[parent[q] * L.ps + (cy + 1) * L.sx + cx + 1]));
-    }
-    return v;
-  }
-};
-
 template <typename T, typename TC>
 struct FusedArgs {
   const TC* uc;

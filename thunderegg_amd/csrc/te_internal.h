@@ -165,10 +165,8 @@ struct te_domain {
   te::DevPatch* d_patches = nullptr;
   int any_coarse_fine = 0;         // some face/edge/corner is a coarse/fine interface
   double* d_scratch = nullptr;     // reduction partials
-  unsigned* d_counter = nullptr;   // last-block counter for reductions
   double* result = nullptr;        // a reduction's result: host memory that the kernels write (take_result)
   int32_t* d_flags = nullptr;      // breakdown flags
-  int scratch_len = 0;
   int32_t* d_ring = nullptr;       // 2D: ring table (te::ring_table), pq fields 0
 };
 
