@@ -39,46 +39,60 @@ __device__ __forceinline__ T vec_value(T x, T a, T b, T alpha, T beta, T gamma)
   }
 }
 
-// One interior update.  HBM bound: each thread takes kVecItems groups (te::Rows), their loads
-// issued together before the first store; a group is 16 bytes of FP64 (8 of FP32: rows of n + 2
-// values start on 8-byte multiples only), so that a wave's accesses run through consecutive rows
-// without gaps.  A row's end groups hold a ghost value, which is read and not written.
-// 4096 patches of 16^3 in FP64 (134 MB a vector), against one thread per padded value with its
-// place found by five divisions: copy 96 -> 81 us, x += a y 95 -> 88 (5.1 TB/s with the ghost
-// values of the lines it touches; a plain copy of that size reaches 4.9 to 5.2).
-constexpr int kVecItems = 4;
+// Every padded value in groups of V consecutive ones, ghost rows too: V * i, or -1 for a group
+// without an interior cell; *g: its place in the row.  V divides the row
+struct FlatGroups {
+  FastDiv per_row, ry, rz;
+  int items, n1, n2, last;
+  FlatGroups(const Layout& L, int V)
+      : per_row(L.sx / V), ry(L.n[1] + 2), rz(L.dim == 3 ? L.n[2] + 2 : 1), items((int)((long)L.np * L.ps / V)),
+        n1(L.n[1]), n2(L.dim == 3 ? L.n[2] : 0), last(L.sx / V - 1)
+  {
+  }
+  template <int V>
+  __device__ __forceinline__ int at(int i, int* g) const
+  {
+    const int row = per_row(i), zz = ry(row), y = row - zz * (int)ry.d;
+    *g = i - row * (int)per_row.d;
+    bool in = y >= 1 && y <= n1 && (V > 1 || (*g > 0 && *g < last));
+    if (n2) {
+      const int z = zz - rz(zz) * (int)rz.d;
+      in = in && z >= 1 && z <= n2;
+    }
+    return in ? V * i : -1;
+  }
+};
 
+// One interior update.  HBM bound: a thread takes one group, neighbours in memory are neighbours in
+// the launch, and the ghost rows' threads leave.  Lines are then read in the order in which they
+// lie: four groups of interior rows a thread (Rows, below) made the streams of large vectors
+// slower, at 32768 patches of 16^3 in FP64 (1.5 GB a vector) x = a 888 us, x += a y 830, with
+// two such terms 1075, against 763, 723 and 975 here; one FP64 value a thread with its place found
+// by five divisions took 786, 743 and 941, and in FP32 590, 619 and 642 against 376, 381 and 512.
+// At 4096 patches x = a 95 us, x += a y 92 (4.9 TB/s with the ghost values of the lines it touches).
+// A row's end groups hold a ghost value, which is read and not written.
 template <typename T, int OP, int V>
-__global__ void __launch_bounds__(256) vec_op_kernel(Rows R, T* __restrict__ x, const T* __restrict__ a,
+__global__ void __launch_bounds__(256) vec_op_kernel(FlatGroups R, T* __restrict__ x, const T* __restrict__ a,
                                                      const T* __restrict__ b, T alpha, T beta, T gamma)
 {
   typedef typename Pack<T, V>::Vec P;
   constexpr bool RX = OP != VOP_SET && OP != VOP_COPY, RA = OP >= VOP_COPY,
                  RB = OP == VOP_ADD_SCALED2 || OP == VOP_SCALE_THEN_ADD_SCALED2;
-  int idx[kVecItems], g[kVecItems];
-  P vx[kVecItems], va[kVecItems], vb[kVecItems];
-  const int i0 = blockIdx.x * (256 * kVecItems) + threadIdx.x;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  int g = 0;
+  const int k = i < R.items ? R.at<V>(i, &g) : -1;
+  if (k < 0) return;
+  P vx, va, vb, r;
+  if (RX) vx = *reinterpret_cast<const P*>(x + k);
+  if (RA) va = *reinterpret_cast<const P*>(a + k);
+  if (RB) vb = *reinterpret_cast<const P*>(b + k);
 #pragma unroll
-  for (int k = 0; k < kVecItems; k++) {
-    const int i = i0 + k * 256;
-    idx[k] = i < R.items ? R.at<V>(i, &g[k]) : -1;
-    if (idx[k] < 0) continue;
-    if (RX) vx[k] = *reinterpret_cast<const P*>(x + idx[k]);
-    if (RA) va[k] = *reinterpret_cast<const P*>(a + idx[k]);
-    if (RB) vb[k] = *reinterpret_cast<const P*>(b + idx[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < kVecItems; k++) {
-    if (idx[k] < 0) continue;
-    P r;
-#pragma unroll
-    for (int j = 0; j < V; j++)
-      lane<T, V>(r, j) = vec_value<T, OP>(RX ? lane<T, V>(vx[k], j) : T(0), RA ? lane<T, V>(va[k], j) : T(0),
-                                          RB ? lane<T, V>(vb[k], j) : T(0), alpha, beta, gamma);
-    if (V == 1 || (g[k] > 0 && g[k] < R.last)) *reinterpret_cast<P*>(x + idx[k]) = r;
-    else if (g[k] == 0) x[idx[k] + 1] = lane<T, V>(r, V - 1);
-    else x[idx[k]] = lane<T, V>(r, 0);
-  }
+  for (int j = 0; j < V; j++)
+    lane<T, V>(r, j) = vec_value<T, OP>(RX ? lane<T, V>(vx, j) : T(0), RA ? lane<T, V>(va, j) : T(0),
+                                        RB ? lane<T, V>(vb, j) : T(0), alpha, beta, gamma);
+  if (V == 1 || (g > 0 && g < R.last)) *reinterpret_cast<P*>(x + k) = r;
+  else if (g == 0) x[k + 1] = lane<T, V>(r, V - 1);
+  else x[k] = lane<T, V>(r, 0);
 }
 
 // every padded value of a vector: V at a time (16 bytes, or 1 where x starts off that grid),
@@ -107,7 +121,7 @@ __global__ void __launch_bounds__(256) convert_kernel(long n, TD* __restrict__ d
 
 namespace {
 
-// One partial per workgroup over the interior cells (groups as in vec_op_kernel), kRedItems
+// One partial per workgroup over the interior cells (groups of interior rows: te::Rows), kRedItems
 // groups a thread and step so that their loads are in flight together: dot product 88 -> 55 us,
 // norm of a vector just written 77 -> 31 us (the same vectors; one load in flight before)
 constexpr int kRedItems = 4;
@@ -203,9 +217,13 @@ void vec_op_t(const Layout& L, int op, T* x, const T* a, const T* b, double alph
       hipLaunchKernelGGL((vec_fill_kernel<T, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, x, T(alpha));
     return;
   }
-  const int V = group_of<T>(L, x, a, b);
-  const Rows R(L, V);
-  const int grid = (R.items + 256 * kVecItems - 1) / (256 * kVecItems);
+  // FP64 with three streams or more by single values: x += a y at 32768 patches of 16^3 723 us
+  // against 772 in pairs, with two terms 975 against 1018 (8^3: 117 against 126, 154 against 164).
+  // Pairs for fewer streams (x = a at 512 patches of 64^3 454 us against 529) and in FP32 (x = a
+  // at 32768 patches of 16^3 376 against 590)
+  const int V = sizeof(T) == 8 && op >= VOP_ADD ? 1 : group_of<T>(L, x, a, b);
+  const FlatGroups R(L, V);
+  const int grid = (int)(((long)R.items + 255) / 256);
 #define TE_VO(OP_)                                                                                                  \
   case OP_:                                                                                                         \
     if (V == 2)                                                                                                     \
