@@ -863,7 +863,7 @@ def test_patches_of_many_cells(ns):
             assert relerr(dcv.get(), O.restrict(of, oc, f0)) <= (TOL64 if t64 else TOL32)
 
 
-@pytest.mark.parametrize("ns", [(2, 2, 2), (2, 2, 8), (4, 2, 4), (4, 4, 6), (8, 8, 8), (4, 16, 6), (12, 6, 10)])
+@pytest.mark.parametrize("ns", [(2, 2, 2), (2, 2, 8), (4, 2, 4), (4, 4, 6), (8, 8, 8), (4, 16, 6), (12, 6, 10), (16, 16, 2)])
 @pytest.mark.parametrize("big", [False, True])
 def test_ghost_fill_3d_forms(ns, big):
     """Every form of the 3D face fill (faces of at most 16 cells, of at most 64, of more; few

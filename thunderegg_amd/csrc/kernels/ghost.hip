@@ -78,16 +78,16 @@ __global__ void ghost_corners_2d(const DevPatch* __restrict__ dp, T* __restrict_
 //  FACES_SMALL, faces of at most 16 cells: a wave per patch, the six faces' cells in a row
 //    (fill_faces3_small; 32,768 patches of 4^3: 36 -> 26 us, 48 as FACES_SIDES);
 //  FACES_SIDES, up to 64 cells: a workgroup per patch, a wave per side (4,096 of 8^3: 23 -> 12);
-//  FACES_PARTS, more, on levels that leave the card partly idle: as FACES_SIDES, the patch's faces shared by
-//    several workgroups (512 of 16^3: 11.8 -> 6.8, 8.0 as FACES_ALL; 64 of 64^3: 13.6 -> 12.6, 54;
-//    8 of 128^3: 6.8 -> 5.1, 107).  Up to one patch a CU they are dealt to the XCDs in turn:
-//    contiguous eighths take 15.3 us for 64 of 64^3, but 6.8 against 9.9 for 512 of 16^3;
-//  FACES_ALL, more, on the other levels: a workgroup per patch, each thread a cell of all six sides
-//    (fill_faces3), so that one workgroup reads a neighbour's lines (4,096 of 16^3: 76 -> 62).
-enum FaceForm { FACES_SMALL, FACES_SIDES, FACES_PARTS, FACES_ALL };
+//  FACES_PARTS, more: as FACES_SIDES, the patch's faces shared by several workgroups, on large
+//    levels in parts of under three passes of a wave (4,096 of 12^3: 42 -> 27, of 16^3 77 -> 49, of
+//    32^3 327 -> 318; in one workgroup a patch, a thread the same cell of all six sides: 32, 60 and
+//    356), on small ones in as many as fill the card (512 of 16^3: 11.8 -> 7.1; 64 of 64^3: 13.1 ->
+//    12.4; 8 of 128^3: 6.8 -> 5.1).  Up to one patch a CU they are dealt to the XCDs in turn:
+//    contiguous eighths take 15.3 us for 64 of 64^3, but 6.8 against 9.9 for 512 of 16^3
+enum FaceForm { FACES_SMALL, FACES_SIDES, FACES_PARTS };
 
 template <typename T, int FORM>
-__global__ void __launch_bounds__(FORM == FACES_SIDES || FORM == FACES_PARTS ? 384 : 256)
+__global__ void __launch_bounds__(FORM == FACES_SMALL ? 256 : 384)
   ghost_faces_3d(const DevPatch* __restrict__ dp, T* u, Layout L, int split, bool in_turn)
 {
   const int b = FORM == FACES_PARTS && in_turn ? blockIdx.x : xcd_item(blockIdx.x, gridDim.x);
@@ -99,13 +99,6 @@ __global__ void __launch_bounds__(FORM == FACES_SIDES || FORM == FACES_PARTS ? 3
   const int p = FORM == FACES_PARTS ? b >> split : b;
   if (p >= L.np) return;
   const DevPatch& P = dp[p];
-  if (FORM == FACES_ALL) {
-    int first[6] = { 0, 0, 0, 0, 0, 0 }, last[6];
-#pragma unroll
-    for (int s = 0; s < 6; s++) last[s] = L.n[s < 2 ? 1 : 0] * L.n[s < 4 ? 2 : 1];
-    fill_faces3<T>(L, P, u, p, threadIdx.x, blockDim.x, first, last);
-    return;
-  }
   const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int type = P.type[20 + s], ni = L.n[s < 2 ? 1 : 0], nj = L.n[s < 4 ? 2 : 1];
   if (type < 0) return;
@@ -241,7 +234,8 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, bool low
     }
   } else {
     const int face = largest_face(L);
-    const int split = patch_split(d->np, face, 64, 2, face);  // of FACES_PARTS: short waves, so 48 of them a CU
+    int split = patch_split(d->np, face, 64, 2, face);  // of FACES_PARTS: short waves, so 48 of them a CU
+    while ((face >> split) >= 3 * 64) split++;
 #define TE_GF(FORM_, UNITS_, BLOCK_)                                                                                \
   hipLaunchKernelGGL((ghost_faces_3d<T, FORM_>), dim3(xcd_grid(UNITS_)), dim3(BLOCK_), 0, s, d->d_patches, u, L, split, \
                      d->np <= cu_count())
@@ -250,10 +244,8 @@ int ghost_fill_t(const te_ghost_filler* g, T* u, int ncomp, bool faces, bool low
       TE_GF(FACES_SMALL, (d->np + 3) / 4, B);
     } else if (face <= 64) {
       TE_GF(FACES_SIDES, d->np, 384);
-    } else if (d->np * 6L < 16L * cu_count()) {
-      TE_GF(FACES_PARTS, d->np << split, 384);
     } else {
-      TE_GF(FACES_ALL, d->np, std::min(B, (face + 63) / 64 * 64));
+      TE_GF(FACES_PARTS, d->np << split, 384);
     }
 #undef TE_GF
     if (lowdim && g->fill_type != TE_FACES) {
