@@ -85,9 +85,9 @@ int cu_count()
   return v;
 }
 
-int patch_split(int np, long items, int pass, int waves, long most)
+int patch_split(int np, long items, int pass, int waves, long most, int per_cu)
 {
-  const long full = 16L * cu_count();
+  const long full = (long)per_cu * cu_count();
   int s = 0;
   while ((items >> s) > 2L * pass && ((long)np << s) * waves < full && (2L << s) <= most && s < 16) s++;
   return s;

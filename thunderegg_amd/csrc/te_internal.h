@@ -208,12 +208,12 @@ std::vector<int32_t> ring_table(const te_domain* d, const int32_t* parent, const
 int cu_count();
 // Each of np patches is shared by 2^s units (workgroups or wavefronts) of `waves` waves, `pass` of
 // its `items` work items a pass: s grows while a unit would take more than two passes and the
-// launch has fewer than 16 waves a CU, and not past `most` units.  A patch that one wave walks
+// launch has fewer than per_cu waves a CU, and not past `most` units.  A patch that one wave walks
 // alone takes as long as its cells: the operator on 4 patches of 1024^2 (FP64) 3,460 us as one wave
-// a patch, 27 shared; 8 of 64^3 148 and 17; 64 of 32^2 7.0 and 4.4.  Not more waves, nor fewer (the
-// same for 1,024 patches of 128^2 in FP32 at 8 / 16 / 32 waves a CU: 41 / 30 / 34 us; 512 of 16^3 in
-// FP64: 17 / 16 / 20; only 16 patches of 1024^2 gain from more, 96 / 80).
-int patch_split(int np, long items, int pass, int waves, long most);
+// a patch, 26 shared; 8 of 64^3 148 and 17; 64 of 32^2 7.0 and 4.4.  Neither more nor fewer than 16
+// (1,024 patches of 128^2 in FP32 at 8 / 16 / 32 waves a CU: 41 / 30 / 34 us; 512 of 16^3 in FP64:
+// 17 / 16 / 20), but for the long rows that launch_one (stencil.hip) names.
+int patch_split(int np, long items, int pass, int waves, long most, int per_cu = 16);
 // workgroups of `block` threads and `shmem` dynamic LDS bytes of `kernel` resident at once
 // on the whole current device (occupancy query, cached)
 int resident_blocks(const void* kernel, int block, size_t shmem);
